@@ -115,9 +115,11 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
 /*
  * Bytes of the optional workspace (`seg_ws`) of tops_gla_chunk_fwd (backward = 0) or
  * tops_gla_chunk_bwd (backward = 1) for this problem (0: the call does not use one); N =
- * sequences (B, or the number of cu_seqlens sequences with varlen = 1). Parts, each
- * 256-byte aligned, in this order:
- *  - sequence segments (full-head kernels, fixed length): the inter-chunk scans run as
+ * sequences (B, or the number of cu_seqlens sequences with varlen != 0). varlen = 1: the
+ * flags and final states alone (every sequence one segment, gated in every block); varlen =
+ * 2: with the segment and gating parts too, after them. Parts, each 256-byte aligned, in this
+ * order for fixed-length sequences:
+ *  - sequence segments (full-head kernels): the inter-chunk scans run as
  *    parallel segments (local states, then all segments at once, each folding its entry
  *    state from them) instead of one chunk after another;
  *  - gate-range flags (K <= 512): the chunk kernels factor e^{g~_i - g~_j} per element as
@@ -128,11 +130,12 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
  *    (exact for any decay) then recompute the flagged sequences and heads: o and ht in the
  *    forward; dq, dk, dv, dg and dh0 in the backward (K and V <= 512). Without this part a
  *    gate range beyond the limit gives non-finite or inaccurate values;
- *  - wide heads (K = 256, three or more 64-column V tiles, fixed length): the per-chunk
+ *  - wide heads (K = 256, three or more 64-column V tiles): the per-chunk
  *    gating that the scans, the forward and the dv kernel then stream;
  *  - backward only: the fallback's final states (f32 [N, H, K, V], K and V <= 512; without
  *    it a call with dht is not checked).
- * A shorter workspace drops the later parts. The per-chunk states h_ws that the forward
+ * A shorter workspace drops the later parts (varlen: the segments and the gating together,
+ * below the varlen = 2 size). The per-chunk states h_ws that the forward
  * stores for flagged pairs are not meaningful (the backward recomputes those pairs).
  * No counterpart in the reference (its scans are sequential grid axes, chunk_h.py:252-271).
  */

@@ -135,8 +135,11 @@ bool use_head(int dtype, int chunk, int64_t K, int64_t V, bool g_is_cumsum,
 
 // Workspace of tops_gla_chunk_fwd / _bwd, each part 256-byte aligned:
 //   [segment states, decays (full-head, NS > 1)] [gate-range flags, int32]
-//   [wide heads' per-chunk gating (full-head, fixed length)]
+//   [wide heads' per-chunk gating (full-head)]
 //   [backward only: fallback final states f32 [N, H, K, V]]
+// for fixed-length sequences. Varlen sequences have two layouts, told apart by the bytes
+// given: [flags] [final states], which runs every sequence as one segment and gates in every
+// block, and (full-head kernels) that with [segment states, decays] [gating] after it.
 // The flags part holds the full-head kernels' per-block flags or the per-chunk flags [NC, H]
 // of the other paths (its size is the larger of the two, NC bounded by N ceil(T / C), or
 // ceil(T / C) + N for varlen). Flags exist when the recurrent fallback runs the shape (K <=
@@ -147,28 +150,48 @@ long align256(long x) { return (x + 255) / 256 * 256; }
 
 struct WsLayout {
   int NS = 1, SL = 0, VT = 1;
+  long slots = 0;                              // segment states held
   long seg = 0, flags = 0, gate = 0, ht = 0;   // bytes of each part
-  long off_flags = 0, off_gate = 0, off_ht = 0, total = 0;
+  long off_seg = 0, off_flags = 0, off_gate = 0, off_ht = 0, total = 0;
+  long flags_end() const { return off_flags + flags; }
 };
 
+// `packed`: varlen sequences with the segment and gating parts.
 WsLayout ws_layout(int N, int T, int H, int K, int V, int C, bool varlen, bool head,
-                   bool backward) {
+                   bool backward, bool packed) {
   WsLayout w;
-  long nflag = (varlen ? (long)(T + C - 1) / C + N : (long)N * ((T + C - 1) / C)) * H;
+  const long nc = varlen ? (long)(T + C - 1) / C + N : (long)N * ((T + C - 1) / C);
+  long nflag = nc * H;
   if (head) {
     w.VT = tops::head_vtiles(K, V);
-    tops::head_seg_plan(N, H, T, C, varlen, w.NS, w.SL, w.VT);
-    w.seg = align256(tops::head_seg_ws_bytes(N, w.NS, H, K, V));
-    w.gate = varlen ? 0 : align256(tops::head_gate_ws_bytes(N, T, H, K, V));
-    const long nblk = (long)N * w.NS * H * w.VT;
+    long nblk;
+    if (varlen) {
+      if (packed) w.SL = tops::head_varlen_seg(N, nc, H, w.VT);
+      w.slots = w.SL > 0 ? nc / w.SL + 1 : 0;
+      nblk = (w.SL > 0 ? nc / w.SL + N : (long)N) * H * w.VT;
+    } else {
+      tops::head_seg_plan(N, H, T, C, varlen, w.NS, w.SL, w.VT);
+      w.slots = w.NS > 1 ? (long)N * w.NS : 0;
+      nblk = (long)N * w.NS * H * w.VT;
+    }
+    if (w.slots > 0) w.seg = align256(tops::head_seg_ws_bytes(w.slots, H, K, V));
+    if (!varlen || packed) w.gate = align256(tops::head_gate_ws_bytes(nc, H, K, V));
     if (nblk > nflag) nflag = nblk;
   }
   w.flags = K <= 512 ? align256(nflag * 4) : 0;
   w.ht = backward && tops::recurrent_supported(K, V) ? align256((long)N * H * K * V * 4) : 0;
-  w.off_flags = w.seg;
-  w.off_gate = w.off_flags + w.flags;
-  w.off_ht = w.off_gate + w.gate;
-  w.total = w.off_ht + w.ht;
+  if (varlen) {
+    w.off_flags = 0;
+    w.off_ht = w.flags;
+    w.off_seg = w.off_ht + w.ht;
+    w.off_gate = w.off_seg + w.seg;
+    w.total = w.off_gate + w.gate;
+  } else {
+    w.off_flags = w.seg;
+    w.off_gate = w.off_flags + w.flags;
+    w.off_ht = w.off_gate + w.gate;
+    w.total = w.off_ht + w.ht;
+  }
   return w;
 }
 
@@ -184,23 +207,38 @@ struct WsParts {
 
 WsParts ws_parts(const tops::SeqInfo& si, int64_t H, int64_t K, int64_t V, void* ws,
                  int64_t ws_bytes, bool head, bool backward) {
-  const WsLayout w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, si.cu != nullptr,
-                               head, backward);
+  const bool varlen = si.cu != nullptr;
+  WsLayout w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, true);
+  if (varlen && ws_bytes < w.total)
+    w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, false);
   WsParts p;
   p.VT = w.VT;
   const bool usable = ws != nullptr && ((uintptr_t)ws & 255u) == 0;
   if (!usable) return p;
   char* b = (char*)ws;
-  if (w.NS > 1 && ws_bytes >= w.seg) {
+  if (w.slots > 0 && ws_bytes >= w.off_seg + w.seg) {
     p.NS = w.NS;
     p.SL = w.SL;
-    p.st = (float*)b;
-    p.gm = (float*)(b + (long)si.N * w.NS * H * K * V * 4);
+    p.st = (float*)(b + w.off_seg);
+    p.gm = p.st + w.slots * H * K * V;
   }
-  if (w.flags > 0 && ws_bytes >= w.off_gate) p.flags = (int*)(b + w.off_flags);
-  if (w.gate > 0 && ws_bytes >= w.off_ht) p.gate = b + w.off_gate;
-  if (w.ht > 0 && ws_bytes >= w.total) p.ht = (float*)(b + w.off_ht);
+  if (w.flags > 0 && ws_bytes >= w.off_flags + w.flags) p.flags = (int*)(b + w.off_flags);
+  if (w.gate > 0 && ws_bytes >= w.off_gate + w.gate) p.gate = b + w.off_gate;
+  if (w.ht > 0 && ws_bytes >= w.off_ht + w.ht) p.ht = (float*)(b + w.off_ht);
   return p;
+}
+
+// Per-block flags of the full-head kernels in the recurrent fallback's layout.
+tops::GateFlags block_flags(int* f, const tops::SeqInfo& si, int NS, int SL, int vt) {
+  tops::GateFlags g = {};
+  g.p = f;
+  g.ns = NS;
+  g.vt = vt;
+  if (si.cu && SL > 0) {
+    g.co = si.chunk_cu;
+    g.sl = SL;
+  }
+  return g;
 }
 
 // Per-chunk flags [NC, H] in the recurrent fallback's layout.
@@ -297,7 +335,7 @@ int64_t tops_gla_chunk_ws_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int6
   if (!dtype_ok(dtype) || chunk_size <= 0 || chunk_size > 64) return 0;
   const bool head = tops::head_supported(dtype, chunk_size, (int)K, (int)V, false);
   return ws_layout((int)N, (int)T, (int)H, (int)K, (int)V, chunk_size, varlen != 0, head,
-                   backward != 0).total;
+                   backward != 0, varlen == 2).total;
 }
 
 int tops_gla_chunk_local_cumsum(const void* g, void* out, int64_t B, int64_t T, int64_t H,
@@ -673,7 +711,7 @@ int tops_gla_chunk_fwd(const void* q, const void* k, const void* v, const void* 
     r.K = (int)K;
     r.V = (int)V;
     r.si = si;
-    r.flags = per_chunk ? chunk_flags(f.flags, si) : tops::GateFlags{f.flags, w.NS, w.VT};
+    r.flags = per_chunk ? chunk_flags(f.flags, si) : block_flags(f.flags, si, w.NS, w.SL, w.VT);
     return hip_status(tops::run_recurrent_fwd(r, dtype, dtype, st),
                       "chunk_fwd (gate-range fallback)");
   }
@@ -754,7 +792,7 @@ int tops_gla_chunk_fwd_noalloc(const void* q, const void* k, const void* v, cons
   // the segment part (full-head shapes) and the gate-range flags
   const bool head = tops::head_supported(dtype, chunk_size, (int)K, (int)V, false);
   const long need = K <= 512 ? ws_layout(si.N, si.T, (int)H, (int)K, (int)V, chunk_size,
-                                         si.cu != nullptr, head, false).off_gate
+                                         si.cu != nullptr, head, false, false).flags_end()
                              : 0;
   if (need > kScratchBytes)
     return fail(TOPS_GLA_EINVAL,
@@ -932,7 +970,7 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
     r.K = (int)K;
     r.V = (int)V;
     r.si = si;
-    r.flags = {b.flags, NS, 1};
+    r.flags = block_flags(b.flags, si, NS, SL, 1);
     return hip_status(tops::run_recurrent_bwd(r, dtype, dtype, st),
                       "chunk_bwd (gate-range fallback)");
   } else if (head) {

@@ -260,19 +260,90 @@ __device__ __forceinline__ void mask_rows(uint4 (&r)[N], int row0, int len, bool
   for (int j = 0; j < N; ++j) r[j] = mask16(r[j], (col_ok && row0 + j < len) ? ~0u : 0u);
 }
 
-// Chunk range of the block's segment.
+// The block's segment: `s` of the `ns` segments of sequence `seq`, chunks [cb, ce); its
+// sequence's local states start at workspace slot `st0` (slot of segment u: st0 + u).
 struct Seg {
-  int seq, s, bos, eos, c0, cb, ce;
+  int seq, s, ns, bos, eos, c0, cb, ce;
+  long st0;
 };
+
+// Fixed-length sequences: NS segments of SL chunks each.
 __device__ __forceinline__ Seg seg_of(const SeqInfo& si, int seq, int s, int NS, int SL) {
   Seg r;
   int nc;
   seq_range(si, seq, r.bos, r.eos, r.c0, nc);
   r.seq = seq;
   r.s = s;
+  r.ns = NS;
+  r.st0 = (long)seq * NS;
   r.cb = NS > 1 ? min(nc, s * SL) : 0;
   r.ce = NS > 1 ? min(nc, r.cb + SL) : nc;
   return r;
+}
+
+// Varlen sequences: sequence i of nc chunks (from chunk c0 = chunk_cu[i]) has ns = ceil(nc /
+// SL) segments of nearly equal size. The launcher knows only the numbers of chunks and
+// sequences, so the blocks index slots that the chunk offsets alone give:
+// * BLOCK slots c0 / SL + i + s (NC / SL + N in all): a sequence's slots never meet the next
+//   one's, since ceil(nc / SL) <= (c0 + nc) / SL - c0 / SL + 1;
+// * STATE slots c0 / SL + u (NC / SL + 1 in all) for the ns - 1 segments whose local states
+//   are needed (ns - 1 <= (c0 + nc) / SL - c0 / SL): forward segments 0 .. ns - 2, reverse
+//   segments 1 .. ns - 1 (u = s - 1).
+// The sequence of a slot is the last one whose first slot is not past it (binary search).
+// False: the slot is empty.
+template <bool REV>
+__device__ __forceinline__ bool seg_of_slot(const SeqInfo& si, int slot, int SL, bool states,
+                                            Seg& r) {
+  int lo = 0, hi = si.N - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (si.chunk_cu[mid] / SL + (states ? 0 : mid) <= slot) lo = mid; else hi = mid - 1;
+  }
+  int nc;
+  seq_range(si, lo, r.bos, r.eos, r.c0, nc);
+  r.seq = lo;
+  r.ns = (nc + SL - 1) / SL;
+  const int u = slot - r.c0 / SL - (states ? 0 : lo);
+  r.s = states && REV ? u + 1 : u;
+  r.st0 = r.c0 / SL - (REV ? 1 : 0);
+  if (u < 0 || u >= r.ns - (states ? 1 : 0)) return false;
+  r.cb = (int)((long)r.s * nc / r.ns);
+  r.ce = (int)((long)(r.s + 1) * nc / r.ns);
+  return true;
+}
+
+// Block -> (unit, V tile), unit = segment and head. The V tiles of a unit go to one XCD (its
+// L2 serves their re-reads of q / k / g). Fixed-length sequences: consecutive units on one XCD
+// (xcd_remap). Varlen: units dealt round-robin, since consecutive ones are pieces of one
+// sequence and a contiguous share per XCD would leave some XCDs with the long sequences'
+// full pieces and others with short or empty slots (the packed training shape of 13 documents
+// in 16384 tokens, 16 heads of 128 x 128, forward + backward: 699 us contiguous, 444 us dealt).
+__device__ __forceinline__ void unit_of_block(const SeqInfo& si, int SL, int VT, int& unit,
+                                              int& vt) {
+  const int L = blockIdx.x, total = gridDim.x;
+  if (si.cu && SL > 0) {
+    const int u8 = total / VT & ~7;   // units in whole rounds of 8
+    if (L < u8 * VT) {
+      unit = (L >> 3) / VT * 8 + (L & 7);
+      vt = (L >> 3) % VT;
+    } else {
+      unit = L / VT;
+      vt = L % VT;
+    }
+    return;
+  }
+  const int L0 = xcd_remap(L, total);
+  unit = L0 / VT;
+  vt = L0 % VT;
+}
+
+// Segment of block index j (of all segments; `states`: varlen pass 1, the state slots).
+template <bool REV>
+__device__ __forceinline__ bool find_seg(const SeqInfo& si, int j, int NS, int SL, bool states,
+                                         Seg& r) {
+  if (si.cu && SL > 0) return seg_of_slot<REV>(si, j, SL, states, r);
+  r = seg_of(si, j / NS, j % NS, NS, SL);
+  return true;
 }
 
 // Scans over the four 16-lane rows of a wave, lane l of every row holding the same column
@@ -500,16 +571,17 @@ __device__ __forceinline__ void load_state(f32x4 (&acc)[NTV][NTK], const float* 
 // Entry state of segment s of a segmented scan, folded from the pass-1 local states L_u and
 // segment decays Gamma_u (base 2) in the workspace, in the order the scan runs: forward
 // L_0, then H <- 2^{Gamma_u} H + L_u for u = 1 .. s-1; reverse L_{NS-1}, then u = NS-2 ..
-// s+1. Slot u of (sequence, head) is st + ((seq NS + u) H + h) K ld (+ cv: a V tile's
-// first column), its decays gm + ((seq NS + u) H + h) K.
+// s+1. Segment u's state is st + ((st0 + u) H + h) K ld (+ cv: a V tile's first column), its
+// decays gm + ((st0 + u) H + h) K.
 template <int NTV, int NTK, bool REV>
 __device__ __forceinline__ void load_entry_state(f32x4 (&acc)[NTV][NTK], const float* st,
-                                                 const float* gm, int seq, int s, int NS,
-                                                 int H, int hh, int K, int Vw, int cv, int ld,
-                                                 int vt0, int kt0, int lane) {
+                                                 const float* gm, const Seg& sg, int H, int hh,
+                                                 int K, int Vw, int cv, int ld, int vt0,
+                                                 int kt0, int lane) {
   const long KV = (long)K * ld;
-  auto slot = [&](int u) { return st + ((long)(seq * NS + u) * H + hh) * KV + cv; };
-  const int u0 = REV ? NS - 1 : 0;
+  const int s = sg.s;
+  auto slot = [&](int u) { return st + ((sg.st0 + u) * H + hh) * KV + cv; };
+  const int u0 = REV ? sg.ns - 1 : 0;
   load_state<NTV, NTK>(acc, slot(u0), K, Vw, vt0, kt0, lane, ld);
   for (int u = REV ? u0 - 1 : 1; REV ? u > s : u < s; u += REV ? -1 : 1) {
     f32x4 x[NTV][NTK];
@@ -517,7 +589,7 @@ __device__ __forceinline__ void load_entry_state(f32x4 (&acc)[NTV][NTK], const f
 #pragma unroll
     for (int j = 0; j < NTK; ++j) {
       const int kk = (kt0 + j) * 16 + (lane & 15);
-      const float g = kk < K ? exp2_hw(gm[((long)(seq * NS + u) * H + hh) * K + kk]) : 0.f;
+      const float g = kk < K ? exp2_hw(gm[((sg.st0 + u) * H + hh) * K + kk]) : 0.f;
 #pragma unroll
       for (int i = 0; i < NTV; ++i)
 #pragma unroll
@@ -656,17 +728,21 @@ __global__ __launch_bounds__(NT) void head_scan_kernel(HeadScanArgs p) {
   const int H = p.H, K = p.K, V = p.V;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
-  const int L0 = xcd_remap(blockIdx.x, gridDim.x);
   const int VT = (V + VP - 1) / VP;            // V tiles (blocks of one segment and head)
-  const int vt = L0 % VT, L = L0 / VT;
+  int L, vt;
+  unit_of_block(p.si, p.SL, VT, L, vt);
   const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
   const int hh = L % H;
-  const int nsl = p.ns_launch;
-  const int s = p.s_begin + (L / H) % nsl;
-  const Seg sg = seg_of(p.si, (L / H) / nsl, s, p.NS, p.SL);
+  Seg sg;
+  if (p.si.cu && p.SL > 0) {
+    if (!seg_of_slot<REV>(p.si, L / H, p.SL, p.pass == 1, sg)) return;   // uniform
+  } else {
+    const int nsl = p.ns_launch;
+    sg = seg_of(p.si, (L / H) / nsl, p.s_begin + (L / H) % nsl, p.NS, p.SL);
+  }
   const int nsteps = CR == HC ? sg.ce - sg.cb : (sg.ce - sg.cb + 1) / 2;
-  const bool first_seg = REV ? (s == p.NS - 1) : (s == 0);
-  const bool last_seg = REV ? (s == 0) : (s == p.NS - 1);
+  const bool first_seg = REV ? (sg.s == sg.ns - 1) : (sg.s == 0);
+  const bool last_seg = REV ? (sg.s == 0) : (sg.s == sg.ns - 1);
   const long rsK = (long)H * K, rsV = (long)H * V;
   const long KV = (long)K * V;
 
@@ -680,8 +756,8 @@ __global__ __launch_bounds__(NT) void head_scan_kernel(HeadScanArgs p) {
   f32x4 acc[NTV][NTK];
   {
     if (!first_seg && p.pass == 3)
-      load_entry_state<NTV, NTK, REV>(acc, p.seg_state, p.seg_gam, sg.seq, s, p.NS, H, hh, K,
-                                      Vw, cv, V, vt0, kt0, lane);
+      load_entry_state<NTV, NTK, REV>(acc, p.seg_state, p.seg_gam, sg, H, hh, K, Vw, cv, V,
+                                      vt0, kt0, lane);
     else
       load_state<NTV, NTK>(acc,
                            first_seg && p.s_init
@@ -931,10 +1007,10 @@ __global__ __launch_bounds__(NT) void head_scan_kernel(HeadScanArgs p) {
   }
 
   if (p.pass == 1) {
-    store_state_f32<NTV, NTK>(acc, p.seg_state + ((long)(sg.seq * p.NS + s) * H + hh) * KV + cv,
-                              K, Vw, vt0, kt0, lane, V);
+    store_state_f32<NTV, NTK>(acc, p.seg_state + ((sg.st0 + sg.s) * H + hh) * KV + cv, K, Vw,
+                              vt0, kt0, lane, V);
     if (vt == 0 && rs == TRS && colA)   // the decays are the same for every V tile
-      st_f8(p.seg_gam + ((long)(sg.seq * p.NS + s) * H + hh) * K + cg * 8, gsum);
+      st_f8(p.seg_gam + ((sg.st0 + sg.s) * H + hh) * K + cg * 8, gsum);
   } else if (last_seg && p.s_final) {
     store_state_f32<NTV, NTK>(acc, p.s_final + ((long)sg.seq * H + hh) * KV + cv, K, Vw, vt0,
                               kt0, lane, V);
@@ -973,11 +1049,9 @@ __global__ __launch_bounds__(HNT) void head_gate_kernel(HeadFwdArgs p) {
   const int H = p.H, K = p.K;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int hh = blockIdx.x % H, ci = blockIdx.x / H, seq = blockIdx.y;
-  int bos, eos, c0, nc;
-  seq_range(p.si, seq, bos, eos, c0, nc);
-  if (ci >= nc) return;   // uniform
-  const int t0 = bos + ci * HC, len = min(HC, eos - t0);
+  const int hh = blockIdx.x % H, c = blockIdx.x / H;   // global chunk
+  int seq, t0, len;
+  chunk_range(p.si, c, seq, t0, len);
   const long rsK = (long)H * K;
   const int cg = tid % M::NCG, rs = tid / M::NCG;
   const bool colA = cg * 8 < K;
@@ -991,7 +1065,7 @@ __global__ __launch_bounds__(HNT) void head_gate_kernel(HeadFwdArgs p) {
   for (int j = 0; j < RPT; ++j) gm[j] = mask16(Rg[j], (colA && rs * RPT + j < len) ? ~0u : 0u);
   float gt[RPT][8], gam[8], first[8];
   head_cumsum<KP>(gm, gt, gam, first, sTot, sFirst, cg, rs, lane, w);
-  unsigned char* ent = (unsigned char*)p.gate_ws + ((long)(c0 + ci) * H + hh) * gate_ws_entry(K);
+  unsigned char* ent = (unsigned char*)p.gate_ws + ((long)c * H + hh) * gate_ws_entry(K);
   bf16* gq = (bf16*)ent;
   bf16* gk = gq + HC * K;
   bf16* gA = gk + HC * K;
@@ -1006,7 +1080,7 @@ __global__ __launch_bounds__(HNT) void head_gate_kernel(HeadFwdArgs p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) dmax = fmaxf(dmax, fabsf(gt[j][e] - r[e]));
     const int bad = __syncthreads_or(dmax > kGateLimit2 ? 1 : 0);
-    if (tid == 0) p.flags[(long)(c0 + ci) * H + hh] = bad ? 1 : 0;
+    if (tid == 0) p.flags[(long)c * H + hh] = bad ? 1 : 0;
   }
   float fs[8];   // scale 2^r: qs = qg fs
 #pragma unroll
@@ -1573,13 +1647,13 @@ __global__ __launch_bounds__(HNT) void head_fwd_kernel(HeadFwdArgs p) {
   const int H = p.H, K = p.K, V = p.V;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
-  const int L0 = xcd_remap(blockIdx.x, gridDim.x);
   const int VT = (V + VP - 1) / VP;            // V tiles (blocks of one segment and head)
-  const int vt = L0 % VT, L = L0 / VT;
+  int L, vt;
+  unit_of_block(p.si, p.SL, VT, L, vt);
   const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
   const int hh = L % H;
-  const int s = (L / H) % p.NS;
-  const Seg sg = seg_of(p.si, (L / H) / p.NS, s, p.NS, p.SL);
+  Seg sg;
+  if (!find_seg<false>(p.si, L / H, p.NS, p.SL, false, sg)) return;   // uniform
   const int nsteps = sg.ce - sg.cb;
   const long rsK = (long)H * K, rsV = (long)H * V;
   const long KV = (long)K * V;
@@ -1601,9 +1675,9 @@ __global__ __launch_bounds__(HNT) void head_fwd_kernel(HeadFwdArgs p) {
   float dmax = 0.f;   // largest |g~ - r| of the factors (base 2): the gate-range check
   f32x4 acc[NTV][NTK];
   {
-    if (s > 0)
-      load_entry_state<NTV, NTK, false>(acc, p.seg_state, p.seg_gam, sg.seq, s, p.NS, H, hh, K,
-                                        Vw, cv, V, vt0, kt0, lane);
+    if (sg.s > 0)
+      load_entry_state<NTV, NTK, false>(acc, p.seg_state, p.seg_gam, sg, H, hh, K, Vw, cv, V,
+                                        vt0, kt0, lane);
     else
       load_state<NTV, NTK>(acc, p.h0 ? p.h0 + ((long)sg.seq * H + hh) * KV + cv : nullptr, K,
                            Vw, vt0, kt0, lane, V);
@@ -2023,12 +2097,12 @@ __global__ __launch_bounds__(HNT) void head_fwd_kernel(HeadFwdArgs p) {
     }
   }
 
-  if (s == p.NS - 1 && p.ht)
+  if (sg.s == sg.ns - 1 && p.ht)
     store_state_f32<NTV, NTK>(acc, p.ht + ((long)sg.seq * H + hh) * KV + cv, K, Vw, vt0, kt0,
                               lane, V);
   if (p.flags) {   // uniform; every block writes its flag, so nothing needs clearing
     const int bad = __syncthreads_or(dmax > kGateLimit2 ? 1 : 0);
-    if (tid == 0) p.flags[L0] = bad ? 1 : 0;
+    if (tid == 0) p.flags[(long)L * VT + vt] = bad ? 1 : 0;
   }
 }
 
@@ -2160,10 +2234,11 @@ __global__ __launch_bounds__(NT) void head_bwd_kernel(HeadBwdArgs p) {
   const int H = p.H, K = p.K, V = p.V;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
-  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  int L, vtile;
+  unit_of_block(p.si, p.SL, 1, L, vtile);
   const int hh = L % H;
-  const int s = (L / H) % p.NS;
-  const Seg sg = seg_of(p.si, (L / H) / p.NS, s, p.NS, p.SL);
+  Seg sg;
+  if (!find_seg<true>(p.si, L / H, p.NS, p.SL, false, sg)) return;   // uniform
   const int nsteps = sg.ce - sg.cb;
   const long rsK = (long)H * K, rsV = (long)H * V;
   const long KV = (long)K * V;
@@ -2183,9 +2258,9 @@ __global__ __launch_bounds__(NT) void head_bwd_kernel(HeadBwdArgs p) {
   int gbad = 0;          // uniform: a chunk had a factor beyond the gate-range limit
   f32x4 acc[NTV][NTK];   // dh[v][k]
   {
-    if (s < p.NS - 1)
-      load_entry_state<NTV, NTK, true>(acc, p.seg_state, p.seg_gam, sg.seq, s, p.NS, H, hh, K, V,
-                                       0, V, vt0, kt0, lane);
+    if (sg.s < sg.ns - 1)
+      load_entry_state<NTV, NTK, true>(acc, p.seg_state, p.seg_gam, sg, H, hh, K, V, 0, V, vt0,
+                                       kt0, lane);
     else
       load_state<NTV, NTK>(acc, p.dht ? p.dht + ((long)sg.seq * H + hh) * KV : nullptr, K, V,
                            vt0, kt0, lane);
@@ -2709,7 +2784,7 @@ __global__ __launch_bounds__(NT) void head_bwd_kernel(HeadBwdArgs p) {
     }
   }
 
-  if (s == 0 && p.dh0)
+  if (sg.s == 0 && p.dh0)
     store_state_f32<NTV, NTK>(acc, p.dh0 + ((long)sg.seq * H + hh) * KV, K, V, vt0, kt0, lane);
   if (p.flags) {   // uniform; every block writes its flag, so nothing needs clearing
     const int bad = __syncthreads_or(gbad);
@@ -2734,10 +2809,12 @@ int head_vtiles(int K, int V) {
   return (V + vp - 1) / vp;
 }
 
+constexpr long kVarlenMinSeg = 5;   // chunks
+
 void head_seg_plan(int N, int H, int T, int C, bool varlen, int& NS, int& SL, int VT) {
   NS = 1;
   SL = 0;
-  if (varlen || N <= 0 || H <= 0) return;
+  if (varlen || N <= 0 || H <= 0) return;   // varlen: head_varlen_seg
   const int nt = (T + C - 1) / C;
   const long nh = (long)N * H * (VT > 0 ? VT : 1);
   // one block per CU (MI355X: 256 CUs): the full-head kernels hold one block per CU (LDS),
@@ -2753,19 +2830,45 @@ void head_seg_plan(int N, int H, int T, int C, bool varlen, int& NS, int& SL, in
   }
 }
 
-// Per-chunk gating workspace of the wide forward: K = 256 heads split into three or more V
-// tiles (each tile's block would otherwise gate the same chunk again); fixed-length only.
-long head_gate_ws_bytes(int N, int T, int H, int K, int V) {
-  if (head_kp(K) != 256 || head_vtiles(K, V) < 3 || N <= 0 || T <= 0) return 0;
-  const long nt = (T + HC - 1) / HC;
-  return (long)N * nt * H * gate_ws_entry(K);
+// Varlen: segments of at most the returned number of chunks (0: none), from bounds on the
+// numbers of chunks (nc) and sequences alone -- the lengths are on the device. One block per
+// CU again, but pieces of many sizes share the CUs: they are cut to three quarters of a CU's
+// share of all chunks, so that a round of blocks that is not full costs less than a longer
+// longest piece. Unsegmented, the longest sequence's chunks ran one after another. Measured
+// at 13 documents (5 to 4821 tokens) in 16384 tokens, 16 heads of 128 x 128, forward +
+// backward: 1062 us unsegmented; pieces of 1/2, 3/4, 1 and 3/2 of the share 477, 444, 484
+// and 479 us. 7 prompts in 8192 tokens, 4 heads of 256 x 512, forward: 243 us; 124, 121, 116
+// and 120 us. Pieces below 5 chunks do not pay for the entry state they fold: 11 documents
+// in 1819 tokens 61 us with 5, 110 us with 3, 65 us with 8.
+int head_varlen_seg(int N, long nc, int H, int VT) {
+  if (N <= 0 || H <= 0) return 0;
+  const long nh = (long)H * (VT > 0 ? VT : 1);
+  const long sl = (nc * nh * 3 + 4 * 256 - 1) / (4 * 256);
+  const long SL = sl < kVarlenMinSeg ? kVarlenMinSeg : sl;
+  // the longest sequence has at most nc - (N - 1) chunks: nothing to cut
+  return nc - (N - 1) <= SL ? 0 : (int)SL;
 }
 
-long head_seg_ws_bytes(int N, int NS, int H, int K, int V) {
-  if (NS <= 1) return 0;
-  const long st = (long)N * NS * H * K * V * 4;
-  const long gm = (long)N * NS * H * K * 4;
+// Per-chunk gating workspace of the wide forward: K = 256 heads split into three or more V
+// tiles (each tile's block would otherwise gate the same chunk again). nc: chunks.
+long head_gate_ws_bytes(long nc, int H, int K, int V) {
+  if (head_kp(K) != 256 || head_vtiles(K, V) < 3 || nc <= 0) return 0;
+  return nc * H * gate_ws_entry(K);
+}
+
+// `slots`: segments whose states the workspace holds.
+long head_seg_ws_bytes(long slots, int H, int K, int V) {
+  const long st = slots * H * K * V * 4;
+  const long gm = slots * H * K * 4;
   return st + (gm + 255) / 256 * 256;
+}
+
+// Blocks of a launch over every segment, per head and V tile (varlen: the block slots).
+static long seg_blocks(const SeqInfo& si, int NS, int SL) {
+  return si.cu && SL > 0 ? (long)si.NC / SL + si.N : (long)si.N * NS;
+}
+static bool segmented(const SeqInfo& si, int NS, int SL) {
+  return NS > 1 || (si.cu && SL > 0);
 }
 
 template <int KP, int VP, bool REV, bool SG, int CR, bool PRE = false>
@@ -2818,7 +2921,11 @@ static hipError_t head_scan_launch(HeadScanArgs p, bool reverse, hipStream_t st,
     p.s_all = nullptr;
     p.s_final = nullptr;
   }
-  const long blocks = (long)p.si.N * ns_launch * p.H;
+  // varlen pass 1: the state slots
+  const long segs = p.si.cu && p.SL > 0
+                        ? (pass == 1 ? (long)p.si.NC / p.SL : seg_blocks(p.si, 1, p.SL))
+                        : (long)p.si.N * ns_launch;
+  const long blocks = segs * p.H;
   if (blocks == 0) return hipSuccess;
   return reverse ? head_scan_kp<true>(p, st, blocks) : head_scan_kp<false>(p, st, blocks);
 }
@@ -2826,7 +2933,7 @@ static hipError_t head_scan_launch(HeadScanArgs p, bool reverse, hipStream_t st,
 // Segment pass 1 (no-op when NS == 1): the local states; every segment's block folds its
 // own entry state from them (load_entry_state).
 static hipError_t head_prepare_segments(const HeadScanArgs& p, bool reverse, hipStream_t st) {
-  if (p.NS <= 1) return hipSuccess;
+  if (!segmented(p.si, p.NS, p.SL)) return hipSuccess;
   // pass 1 skips the last segment in flow order (its local state is never needed)
   return head_scan_launch(p, reverse, st, 1, reverse ? 1 : 0, p.NS - 1);
 }
@@ -2852,15 +2959,14 @@ static hipError_t launch_head_fwd_sg(const HeadFwdArgs& p, hipStream_t st, long 
 }
 
 hipError_t run_head_gate(const HeadFwdArgs& p, hipStream_t st) {
-  if (head_kp(p.K) != 256 || p.si.cu || !p.g || !p.gate_ws) return hipErrorInvalidValue;
-  const int nt = (p.si.T + HC - 1) / HC;
-  if ((long)nt * p.H * p.si.N == 0) return hipSuccess;
+  if (head_kp(p.K) != 256 || !p.g || !p.gate_ws) return hipErrorInvalidValue;
+  if (p.si.NC == 0) return hipSuccess;
   using GL = GPLayout<256>;
   hipError_t e = hipFuncSetAttribute((const void*)head_gate_kernel<256>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, GL::bytes);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((head_gate_kernel<256>), dim3((unsigned)(nt * p.H), (unsigned)p.si.N),
-                     dim3(HNT), GL::bytes, st, p);
+  hipLaunchKernelGGL((head_gate_kernel<256>), dim3((unsigned)((long)p.si.NC * p.H)), dim3(HNT),
+                     GL::bytes, st, p);
   return hipGetLastError();
 }
 
@@ -2890,7 +2996,7 @@ hipError_t run_head_dqkg(const BwdArgs& p, hipStream_t st) {
 
 template <int KP, int VP>
 static hipError_t launch_head_fwd(const HeadFwdArgs& p, hipStream_t st) {
-  const long blocks = (long)p.si.N * p.NS * p.H * ((p.V + VP - 1) / VP);
+  const long blocks = seg_blocks(p.si, p.NS, p.SL) * p.H * ((p.V + VP - 1) / VP);
   if (blocks == 0) return hipSuccess;
   if constexpr (KP == 256) {
     if (p.g && p.gate_ws) {   // the V tiles' blocks stream the per-chunk gating
@@ -2925,7 +3031,7 @@ hipError_t run_head_fwd(const HeadFwdArgs& p, hipStream_t st) {
     hipError_t e = run_head_gate(p, st);
     if (e != hipSuccess) return e;
   }
-  if (p.NS > 1) {
+  if (segmented(p.si, p.NS, p.SL)) {
     HeadScanArgs s = {};
     s.gate_ws = gated ? p.gate_ws : nullptr;
     s.a = p.k;
@@ -2971,14 +3077,14 @@ static hipError_t launch_head_bwd_sg(const HeadBwdArgs& p, hipStream_t st, long 
 
 template <int KP, int VP>
 static hipError_t launch_head_bwd(const HeadBwdArgs& p, hipStream_t st) {
-  const long blocks = (long)p.si.N * p.NS * p.H;
+  const long blocks = seg_blocks(p.si, p.NS, p.SL) * p.H;
   if (blocks == 0) return hipSuccess;
   return p.g ? launch_head_bwd_sg<KP, VP, false>(p, st, blocks)
              : launch_head_bwd_sg<KP, VP, true>(p, st, blocks);
 }
 
 hipError_t run_head_bwd(const HeadBwdArgs& p, hipStream_t st) {
-  if (p.NS > 1) {
+  if (segmented(p.si, p.NS, p.SL)) {
     HeadScanArgs s = {};
     s.a = p.q;
     s.b = p.dout;

@@ -106,12 +106,15 @@ hipError_t run_cumsum(const CumsumArgs& p, int in_dtype, int out_dtype, hipStrea
 // * per chunk (gate_range_kernel, head_gate_kernel; vt = 1): s = the sequence's chunk, i.e.
 //   [NC, H]; with varlen sequences `co` (chunk offsets [N + 1]) gives each sequence's chunk
 //   range instead of ns chunks from seq * ns.
+// Per-block flags of segmented varlen sequences (`co` and sl > 0): s = the segments of at most
+// sl chunks, from block slot co[seq] / sl + seq.
 // The recurrent fallback (exact for any decay) then recomputes the flagged (sequence, head)
 // pairs.
 struct GateFlags {
   int* p;         // nullable: no check, no fallback
   int ns, vt;     // segments (or chunks) and V tiles per (sequence, head)
-  const int* co;  // nullable: per-chunk flags of varlen sequences (ns unused)
+  const int* co;  // nullable: varlen sequences' chunk offsets (ns unused)
+  int sl;         // with co: 0 per-chunk flags, else per-block flags of segments of sl chunks
 };
 constexpr float kGateLimit2 = 100.f;
 
@@ -238,14 +241,17 @@ hipError_t run_recurrent_bwd(const RecBwdArgs& p, int dtype, int o_dtype, hipStr
 
 // Full-head kernels (chunk_head.hip): bf16, chunk 64, raw gates, K and V multiples of 8
 // (16-byte aligned rows); scans and forward for K <= 256 and any V (V tiles of 64 or 128
-// columns), the fused backward for K, V <= 128. Optional sequence segments (fixed-length
-// sequences): seg_state [N, NS, H, K, V] f32 and seg_gam [N, NS, H, K] f32 workspaces.
+// columns), the fused backward for K, V <= 128. Optional sequence segments: seg_state
+// [slots, H, K, V] f32 and seg_gam [slots, H, K] f32 workspaces; fixed-length sequences NS
+// segments of SL chunks (slots N NS), varlen ones (NS 1, SL > 0) segments of at most SL
+// chunks (slots NC / SL + 1).
 bool head_supported(int dtype, int C, int K, int V, bool g_is_cumsum);   // scans, forward
 bool head_bwd_supported(int K, int V);                                     // + backward
 int head_vtiles(int K, int V);   // V tiles (blocks per segment and head)
 void head_seg_plan(int N, int H, int T, int C, bool varlen, int& NS, int& SL, int VT);
-long head_seg_ws_bytes(int N, int NS, int H, int K, int V);
-long head_gate_ws_bytes(int N, int T, int H, int K, int V);   // 0 unless it pays
+int head_varlen_seg(int N, long nc, int H, int VT);   // varlen: chunks of a segment, or 0
+long head_seg_ws_bytes(long slots, int H, int K, int V);
+long head_gate_ws_bytes(long nc, int H, int K, int V);   // 0 unless it pays
 
 // Full-head kernels. Gates: g ([T, H, K] bf16, raw) or, with g == nullptr, the scalar
 // gates of simple GLA: gate(t, h) = gs[t * gs_ts + h] for every key column (float; gs_ts = H
@@ -257,7 +263,7 @@ struct HeadScanArgs {
   const float* s_init;    // forward: h0 ; reverse: dht (nullable)
   void* s_all;            // per-chunk states [NC, H, K, V] bf16 (nullable)
   float* s_final;         // forward: ht ; reverse: dh0 (nullable)
-  float* seg_state;       // NS > 1 only
+  float* seg_state;       // segmented only
   float* seg_gam;
   int NS, SL;
   int pass, s_begin, ns_launch;   // set by the launcher
@@ -279,7 +285,7 @@ struct HeadFwdArgs {
   void* h_out;            // [NC, H, K, V] bf16 (nullable)
   void* gate_ws;          // per-chunk gating workspace of wide heads (nullable; fixed length)
   float* ht;              // nullable
-  float* seg_state;       // NS > 1 only
+  float* seg_state;       // segmented only
   float* seg_gam;
   int NS, SL;
   float scale;
@@ -302,7 +308,7 @@ struct HeadBwdArgs {
   const float* dht;       // nullable
   void *dq, *dk, *dv, *dg;  // dg nullable with scalar gates
   float* dh0;             // nullable
-  float* seg_state;       // NS > 1 only
+  float* seg_state;       // segmented only
   float* seg_gam;
   int NS, SL;
   float scale;

@@ -158,9 +158,10 @@ __device__ __forceinline__ void put(void* p, long i, float x) {
 __device__ __forceinline__ bool pair_flagged(const GateFlags& f, int seq, int hh, int H) {
   long s0 = (long)seq * f.ns;
   int n = f.ns * f.vt;
-  if (f.co) {   // per-chunk flags of varlen sequences
-    s0 = f.co[seq];
-    n = (f.co[seq + 1] - f.co[seq]) * f.vt;
+  if (f.co) {   // varlen sequences: per-chunk flags, or per-block ones of segments
+    const int c0 = f.co[seq], nc = f.co[seq + 1] - c0;
+    s0 = f.sl > 0 ? c0 / f.sl + seq : c0;
+    n = (f.sl > 0 ? (nc + f.sl - 1) / f.sl : nc) * f.vt;
   }
   int x = 0;
   for (int i = (int)(threadIdx.x & 63); i < n; i += 64)

@@ -149,7 +149,7 @@ def seg_workspace(B, T, H, K, V, chunk, varlen, dtype, device, N=None, backward=
     (or a true value with ``N`` given), else falsy."""
     if N is None:
         N = len(varlen) - 1 if isinstance(varlen, (list, tuple)) else B
-    n = int(load().tops_gla_chunk_ws_bytes(B, T, H, K, V, chunk, N, int(bool(varlen)),
+    n = int(load().tops_gla_chunk_ws_bytes(B, T, H, K, V, chunk, N, 2 if varlen else 0,
                                            dtype_code(dtype), int(bool(backward))))
     if n <= 0:
         return None, 0

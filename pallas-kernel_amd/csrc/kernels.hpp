@@ -170,6 +170,11 @@ struct RecScanArgs {
   SeqInfo si;  // C unused
   GateFlags flags;   // nullable: only the flagged (sequence, head) pairs run
 };
+// Forward scans of bf16 inputs with row gates alone (or none), on the matrix cores 16 tokens
+// at a time (recurrent_chunk.hip): no gate-gradient epilogue, transposed state, shifted gates
+// or flags, float32 output, at most 256 rows.
+bool rec_chunk_supported(const RecScanArgs& p, int dtype, int o_dtype);
+hipError_t run_rec_chunk(const RecScanArgs& p, hipStream_t st);
 struct RecBwdArgs {
   const void *q, *k, *v, *gk, *gv, *dout;  // gk / gv nullable
   const float* o;                          // forward output f32 (needed with gv)

@@ -1,0 +1,89 @@
+"""GPU parity of fused_recurrent_gla's bf16 forward on the matrix cores (16 tokens at a time;
+sequences of 24 tokens and more, packed ones of 24 on average) against the oracle, at the float32 bar (max-abs error <= 1e-4) and at the sizes where its tiles
+end: tokens around multiples of 16, key sizes around 64 / 128 / 256 and odd ones (element
+loads), column counts around the 16-column tiles and the 64- and 128-column blocks, packed
+sequences of one token, reversed order; gates beyond the factoring's range and non-finite
+inputs, which it takes token by token."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as orc
+from gla_cases import check, logsigmoid, round_bf16, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    dict(B=1, T=24, H=1, K=16, V=1),
+    dict(B=2, T=31, H=3, K=63, V=17),
+    dict(B=1, T=32, H=2, K=64, V=64, reverse=True),
+    dict(B=1, T=33, H=2, K=65, V=65),
+    dict(B=3, T=49, H=1, K=128, V=128),
+    dict(B=1, T=47, H=2, K=130, V=40, reverse=True),
+    dict(B=1, T=100, H=1, K=256, V=130),
+    dict(B=40, T=31, H=8, K=72, V=136),                    # 32 columns a wave, partial tiles
+    dict(B=64, T=40, H=5, K=40, V=128, gate="none"),
+    dict(B=1, T=170, H=2, K=96, V=96, cu=[0, 1, 2, 18, 35, 36, 170]),
+    dict(B=1, T=90, H=2, K=33, V=20, cu=[0, 16, 69, 70], reverse=True),   # tokens past the last
+    dict(B=1, T=90, H=2, K=128, V=70, gate_mul=12.0),      # every chunk beyond the range
+    dict(B=1, T=150, H=2, K=256, V=64, strong=(37, 60)),   # some chunks
+    dict(B=2, T=80, H=1, K=64, V=32, strong=(20, 21), reverse=True),
+    dict(B=1, T=23, H=2, K=64, V=64),                      # below: the VALU scan
+]
+
+
+def _inputs(c, seed=11):
+    r = np.random.default_rng(seed)
+    B, T, H, K, V = (c[n] for n in "BTHKV")
+    q, k, v = (round_bf16(r.standard_normal((B, T, H, D))) for D in (K, K, V))
+    g = logsigmoid(r.standard_normal((B, T, H, K))) * c.get("gate_mul", 1.0) / (
+        1.0 if "gate_mul" in c else 4.0)
+    if "strong" in c:
+        g[:, slice(*c["strong"])] -= 30.0
+    g = None if c.get("gate") == "none" else round_bf16(g)
+    N = len(c["cu"]) - 1 if "cu" in c else B
+    return q, k, v, g, r.standard_normal((N, H, K, V))
+
+
+def _call(q, k, v, g, s0, c):
+    import tops.ops.gla as G
+
+    d = lambda x: None if x is None else to_dev(x, "bf16")  # noqa: E731
+    cu = c.get("cu")
+    o, ht = G.fused_recurrent_gla(d(q), d(k), d(v), gk=d(g), initial_state=to_dev(s0, "state"),
+                                  output_final_state=True, reverse=c.get("reverse", False),
+                                  cu_seqlens=None if cu is None else torch.tensor(cu))
+    torch.cuda.synchronize()
+    return to_np(o), to_np(ht)
+
+
+def _oracle(q, k, v, g, s0, c):
+    return orc.fused_recurrent_gla(q, k, v, gk=g, initial_state=s0, output_final_state=True,
+                                   reverse=c.get("reverse", False), cu_seqlens=c.get("cu"))
+
+
+@pytest.mark.parametrize("c", CASES, ids=lambda c: "-".join(f"{a}{b}" for a, b in c.items()))
+def test_recurrent_chunk(c):
+    print(f"recurrent chunk {c}", flush=True)
+    x = _inputs(c)
+    for name, got, ref in zip(("o", "ht"), _call(*x, c), _oracle(*x, c)):
+        check(name, got, ref, "f32")
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "g", "s0"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_recurrent_chunk_non_finite(where, value):
+    """A non-finite input reaches the outputs that the recurrence carries it to, and no other
+    (a gate of -inf clears its row of the state)."""
+    c = dict(B=1, T=50, H=2, K=64, V=40)
+    x = dict(zip(("q", "k", "v", "g", "s0"), _inputs(c)))
+    x[where][(0, 1, 21, 3) if where == "s0" else (0, 21, 1, 3)] = value
+    print(f"recurrent chunk, {value} in {where}", flush=True)
+    args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
+    with np.errstate(all="ignore"):
+        refs = _oracle(*args, c)
+    for name, got, ref in zip(("o", "ht"), _call(*args, c), refs):
+        assert np.array_equal(np.isfinite(got), np.isfinite(ref)), name
+        m = np.isfinite(ref)
+        check(name, got[m], ref[m], "f32")

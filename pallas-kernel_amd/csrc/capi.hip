@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "../../include/tops_gla.h"
+#include "../../include/tops_gla_layer.h"
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -1494,6 +1495,52 @@ int tops_gla_concat_cols(const void* const* srcs, const int64_t* widths, int nsr
   return hip_status(tops::run_concat_cols(srcs, w, nsrc, (long)rows, dst, es,
                                           (hipStream_t)stream),
                     "concat_cols");
+}
+
+int tops_gla_small_linear(const void* x, int x_dtype, const void* const* ws, const int64_t* ns,
+                          int nw, int64_t M, int64_t K, void* const* ys, int f32_mask,
+                          void* stream) {
+  if (!dtype_ok(x_dtype)) return fail(TOPS_GLA_EINVAL, "bad dtype");
+  if (nw < 1 || nw > tops::kSmallMaxW || ws == nullptr || ns == nullptr || ys == nullptr)
+    return fail(TOPS_GLA_EINVAL, "nw must be in [1, 8], ws, ns and ys set");
+  if (M < 0 || M > tops::kSmallMaxM)
+    return fail(TOPS_GLA_EUNSUPPORTED, "M must be in [0, 128] (M=%lld)", (long long)M);
+  if (K <= 0 || K % 256 != 0 || K > (1 << 20))
+    return fail(TOPS_GLA_EUNSUPPORTED, "K must be a positive multiple of 256 (K=%lld)",
+                (long long)K);
+  tops::SmallLinearArgs p = {};
+  if (M > 0 && (x == nullptr || !aligned16(x)))
+    return fail(TOPS_GLA_EINVAL, "x must be non-NULL and 16-byte aligned");
+  for (int i = 0; i < nw; ++i) {
+    if (ns[i] <= 0 || ns[i] % 4 != 0 || ns[i] > (1 << 24))
+      return fail(TOPS_GLA_EUNSUPPORTED, "every n must be a positive multiple of 4");
+    if (M > 0 && (ws[i] == nullptr || ys[i] == nullptr || !aligned16(ws[i]) || !aligned16(ys[i])))
+      return fail(TOPS_GLA_EINVAL, "weights and outputs must be non-NULL and 16-byte aligned");
+    p.w[i] = ws[i];
+    p.y[i] = ys[i];
+    p.n[i] = (int)ns[i];
+  }
+  p.x = x;
+  p.nw = nw;
+  p.M = (int)M;
+  p.K = (int)K;
+  p.f32_mask = f32_mask;
+  return hip_status(tops::run_small_linear(p, x_dtype, (hipStream_t)stream), "small_linear");
+}
+
+int tops_gla_low_rank_gate(const void* x, const void* w, const void* bias, void* y, int64_t M,
+                           int64_t N, int R, float normalizer, int has_clamp, float clamp_min,
+                           void* stream) {
+  if (M < 0 || N < 0 || M > (1 << 16) || N > (1 << 24) || normalizer == 0.f)
+    return fail(TOPS_GLA_EINVAL, "bad M, N or normalizer");
+  if (R <= 0 || R % 8 != 0 || R > 4096)
+    return fail(TOPS_GLA_EUNSUPPORTED, "R must be a positive multiple of 8 (R=%d)", R);
+  if (M * N > 0 && (x == nullptr || w == nullptr || y == nullptr || !aligned16(x) ||
+                    !aligned16(w)))
+    return fail(TOPS_GLA_EINVAL, "x, w and y must be non-NULL, x and w 16-byte aligned");
+  return hip_status(tops::run_low_rank_gate(x, w, bias, y, (int)M, (int)N, R, 1.f / normalizer,
+                                            has_clamp, clamp_min, (hipStream_t)stream),
+                    "low_rank_gate");
 }
 
 int tops_gla_gate_logsigmoid_bwd(const void* x, const void* dy, void* dx, int64_t count,

@@ -226,6 +226,24 @@ constexpr int kConcatMax = 8;
 hipError_t run_concat_cols(const void* const* src, const long* widths, int nsrc, long rows,
                            void* dst, int esize, hipStream_t st);
 
+// y_i [M, n_i] = x [M, K] W_i^T for M <= kSmallMaxM rows, W_i [n_i, K] bf16 (small_linear.hip);
+// K % 256 == 0, n_i % 4 == 0, 16-byte aligned pointers. bf16 x: bf16 y_i (bit i of f32_mask: the
+// rounded values as float32); float32 x: float32 y_i.
+constexpr int kSmallMaxW = 8, kSmallMaxM = 128;
+struct SmallLinearArgs {
+  const void* x;
+  const void* w[kSmallMaxW];
+  void* y[kSmallMaxW];
+  int n[kSmallMaxW];
+  int nw, M, K;
+  int f32_mask;
+};
+hipError_t run_small_linear(const SmallLinearArgs& p, int x_dtype, hipStream_t st);
+// y [M, N] = max(log_sigmoid(x [M, R] w [N, R]^T + bias) inv_n, clamp), bf16, R % 8 == 0.
+hipError_t run_low_rank_gate(const void* x, const void* w, const void* bias, void* y, int M,
+                             int N, int R, float inv_n, int has_clamp, float clamp,
+                             hipStream_t st);
+
 // Causal depthwise convolution with optional bias and SiLU (short_conv.hip).
 struct ShortConvArgs {
   const void *x, *dy;   // [tokens, D] input dtype

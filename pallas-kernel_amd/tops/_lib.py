@@ -75,6 +75,12 @@ _SIGS = {
 _SIGS["tops_gla_kernel_timing"] = [_I]
 _SIGS["tops_gla_kernel_ms"] = [_I]
 
+# the layer's decode entry points (order of include/tops_gla_layer.h)
+_LAYER_SIGS = {
+    "tops_gla_small_linear": [_P, _I, _P, _P, _I, _I64, _I64, _P, _I, _P],
+    "tops_gla_low_rank_gate": [_P, _P, _P, _P, _I64, _I64, _I, _F, _I, _F, _P],
+}
+
 # entry points that do not return a status code
 _RESTYPE = {"tops_gla_chunk_ws_bytes": ctypes.c_int64, "tops_gla_kernel_ms": ctypes.c_float,
             "tops_gla_rmsnorm_ws_bytes": ctypes.c_int64,
@@ -116,7 +122,7 @@ def load():
             lib.tops_gla_last_error.argtypes = []
             lib.tops_gla_version.restype = ctypes.c_char_p
             lib.tops_gla_version.argtypes = []
-            for name, args in _SIGS.items():
+            for name, args in (*_SIGS.items(), *_LAYER_SIGS.items()):
                 fn = getattr(lib, name)
                 fn.argtypes = args
                 fn.restype = _RESTYPE.get(name, ctypes.c_int)

@@ -194,6 +194,61 @@ class _FanOutLinear(torch.autograd.Function):
         return (dx, *dws)
 
 
+def _small_rows(x):
+    """x as the few-row kernels take it: at most 128 rows of a multiple of 256 features, whole
+    16-byte rows in place, and nothing that an F.linear call would see beyond the values
+    (subclass, autocast)."""
+    return (type(x) is torch.Tensor and x.is_cuda and x.is_contiguous()
+            and x.dtype in (torch.bfloat16, torch.float32)
+            and x.shape[-1] % 256 == 0 and 0 < x.numel() // x.shape[-1] <= 128
+            and x.data_ptr() % 16 == 0 and not torch.is_autocast_enabled())
+
+
+def _plain_linear(m, x, bias=False):
+    """Whether calling module ``m`` on x is exactly x W^T (+ bias) with a bfloat16 weight: our
+    Linear, no hooks, no parametrization."""
+    w = m.weight if type(m) is Linear else None
+    return (w is not None and w.dtype == torch.bfloat16 and (m.bias is None or bias)
+            and type(w) is torch.nn.Parameter and w.device == x.device and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
+            and not m._forward_hooks and not m._forward_pre_hooks)
+
+
+def _small_linear(x, weights, f32_outputs=()):
+    """``[F.linear(x, w) for w in weights]`` (bfloat16 weights) for a few rows, in one launch:
+    a decode step's projections read their weights once and cost one launch instead of a
+    library call each. float32 x gives float32 results; outputs in ``f32_outputs`` hold the
+    bfloat16 results as float32."""
+    import ctypes
+
+    from .._lib import call, dtype_code, stream_of
+
+    rows = x.numel() // x.shape[-1]
+    ys = [torch.empty(*x.shape[:-1], w.shape[0], device=x.device,
+                      dtype=torch.float32 if i in f32_outputs else x.dtype)
+          for i, w in enumerate(weights)]
+    n = len(weights)
+    call("tops_gla_small_linear", ctypes.c_void_p(x.data_ptr()), dtype_code(x.dtype),
+         (ctypes.c_void_p * n)(*[w.data_ptr() for w in weights]),
+         (ctypes.c_int64 * n)(*[w.shape[0] for w in weights]), n, rows, x.shape[-1],
+         (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys]),
+         sum(1 << i for i in f32_outputs), stream_of(x.device))
+    return ys
+
+
+def _low_rank_gate(x, up, normalizer, clamp_min):
+    """``GateLogSigmoidFn(up(x))`` for a few rows, bfloat16, in one launch."""
+    from .._lib import call, ptr, stream_of
+
+    w, b = up.weight, up.bias
+    rows = x.numel() // x.shape[-1]
+    y = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype, device=x.device)
+    has = clamp_min is not None
+    call("tops_gla_low_rank_gate", ptr(x), ptr(w), ptr(b), ptr(y), rows, w.shape[0], w.shape[1],
+         float(normalizer), int(has), float(clamp_min if has else 0.0), stream_of(x.device))
+    return y
+
+
 def _to_heads(x, head_dim):
     """... (h d) -> ... h d"""
     return x.reshape(*x.shape[:-1], x.shape[-1] // head_dim, head_dim)
@@ -326,10 +381,30 @@ class GatedLinearAttention(torch.nn.Module):
         if self.use_output_gate:
             lins.append(self.g_proj)
         g = None
-        if (torch.is_grad_enabled()
+        gate_done = False   # gk already went through the log-sigmoid gate
+        up = self.gk_proj[1]
+        if (not torch.is_grad_enabled() and _small_rows(hidden_states)
+                and hidden_states.dtype == torch.bfloat16
+                and all(_plain_linear(m, hidden_states) for m in lins)):
+            # a few rows without gradients (decode): one launch for the projections, the low-rank
+            # gate's second matrix and its activation in another; the output gate comes in
+            # float32 where the float32 output of the recurrent kernel meets it
+            f32_g = self.use_output_gate and self.fuse_norm_and_gate and mode == "fused_recurrent"
+            ys = _small_linear(hidden_states, [m.weight for m in lins], (4,) if f32_g else ())
+            q, k, v = ys[0], ys[1], ys[2]
+            if self.use_output_gate:
+                g = ys[4]
+            gate_done = (type(self.gk_proj) is torch.nn.Sequential
+                         and len(self.gk_proj) == 2 and not self.gk_proj._forward_hooks
+                         and not self.gk_proj._forward_pre_hooks
+                         and _plain_linear(up, hidden_states, bias=True)
+                         and up.weight.shape[1] % 8 == 0
+                         and (up.bias is None or up.bias.dtype == torch.bfloat16))
+            gk = (_low_rank_gate(ys[3], up, self.gate_logit_normalizer, self.clamp_min)
+                  if gate_done else up(ys[3]))
+        elif (torch.is_grad_enabled()
                 and all(m.bias is None and m.weight.dtype == hidden_states.dtype for m in lins)):
             ys = _FanOutLinear.apply(hidden_states, *[m.weight for m in lins])
-            up = self.gk_proj[1]
             q, k, v = ys[0], ys[1], ys[2]
             gk = (_NarrowLinear.apply(ys[3], up.weight, up.bias)
                   if up.weight.dtype == hidden_states.dtype and (
@@ -364,7 +439,8 @@ class GatedLinearAttention(torch.nn.Module):
             gk = _to_heads(gk, self.head_k_dim)
             v = _to_heads(v, self.head_v_dim)
 
-        gk = GateLogSigmoidFn.apply(gk, self.gate_logit_normalizer, self.clamp_min)
+        if not gate_done:
+            gk = GateLogSigmoidFn.apply(gk, self.gate_logit_normalizer, self.clamp_min)
 
         if self.feature_map_fn is not None:
             q = self.feature_map_fn(q)
@@ -406,5 +482,8 @@ class GatedLinearAttention(torch.nn.Module):
                 o = o * self.gate_fn_act(g)
         else:
             o = _from_heads(self.g_norm(o))
-        o = self.o_proj(o)
+        if (not torch.is_grad_enabled() and _small_rows(o) and _plain_linear(self.o_proj, o)):
+            o = _small_linear(o, [self.o_proj.weight])[0]
+        else:
+            o = self.o_proj(o)
         return o, None, past_key_values

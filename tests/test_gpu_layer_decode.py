@@ -1,0 +1,105 @@
+"""The layer's few-row kernels: projections and low-rank gate against float64, and the decode
+step through them against the same layer taking one library call per projection."""
+
+import pytest
+import torch
+
+
+def _close(got, ref, tol):
+    err = (got.double() - ref).abs().max().item() / ref.abs().max().item()
+    assert err <= tol, err
+
+
+# rows around the 16-row tiles; weight rows below, at and above a 16-row tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 64, 65, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_small_linear(rows, dtype):
+    from tops.layers.gla import _small_linear
+
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    for K in (256, 1280):
+        print(f"small linear rows {rows} K {K} {dtype}", flush=True)
+        x = torch.randn(rows, K, generator=gen, device="cuda").to(dtype)
+        ws = [torch.randn(n, K, generator=gen, device="cuda").bfloat16() for n in (4, 16, 100)]
+        ys = _small_linear(x, ws, (1,) if dtype == torch.bfloat16 else ())
+        for i, (y, w) in enumerate(zip(ys, ws)):
+            ref = x.double() @ w.double().t()
+            if dtype == torch.float32:   # float32 sums of K products
+                assert y.dtype == torch.float32
+                _close(y, ref, 1e-6)
+            else:   # one rounding to bf16
+                assert y.dtype == (torch.float32 if i == 1 else torch.bfloat16)
+                assert torch.equal(y.bfloat16().to(y.dtype), y)
+                _close(y, ref, 2 ** -8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,clamp,bias", [(1, 256, None, True), (5, 300, -0.03, True),
+                                               (128, 1024, None, False)])
+def test_low_rank_gate(rows, n, clamp, bias):
+    from tops.layers.gla import Linear, _low_rank_gate
+    from tops.modules._norm import GateLogSigmoidFn
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    up = Linear(16, n, bias, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        for p in up.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen, device="cuda"))
+        x = torch.randn(1, rows, 16, generator=gen, device="cuda").bfloat16()
+        y = _low_rank_gate(x, up, 16.0, clamp)
+        # the product may round to the next bf16: then so may the gate
+        ref = GateLogSigmoidFn.apply(up(x), 16.0, clamp)
+        assert y.shape == ref.shape and y.dtype == ref.dtype
+        _close(y, ref.double(), 2 ** -7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", [
+    dict(hidden_size=1024, num_heads=4),
+    dict(hidden_size=512, num_heads=4, num_kv_heads=2, use_output_gate=False),
+    dict(hidden_size=512, num_heads=2, use_short_conv=True, fuse_norm=False, clamp_min=-0.1),
+], ids=["default", "gqa-nogate", "conv-unfused"])
+@pytest.mark.parametrize("batch,tokens", [(1, 1), (33, 1), (2, 40), (1, 100)])
+def test_decode_step_matches_library_path(cfg, batch, tokens):
+    from tops.layers import GatedLinearAttention
+    from tops.layers.gla import LayerCache
+
+    m = GatedLinearAttention(rngs=3, dtype=torch.bfloat16, device="cuda", layer_idx=0, **cfg)
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    x = torch.randn(batch, tokens, cfg["hidden_size"], generator=gen, device="cuda").bfloat16()
+    outs = []
+    with torch.no_grad():
+        for hooked in (False, True):
+            if hooked:   # a hook on a projection keeps every call on the library path
+                for lin in (m.q_proj, m.gk_proj[1], m.o_proj):
+                    lin.register_forward_hook(lambda *a: None)
+            cache = LayerCache()
+            o, _, cache = m(x, past_key_values=cache, use_cache=True)
+            o2, _, cache = m(x, past_key_values=cache, use_cache=True)
+            outs.append([o, o2, cache[0]["recurrent_state"]])
+    for a, b in zip(*outs):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        _close(a, b.double(), 2e-2)
+
+
+def test_entry_points_refuse_bad_arguments():
+    """Host checks (no GPU call is made)."""
+    import ctypes
+
+    from tops import _lib
+
+    lib = _lib.load()
+    arr = lambda t, *v: (t * len(v))(*v)  # noqa: E731
+    P, I64 = ctypes.c_void_p, ctypes.c_int64
+
+    def rc(dt=1, n=64, nw=1, M=4, K=256, x=4096, w=4096):
+        return lib.tops_gla_small_linear(x, dt, arr(P, w), arr(I64, n), nw, M, K, arr(P, 4096),
+                                         0, None)
+
+    assert rc(dt=7) == 1 and rc(nw=9) == 1 and rc(x=None) == 1 and rc(w=8) == 1
+    assert rc(M=129) == 2 and rc(K=128) == 2 and rc(n=6) == 2
+    gate = lib.tops_gla_low_rank_gate
+    assert gate(4096, 4096, None, 4096, 1, 8, 12, 16.0, 0, 0.0, None) == 2
+    assert gate(4096, 4096, None, 4096, 1, 8, 16, 0.0, 0, 0.0, None) == 1
+    assert gate(None, 4096, None, 4096, 1, 8, 16, 16.0, 0, 0.0, None) == 1

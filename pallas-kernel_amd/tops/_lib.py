@@ -130,12 +130,17 @@ def load():
     return _lib
 
 
+_fns: dict = {}   # entry points by name (a lookup in the CDLL goes through its __getattr__)
+
+
 def call(name, *args):
     """Invoke ``name``; map the C status to a Python exception."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    rc = fn(*args)
     if rc != 0:
-        msg = lib.tops_gla_last_error().decode()
+        msg = load().tops_gla_last_error().decode()
         if rc == 1:
             raise ValueError(f"{name}: {msg}")
         if rc == 2:
@@ -177,6 +182,12 @@ def ptr(t):
     return p
 
 
+def addr(t):
+    """Device address of a tensor (None -> NULL) for an argument list. Unlike ``ptr`` it holds
+    no reference: the caller keeps the tensor in a variable until the entry point returns."""
+    return None if t is None else t.data_ptr()
+
+
 def dtype_code(dt):
     if dt not in _DT:
         raise TypeError(f"tops GLA kernels take float32 or bfloat16, got {dt}")
@@ -185,7 +196,7 @@ def dtype_code(dt):
 
 def check_device(*tensors):
     """All tensors on one ROCm device; returns it."""
-    dev = None
+    dev = index = None
     for t in tensors:
         if t is None:
             continue
@@ -193,14 +204,26 @@ def check_device(*tensors):
             raise RuntimeError(
                 "tops GLA runs only on a ROCm GPU (tensor on %s); there is no CPU path" % t.device)
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
     return dev
 
 
+def _stream_address(device):
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+# the stream's address alone, where torch offers it: building the Stream object costs more than
+# the rest of a small call's argument list
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """torch's current stream of a device (with an index, as a tensor's is)."""
+    if _raw_stream is None or device.index is None:
+        return ctypes.c_void_p(_stream_address(device))
+    return ctypes.c_void_p(_raw_stream(device.index))
 
 
 class SeqLayout:

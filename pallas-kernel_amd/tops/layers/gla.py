@@ -207,9 +207,12 @@ def _small_rows(x):
 def _plain_linear(m, x, bias=False):
     """Whether calling module ``m`` on x is exactly x W^T (+ bias) with a bfloat16 weight: our
     Linear, no hooks, no parametrization."""
-    w = m.weight if type(m) is Linear else None
-    return (w is not None and w.dtype == torch.bfloat16 and (m.bias is None or bias)
-            and type(w) is torch.nn.Parameter and w.device == x.device and w.is_contiguous()
+    if type(m) is not Linear:
+        return False
+    w, b = m._parameters.get("weight"), m._parameters.get("bias")
+    return (w is not None and w.dtype == torch.bfloat16 and (b is None or bias)
+            and type(w) is torch.nn.Parameter and w.get_device() == x.get_device()
+            and w.is_contiguous()
             and w.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
             and not m._forward_hooks and not m._forward_pre_hooks)
 

@@ -13,26 +13,40 @@ def _io_dtype(x):
     return x.dtype if x.dtype in (torch.float32, torch.bfloat16) else torch.float32
 
 
+def rms_norm_gated(x, g, w, eps):
+    """``RMSNormGatedFn.apply``; without gradients (and outside forward-mode differentiation)
+    its forward alone, which keeps nothing for a backward."""
+    if torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0:
+        return RMSNormGatedFn.apply(x, g, w, eps)
+    return _rms_norm_gated_fwd(x, g, w, eps, False)[0]
+
+
+def _rms_norm_gated_fwd(x, g, w, eps, keep):
+    """(y, x, g, w as the kernel reads them, rstd or None)."""
+    dev = check_device(x, g, w)
+    dt = _io_dtype(x)
+    D = x.shape[-1]
+    xx = x.to(dt).contiguous()
+    gg = None if g is None else g.to(dt).contiguous()
+    ww = None if w is None else w.to(torch.float32).contiguous()
+    rows = xx.numel() // D if D else 0
+    y = torch.empty_like(xx)
+    rstd = torch.empty(rows, dtype=torch.float32, device=dev) if keep else None
+    call("tops_gla_rmsnorm_gated_fwd", ptr(xx), ptr(gg), ptr(ww), ptr(y), ptr(rstd), rows, D,
+         float(eps), dtype_code(dt), stream_of(dev))
+    return y.to(x.dtype), xx, gg, ww, rstd
+
+
 class RMSNormGatedFn(torch.autograd.Function):
     """y = x rsqrt(mean(x^2) + eps) [* w] [* silu(g)] over the last dimension, computed in
     float32, returned in x's dtype."""
 
     @staticmethod
     def forward(ctx, x, g, w, eps):
-        dev = check_device(x, g, w)
-        dt = _io_dtype(x)
-        D = x.shape[-1]
-        xx = x.to(dt).contiguous()
-        gg = None if g is None else g.to(dt).contiguous()
-        ww = None if w is None else w.to(torch.float32).contiguous()
-        rows = xx.numel() // D if D else 0
-        y = torch.empty_like(xx)
-        rstd = torch.empty(rows, dtype=torch.float32, device=dev)
-        call("tops_gla_rmsnorm_gated_fwd", ptr(xx), ptr(gg), ptr(ww), ptr(y), ptr(rstd), rows, D,
-             float(eps), dtype_code(dt), stream_of(dev))
+        y, xx, gg, ww, rstd = _rms_norm_gated_fwd(x, g, w, eps, True)
         ctx.save_for_backward(xx, gg, ww, rstd)
         ctx.meta = (x.dtype, None if g is None else g.dtype, None if w is None else w.dtype)
-        return y.to(x.dtype)
+        return y
 
     @staticmethod
     def backward(ctx, dy):

@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import torch
 
-from ._norm import RMSNormGatedFn
+from ._norm import rms_norm_gated
 
 
 class FusedRMSNormGated(torch.nn.Module):
@@ -28,4 +28,4 @@ class FusedRMSNormGated(torch.nn.Module):
             self.register_parameter("weight", None)
 
     def forward(self, x, g):
-        return RMSNormGatedFn.apply(x, g, self.weight, self.eps)
+        return rms_norm_gated(x, g, self.weight, self.eps)

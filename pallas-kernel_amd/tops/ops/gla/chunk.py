@@ -18,7 +18,8 @@ import math
 import torch
 
 from ... import _lib
-from ..._lib import SeqLayout, call, check_device, dtype_code, ptr, require, stream_of
+from ..._lib import (SeqLayout, addr, call, check_device, dtype_code, ptr, require,
+                     stream_of)
 from ...utils import pad_to_multiple
 
 __all__ = [
@@ -57,8 +58,8 @@ def _kernel_chunk(chunk_size: int) -> int:
 
 def _compute_dtype(*xs):
     """bf16 if every given tensor is bf16, else float32 (f16 / mixed are upcast)."""
-    dts = {x.dtype for x in xs if x is not None}
-    return torch.bfloat16 if dts == {torch.bfloat16} else torch.float32
+    bf16 = torch.bfloat16
+    return bf16 if all(x is None or x.dtype == bf16 for x in xs) else torch.float32
 
 
 def _c(x, dt=None):
@@ -66,7 +67,7 @@ def _c(x, dt=None):
         return None
     if dt is not None and x.dtype != dt:
         x = x.to(dt)
-    return x.contiguous()
+    return x if x.is_contiguous() else x.contiguous()
 
 
 def _full_head(K, V, C, dtype, backward, *tensors):
@@ -153,8 +154,8 @@ class _ChunkGLAFunction(torch.autograd.Function):
         h_ws = (torch.empty(seq.NC, H, K, V, dtype=q.dtype, device=dev)
                 if keep or not _full_head(K, V, chunk, q.dtype, False, q, k, v, g, h0) else None)
         ws, nws = _lib.seg_workspace(B, T, H, K, V, chunk, cu_list, q.dtype, dev)
-        call("tops_gla_chunk_fwd", ptr(q), ptr(k), ptr(v), ptr(g), ptr(h0), ptr(o), ptr(ht),
-             ptr(h_ws), ptr(ws), nws, scale, B, T, H, K, V, chunk, *seq.args(), dt,
+        call("tops_gla_chunk_fwd", addr(q), addr(k), addr(v), addr(g), addr(h0), addr(o),
+             addr(ht), addr(h_ws), addr(ws), nws, scale, B, T, H, K, V, chunk, *seq.args(), dt,
              stream_of(dev))
         ctx.save_for_backward(q, k, v, g, h0, h_ws)
         ctx.meta = (scale, cu_list, chunk)
@@ -180,9 +181,9 @@ class _ChunkGLAFunction(torch.autograd.Function):
                  else torch.empty(seq.NC, H, K, V, dtype=q.dtype, device=dev))
         ws, nws = _lib.seg_workspace(B, T, H, K, V, chunk, cu_list, q.dtype, dev,
                                      backward=True)
-        call("tops_gla_chunk_bwd", ptr(q), ptr(k), ptr(v), ptr(g), ptr(h0), ptr(h_ws), ptr(do),
-             ptr(dht), ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(dh0), None, ptr(dh_ws), ptr(ws),
-             nws, scale, B, T, H, K, V, chunk, *seq.args(), dtype_code(q.dtype),
+        call("tops_gla_chunk_bwd", addr(q), addr(k), addr(v), addr(g), addr(h0), addr(h_ws),
+             addr(do), addr(dht), addr(dq), addr(dk), addr(dv), addr(dg), addr(dh0), None,
+             addr(dh_ws), addr(ws), nws, scale, B, T, H, K, V, chunk, *seq.args(), dtype_code(q.dtype),
              stream_of(dev))
         return dq, dk, dv, dg, dh0, None, None, None, None
 
@@ -295,13 +296,15 @@ def chunk_gla(q, k, v, g=None, g_gamma=None, scale=None, initial_state=None,
     dtype = q.dtype
     B, T, H, K = q.shape
     V = v.shape[-1]
-    require(k.shape == (B, T, H, K), f"Expected k shape {(B, T, H, K)}, got {tuple(k.shape)}")
-    require(v.shape[:3] == (B, T, H), f"Expected v shape {(B, T, H, V)}, got {tuple(v.shape)}")
+    if k.shape != (B, T, H, K):
+        require(False, f"Expected k shape {(B, T, H, K)}, got {tuple(k.shape)}")
+    if v.shape[:3] != (B, T, H):
+        require(False, f"Expected v shape {(B, T, H, V)}, got {tuple(v.shape)}")
     cu_list = None if cu_seqlens is None else _lib.to_list(cu_seqlens)
     N = B if cu_list is None else len(cu_list) - 1
-    if initial_state is not None:
-        require(initial_state.shape == (N, H, K, V),
-                f"Expected initial_state shape {(N, H, K, V)}, got {tuple(initial_state.shape)}")
+    if initial_state is not None and initial_state.shape != (N, H, K, V):
+        require(False, f"Expected initial_state shape {(N, H, K, V)}, got "
+                       f"{tuple(initial_state.shape)}")
     if cu_list is not None:
         cu_kept, keep = _lib.drop_empty(cu_list)
         if keep is not None:   # empty sequences: run the others, keep their initial states
@@ -319,7 +322,8 @@ def chunk_gla(q, k, v, g=None, g_gamma=None, scale=None, initial_state=None,
                                 output_final_state, cu_list)
         return o.to(dtype), (ht if output_final_state else None)
     g = _gates(g, g_gamma, q)
-    require(g.shape == (B, T, H, K), f"Expected g shape {(B, T, H, K)}, got {tuple(g.shape)}")
+    if g.shape != (B, T, H, K):
+        require(False, f"Expected g shape {(B, T, H, K)}, got {tuple(g.shape)}")
     cdt = _compute_dtype(q, k, v, g)
     o, ht = _ChunkGLAFunction.apply(_c(q, cdt), _c(k, cdt), _c(v, cdt), _c(g, cdt),
                                     _c(initial_state, torch.float32),

@@ -10,7 +10,8 @@ from __future__ import annotations
 import torch
 
 from ... import _lib
-from ..._lib import SeqLayout, call, check_device, dtype_code, ptr, require, stream_of
+from ..._lib import (SeqLayout, addr, call, check_device, dtype_code, ptr, require,
+                     stream_of)
 
 __all__ = ["fused_recurrent_gla", "fused_recurrent_gla_fwd", "fused_recurrent_gla_bwd"]
 
@@ -23,8 +24,36 @@ def _out(B, T, H, D, dtype, dev, cu):
 
 
 def _compute_dtype(*xs):
-    xs = [x for x in xs if x is not None]
-    return torch.bfloat16 if {x.dtype for x in xs} == {torch.bfloat16} else torch.float32
+    bf16 = torch.bfloat16
+    return bf16 if all(x is None or x.dtype == bf16 for x in xs) else torch.float32
+
+
+def _as(x, dt):
+    """x as a contiguous tensor of dtype dt (None stays None)."""
+    if x is None or (x.dtype == dt and x.is_contiguous()):
+        return x
+    return x.to(dt).contiguous()
+
+
+def _check_shapes(q, k, v, gk, gv, initial_state, cu, cu_seqlens):
+    """The argument checks of the public functions; messages are formed only when one fails."""
+    B, T, H, K = q.shape
+    V = v.shape[-1]
+    if k.shape != (B, T, H, K):
+        require(False, f"Expected k shape {(B, T, H, K)}, got {k.shape}")
+    if v.shape != (B, T, H, V):
+        require(False, f"Expected v shape {(B, T, H, V)}, got {v.shape}")
+    if gk is not None and gk.shape != (B, T, H, K):
+        require(False, f"Expected gk shape {(B, T, H, K)}, got {gk.shape}")
+    if gv is not None and gv.shape != (B, T, H, V):
+        require(False, f"Expected gv shape {(B, T, H, V)}, got {gv.shape}")
+    if initial_state is not None:
+        N = len(cu) - 1 if cu is not None else B
+        if initial_state.shape != (N, H, K, V):
+            require(False, f"Expected initial_state shape {(N, H, K, V)}, got "
+                           f"{initial_state.shape}")
+    if cu_seqlens is not None and B != 1:
+        require(False, f"Batch size must be 1 when using cu_seqlens, got {B}")
 
 
 def _run(q, k, v, gk, gv, scale, initial_state, output_final_state, reverse, cu_seqlens,
@@ -33,7 +62,6 @@ def _run(q, k, v, gk, gv, scale, initial_state, output_final_state, reverse, cu_
     V = v.shape[-1]
     dev = check_device(q, k, v, gk, gv, initial_state)
     cdt = _compute_dtype(q, k, v, gk, gv)
-    c = lambda x: None if x is None else x.to(cdt).contiguous()  # noqa: E731
     odt = torch.float32 if out_dtype == torch.float32 or cdt == torch.float32 else cdt
     if cu_seqlens is not None:
         kept, keep = _lib.drop_empty(cu_seqlens)
@@ -45,14 +73,18 @@ def _run(q, k, v, gk, gv, scale, initial_state, output_final_state, reverse, cu_
                 ht = _lib.scatter_states(ht, initial_state, keep,
                                          (len(cu_seqlens) - 1, H, K, V), dev)
             return o, ht
-    seq = SeqLayout(B, T, 1, cu_seqlens, dev)
+        seq = SeqLayout(B, T, 1, cu_seqlens, dev)
+        N, cu = seq.N, seq.cu
+    else:
+        N, cu = B, None
     o = _out(B, T, H, V, odt, dev, cu_seqlens)
-    ht = torch.empty(seq.N, H, K, V, dtype=torch.float32, device=dev) if output_final_state \
-        else None
-    h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
-    call("tops_gla_fused_recurrent_fwd", ptr(c(q)), ptr(c(k)), ptr(c(v)), ptr(c(gk)),
-         ptr(c(gv)), ptr(h0), ptr(o), ptr(ht), float(scale), int(bool(reverse)), B, T, H, K, V,
-         ptr(seq.cu), seq.N, dtype_code(cdt), dtype_code(odt), stream_of(dev))
+    ht = torch.empty(N, H, K, V, dtype=torch.float32, device=dev) if output_final_state else None
+    # every tensor stays in a variable until the call has enqueued its kernels
+    q, k, v, gk, gv = _as(q, cdt), _as(k, cdt), _as(v, cdt), _as(gk, cdt), _as(gv, cdt)
+    h0 = _as(initial_state, torch.float32)
+    call("tops_gla_fused_recurrent_fwd", addr(q), addr(k), addr(v), addr(gk), addr(gv), addr(h0),
+         addr(o), addr(ht), float(scale), 1 if reverse else 0, B, T, H, K, V, addr(cu), N,
+         dtype_code(cdt), dtype_code(odt), stream_of(dev))
     return o, ht
 
 
@@ -63,22 +95,9 @@ def fused_recurrent_gla_fwd(q, k, v, gk=None, gv=None, scale=None, initial_state
     Returns ``(o, ht)``: o ``[B, T, H, V]`` float32 (as the reference, ``:262,369``), ht
     float32 ``[N, H, K, V]`` or None.
     """
-    B, T, H, K = q.shape
-    V = v.shape[-1]
     cu = None if cu_seqlens is None else _lib.to_list(cu_seqlens)
-    N = len(cu) - 1 if cu is not None else B
-    scale = scale if scale is not None else K ** -0.5
-    require(tuple(k.shape) == (B, T, H, K), f"Expected k shape {(B, T, H, K)}, got {k.shape}")
-    require(tuple(v.shape) == (B, T, H, V), f"Expected v shape {(B, T, H, V)}, got {v.shape}")
-    require((gk is None) or (tuple(gk.shape) == (B, T, H, K)),
-            f"Expected gk shape {(B, T, H, K)}, got {getattr(gk, 'shape', None)}")
-    require((gv is None) or (tuple(gv.shape) == (B, T, H, V)),
-            f"Expected gv shape {(B, T, H, V)}, got {getattr(gv, 'shape', None)}")
-    require((initial_state is None) or (tuple(initial_state.shape) == (N, H, K, V)),
-            f"Expected initial_state shape {(N, H, K, V)}, got "
-            f"{getattr(initial_state, 'shape', None)}")
-    require((cu_seqlens is None) or (B == 1),
-            f"Batch size must be 1 when using cu_seqlens, got {B}")
+    scale = scale if scale is not None else q.shape[-1] ** -0.5
+    _check_shapes(q, k, v, gk, gv, initial_state, cu, cu_seqlens)
     return _run(q, k, v, gk, gv, scale, initial_state, output_final_state, reverse, cu,
                 torch.float32)
 
@@ -123,22 +142,9 @@ def fused_recurrent_gla(q, k, v, gk=None, gv=None, scale=None, initial_state=Non
                                        initial_state=initial_state,
                                        output_final_state=output_final_state,
                                        reverse=reverse, cu_seqlens=cu_seqlens)
-    B, T, H, K = q.shape
-    V = v.shape[-1]
     cu = None if cu_seqlens is None else _lib.to_list(cu_seqlens)
-    N = len(cu) - 1 if cu is not None else B
-    require(tuple(k.shape) == (B, T, H, K), f"Expected k shape {(B, T, H, K)}, got {k.shape}")
-    require(tuple(v.shape) == (B, T, H, V), f"Expected v shape {(B, T, H, V)}, got {v.shape}")
-    require((gk is None) or (tuple(gk.shape) == (B, T, H, K)),
-            f"Expected gk shape {(B, T, H, K)}, got {getattr(gk, 'shape', None)}")
-    require((gv is None) or (tuple(gv.shape) == (B, T, H, V)),
-            f"Expected gv shape {(B, T, H, V)}, got {getattr(gv, 'shape', None)}")
-    require((initial_state is None) or (tuple(initial_state.shape) == (N, H, K, V)),
-            f"Expected initial_state shape {(N, H, K, V)}, got "
-            f"{getattr(initial_state, 'shape', None)}")
-    require((cu_seqlens is None) or (B == 1),
-            f"Batch size must be 1 when using cu_seqlens, got {B}")
-    scale = scale if scale is not None else K ** -0.5
+    _check_shapes(q, k, v, gk, gv, initial_state, cu, cu_seqlens)
+    scale = scale if scale is not None else q.shape[-1] ** -0.5
     return _FusedRecurrentGLAFunction.apply(q, k, v, gk, gv, initial_state, float(scale),
                                             bool(output_final_state), bool(reverse), cu)
 

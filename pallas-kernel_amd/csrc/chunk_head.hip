@@ -260,26 +260,13 @@ __device__ __forceinline__ void mask_rows(uint4 (&r)[N], int row0, int len, bool
   for (int j = 0; j < N; ++j) r[j] = mask16(r[j], (col_ok && row0 + j < len) ? ~0u : 0u);
 }
 
-// The block's segment: `s` of the `ns` segments of sequence `seq`, chunks [cb, ce); its
+// The block's segment: `s` of the `ns` segments of sequence `seq`, chunks [cb, ce); `unit`: the
+// segment's and head's place among the blocks (one flag per unit and V tile); its
 // sequence's local states start at workspace slot `st0` (slot of segment u: st0 + u).
 struct Seg {
-  int seq, s, ns, bos, eos, c0, cb, ce;
+  int unit, seq, s, ns, bos, eos, c0, cb, ce;
   long st0;
 };
-
-// Fixed-length sequences: NS segments of SL chunks each.
-__device__ __forceinline__ Seg seg_of(const SeqInfo& si, int seq, int s, int NS, int SL) {
-  Seg r;
-  int nc;
-  seq_range(si, seq, r.bos, r.eos, r.c0, nc);
-  r.seq = seq;
-  r.s = s;
-  r.ns = NS;
-  r.st0 = (long)seq * NS;
-  r.cb = NS > 1 ? min(nc, s * SL) : 0;
-  r.ce = NS > 1 ? min(nc, r.cb + SL) : nc;
-  return r;
-}
 
 // Varlen sequences: sequence i of nc chunks (from chunk c0 = chunk_cu[i]) has ns = ceil(nc /
 // SL) segments of nearly equal size. The launcher knows only the numbers of chunks and
@@ -312,37 +299,69 @@ __device__ __forceinline__ bool seg_of_slot(const SeqInfo& si, int slot, int SL,
   return true;
 }
 
-// Block -> (unit, V tile), unit = segment and head. The V tiles of a unit go to one XCD (its
-// L2 serves their re-reads of q / k / g). Fixed-length sequences: consecutive units on one XCD
-// (xcd_remap). Varlen: units dealt round-robin, since consecutive ones are pieces of one
-// sequence and a contiguous share per XCD would leave some XCDs with the long sequences'
-// full pieces and others with short or empty slots (the packed training shape of 13 documents
-// in 16384 tokens, 16 heads of 128 x 128, forward + backward: 699 us contiguous, 444 us dealt).
-__device__ __forceinline__ void unit_of_block(const SeqInfo& si, int SL, int VT, int& unit,
-                                              int& vt) {
-  const int L = blockIdx.x, total = gridDim.x;
-  if (si.cu && SL > 0) {
-    const int u8 = total / VT & ~7;   // units in whole rounds of 8
-    if (L < u8 * VT) {
-      unit = (L >> 3) / VT * 8 + (L & 7);
-      vt = (L >> 3) % VT;
-    } else {
-      unit = L / VT;
-      vt = L % VT;
-    }
-    return;
-  }
-  const int L0 = xcd_remap(L, total);
-  unit = L0 / VT;
-  vt = L0 % VT;
-}
-
-// Segment of block index j (of all segments; `states`: varlen pass 1, the state slots).
+// The block's segment, head and V tile (of VT); a unit is a segment and head. The V tiles of a
+// unit go to one XCD (its L2 serves their re-reads of q / k / g). False: an empty slot.
+//
+// Fixed-length sequences: NS segments of SL chunks each (a launch may hold only `nsl` of them,
+// from s_begin), consecutive units on one XCD (xcd_remap). Varlen, segmented (SL > 0): units
+// dealt round-robin, since consecutive ones are pieces of one sequence and a contiguous share
+// per XCD would leave some XCDs with the long sequences' full pieces and others with short or
+// empty slots (13 documents in 16384 tokens, 16 heads of 128 x 128, forward + backward: 699 us
+// contiguous, 444 us dealt).
+//
+// The fixed-length path is one straight run of scalar code and the varlen one is out of its
+// way: every block pays this once, its instructions cold, and with the two paths interleaved
+// the training shape's four kernels took 1-3 us more each (B4 T8192 H16 128 x 128: 725 us in
+// all against 717 us without the varlen path; as it is here 708 against 711 us).
 template <bool REV>
-__device__ __forceinline__ bool find_seg(const SeqInfo& si, int j, int NS, int SL, bool states,
-                                         Seg& r) {
-  if (si.cu && SL > 0) return seg_of_slot<REV>(si, j, SL, states, r);
-  r = seg_of(si, j / NS, j % NS, NS, SL);
+__device__ __forceinline__ bool locate_block(const SeqInfo& si, int H, int VT, int NS, int SL,
+                                             int nsl, int s_begin, bool states, int& hh,
+                                             int& vt, Seg& r) {
+  const unsigned total = gridDim.x, b = blockIdx.x;
+  unsigned unit;   // < 2^31, as gridDim
+  if (__builtin_expect(si.cu == nullptr, 1)) {
+    const unsigned L = xcd_remap(b, total);
+    unit = L / (unsigned)VT;
+    vt = L - unit * VT;
+    r.unit = unit;
+    const unsigned j = unit / (unsigned)H;
+    hh = unit - j * H;
+    const unsigned seq = j / (unsigned)nsl;
+    const int nc = (unsigned)(si.T + HC - 1) / HC;
+    r.seq = seq;
+    r.s = s_begin + (int)(j - seq * nsl);
+    r.ns = NS;
+    r.st0 = (long)seq * NS;
+    r.bos = seq * si.T;
+    r.eos = r.bos + si.T;
+    r.c0 = seq * nc;
+    r.cb = NS > 1 ? min(nc, r.s * SL) : 0;
+    r.ce = NS > 1 ? min(nc, r.cb + SL) : nc;
+    return true;
+  }
+  if (SL > 0) {
+    const unsigned u8 = total / (unsigned)VT & ~7u;   // units in whole rounds of 8
+    if (b < u8 * VT) {
+      unit = (b >> 3) / (unsigned)VT * 8 + (b & 7);
+      vt = (b >> 3) % (unsigned)VT;
+    } else {
+      unit = b / (unsigned)VT;
+      vt = b % (unsigned)VT;
+    }
+    hh = unit % (unsigned)H;
+    r.unit = unit;
+    return seg_of_slot<REV>(si, unit / (unsigned)H, SL, states, r);
+  }
+  const unsigned L = xcd_remap(b, total);
+  unit = L / (unsigned)VT;
+  vt = L % (unsigned)VT;
+  hh = unit % (unsigned)H;
+  r.unit = unit;
+  r.seq = unit / (unsigned)H;
+  seq_range(si, r.seq, r.bos, r.eos, r.c0, r.ce);
+  r.s = r.cb = 0;
+  r.ns = 1;
+  r.st0 = r.seq;
   return true;
 }
 
@@ -729,17 +748,12 @@ __global__ __launch_bounds__(NT) void head_scan_kernel(HeadScanArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
   const int VT = (V + VP - 1) / VP;            // V tiles (blocks of one segment and head)
-  int L, vt;
-  unit_of_block(p.si, p.SL, VT, L, vt);
-  const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
-  const int hh = L % H;
+  int hh, vt;
   Seg sg;
-  if (p.si.cu && p.SL > 0) {
-    if (!seg_of_slot<REV>(p.si, L / H, p.SL, p.pass == 1, sg)) return;   // uniform
-  } else {
-    const int nsl = p.ns_launch;
-    sg = seg_of(p.si, (L / H) / nsl, p.s_begin + (L / H) % nsl, p.NS, p.SL);
-  }
+  if (!locate_block<REV>(p.si, H, VT, p.NS, p.SL, p.ns_launch, p.s_begin, p.pass == 1, hh, vt,
+                         sg))
+    return;   // uniform
+  const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
   const int nsteps = CR == HC ? sg.ce - sg.cb : (sg.ce - sg.cb + 1) / 2;
   const bool first_seg = REV ? (sg.s == sg.ns - 1) : (sg.s == 0);
   const bool last_seg = REV ? (sg.s == 0) : (sg.s == sg.ns - 1);
@@ -1648,12 +1662,11 @@ __global__ __launch_bounds__(HNT) void head_fwd_kernel(HeadFwdArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
   const int VT = (V + VP - 1) / VP;            // V tiles (blocks of one segment and head)
-  int L, vt;
-  unit_of_block(p.si, p.SL, VT, L, vt);
-  const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
-  const int hh = L % H;
+  int hh, vt;
   Seg sg;
-  if (!find_seg<false>(p.si, L / H, p.NS, p.SL, false, sg)) return;   // uniform
+  if (!locate_block<false>(p.si, H, VT, p.NS, p.SL, p.NS, 0, false, hh, vt, sg))
+    return;   // uniform
+  const int cv = vt * VP, Vw = min(VP, V - cv);   // this tile's first column and width
   const int nsteps = sg.ce - sg.cb;
   const long rsK = (long)H * K, rsV = (long)H * V;
   const long KV = (long)K * V;
@@ -2102,7 +2115,7 @@ __global__ __launch_bounds__(HNT) void head_fwd_kernel(HeadFwdArgs p) {
                               lane, V);
   if (p.flags) {   // uniform; every block writes its flag, so nothing needs clearing
     const int bad = __syncthreads_or(dmax > kGateLimit2 ? 1 : 0);
-    if (tid == 0) p.flags[(long)L * VT + vt] = bad ? 1 : 0;
+    if (tid == 0) p.flags[(long)sg.unit * VT + vt] = bad ? 1 : 0;
   }
 }
 
@@ -2234,11 +2247,10 @@ __global__ __launch_bounds__(NT) void head_bwd_kernel(HeadBwdArgs p) {
   const int H = p.H, K = p.K, V = p.V;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, scalar
-  int L, vtile;
-  unit_of_block(p.si, p.SL, 1, L, vtile);
-  const int hh = L % H;
+  int hh, vt;
   Seg sg;
-  if (!find_seg<true>(p.si, L / H, p.NS, p.SL, false, sg)) return;   // uniform
+  if (!locate_block<true>(p.si, H, 1, p.NS, p.SL, p.NS, 0, false, hh, vt, sg))
+    return;   // uniform
   const int nsteps = sg.ce - sg.cb;
   const long rsK = (long)H * K, rsV = (long)H * V;
   const long KV = (long)K * V;
@@ -2788,7 +2800,7 @@ __global__ __launch_bounds__(NT) void head_bwd_kernel(HeadBwdArgs p) {
     store_state_f32<NTV, NTK>(acc, p.dh0 + ((long)sg.seq * H + hh) * KV, K, V, vt0, kt0, lane);
   if (p.flags) {   // uniform; every block writes its flag, so nothing needs clearing
     const int bad = __syncthreads_or(gbad);
-    if (tid == 0) p.flags[L] = bad ? 1 : 0;
+    if (tid == 0) p.flags[sg.unit] = bad ? 1 : 0;
   }
 }
 

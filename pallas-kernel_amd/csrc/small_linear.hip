@@ -24,21 +24,30 @@ namespace {
 
 constexpr int SLW = 8;              // waves per block, each an eighth of K
 constexpr int SLT = SLW * 64;
+constexpr float kBf16Max = 3.38953139e38f;   // 0x7f7f0000
 constexpr int SLP = 20;             // LDS row pitch: the 16 rows of a store spread over the banks
 
-// Eight floats as three bf16 fragments that sum to them exactly.
+// Eight floats as three bf16 fragments that sum to them exactly. An infinity or NaN is the
+// first part alone (the rest would be inf - inf), and a finite value that rounds to an infinity
+// (from 0x7f7f8000) starts with the largest bf16 instead.
 __device__ __forceinline__ void split8(const float (&x)[8], Frag<bf16> (&f)[3]) {
   float y[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] = x[e];
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t m = __float_as_uint(x[e]) & 0x7fffffffu;
+    const bool finite = m < 0x7f800000u;
+    y[e] = finite ? (m >= 0x7f7f8000u ? copysignf(kBf16Max, x[e]) : x[e]) : x[e];
+  }
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      w[e] = pack2_bf16(y[2 * e], y[2 * e + 1]);
-      y[2 * e] -= bf16_lo(w[e]);
-      y[2 * e + 1] -= bf16_hi(w[e]);
+    for (int e = 0; e < 4; ++e) w[e] = pack2_bf16(y[2 * e], y[2 * e + 1]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float hi = e & 1 ? bf16_hi(w[e / 2]) : bf16_lo(w[e / 2]);
+      const bool finite = (__float_as_uint(x[e]) & 0x7fffffffu) < 0x7f800000u;
+      y[e] = finite ? (i == 0 ? x[e] : y[e]) - hi : 0.f;
     }
     f[i].d = make_uint4(w[0], w[1], w[2], w[3]);
   }

@@ -15,6 +15,7 @@ from typing import Any
 
 import torch
 import torch.nn.functional as F
+from torch.nn.modules import module as _modules
 
 from .._lib import require
 from ..modules import FusedRMSNormGated, RMSNorm
@@ -197,24 +198,46 @@ class _FanOutLinear(torch.autograd.Function):
 def _small_rows(x):
     """x as the few-row kernels take it: at most 128 rows of a multiple of 256 features, whole
     16-byte rows in place, and nothing that an F.linear call would see beyond the values
-    (subclass, autocast)."""
+    (subclass, autocast, forward-mode tangents, hooks on every module)."""
     return (type(x) is torch.Tensor and x.is_cuda and x.is_contiguous()
             and x.dtype in (torch.bfloat16, torch.float32)
             and x.shape[-1] % 256 == 0 and 0 < x.numel() // x.shape[-1] <= 128
-            and x.data_ptr() % 16 == 0 and not torch.is_autocast_enabled())
+            and x.data_ptr() % 16 == 0 and not torch.is_autocast_enabled()
+            and torch.autograd.forward_ad._current_level < 0
+            and not _modules._global_forward_hooks and not _modules._global_forward_pre_hooks)
 
 
-def _plain_linear(m, x, bias=False):
-    """Whether calling module ``m`` on x is exactly x W^T (+ bias) with a bfloat16 weight: our
-    Linear, no hooks, no parametrization."""
-    if type(m) is not Linear:
+def _unhooked(m):
+    """Whether calling the module runs its class's forward and nothing else."""
+    return not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+
+
+def _plain_linear(m, x):
+    """Whether calling module ``m`` on x is exactly x W^T with a bfloat16 weight of x's width:
+    our Linear, no hooks, no parametrization."""
+    if type(m) is not Linear or m._parameters.get("bias") is not None:
         return False
-    w, b = m._parameters.get("weight"), m._parameters.get("bias")
-    return (w is not None and w.dtype == torch.bfloat16 and (b is None or bias)
-            and type(w) is torch.nn.Parameter and w.get_device() == x.get_device()
-            and w.is_contiguous()
-            and w.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
-            and not m._forward_hooks and not m._forward_pre_hooks)
+    w = m._parameters.get("weight")
+    return (w is not None and _plain_matrix(w, x.shape[-1], x.get_device())
+            and w.shape[0] % 4 == 0 and _unhooked(m))
+
+
+def _plain_matrix(w, features, device):
+    return (type(w) is torch.nn.Parameter and w.dtype == torch.bfloat16 and w.dim() == 2
+            and w.shape[1] == features and w.get_device() == device and w.is_contiguous()
+            and w.data_ptr() % 16 == 0)
+
+
+def _plain_gate(up, x):
+    """Whether the low-rank gate's second module is exactly x W^T (+ bias) in bfloat16."""
+    if type(up) is not Linear or not _unhooked(up):
+        return False
+    w, b = up._parameters.get("weight"), up._parameters.get("bias")
+    return (w is not None and _plain_matrix(w, x.shape[-1], x.get_device())
+            and w.shape[1] % 8 == 0
+            and (b is None or (type(b) is torch.nn.Parameter and b.dtype == torch.bfloat16
+                               and b.shape == w.shape[:1] and b.is_contiguous()
+                               and b.get_device() == w.get_device())))
 
 
 def _small_linear(x, weights, f32_outputs=()):
@@ -388,6 +411,8 @@ class GatedLinearAttention(torch.nn.Module):
         up = self.gk_proj[1]
         if (not torch.is_grad_enabled() and _small_rows(hidden_states)
                 and hidden_states.dtype == torch.bfloat16
+                and type(self.gk_proj) is torch.nn.Sequential and len(self.gk_proj) == 2
+                and _unhooked(self.gk_proj)
                 and all(_plain_linear(m, hidden_states) for m in lins)):
             # a few rows without gradients (decode): one launch for the projections, the low-rank
             # gate's second matrix and its activation in another; the output gate comes in
@@ -397,12 +422,7 @@ class GatedLinearAttention(torch.nn.Module):
             q, k, v = ys[0], ys[1], ys[2]
             if self.use_output_gate:
                 g = ys[4]
-            gate_done = (type(self.gk_proj) is torch.nn.Sequential
-                         and len(self.gk_proj) == 2 and not self.gk_proj._forward_hooks
-                         and not self.gk_proj._forward_pre_hooks
-                         and _plain_linear(up, hidden_states, bias=True)
-                         and up.weight.shape[1] % 8 == 0
-                         and (up.bias is None or up.bias.dtype == torch.bfloat16))
+            gate_done = _plain_gate(up, ys[3])
             gk = (_low_rank_gate(ys[3], up, self.gate_logit_normalizer, self.clamp_min)
                   if gate_done else up(ys[3]))
         elif (torch.is_grad_enabled()

@@ -35,6 +35,23 @@ def test_small_linear(rows, dtype):
 
 
 @pytest.mark.gpu
+def test_small_linear_scratch_values():
+    """float32 rows with infinities, NaN and values above the largest bfloat16 (3.3895e38): as
+    F.linear in float32 gives them (weights of +-1 and powers of two: exact products)."""
+    import torch.nn.functional as F
+
+    from tops.layers.gla import _small_linear
+
+    x = torch.zeros(6, 256, device="cuda")
+    x[0, 3], x[1, 3], x[2, 3] = float("inf"), float("-inf"), float("nan")
+    x[3, 3], x[4, 3], x[5, 200] = 3.4e38, -3.4028234663852886e38, 1e-30
+    w = torch.full((16, 256), 0.5, device="cuda").bfloat16()
+    w[1] = -1.0
+    y = _small_linear(x, [w])[0]
+    assert torch.equal(torch.nan_to_num(y, 7.0), torch.nan_to_num(F.linear(x, w.float()), 7.0))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,n,clamp,bias", [(1, 256, None, True), (5, 300, -0.03, True),
                                                (128, 1024, None, False)])
 def test_low_rank_gate(rows, n, clamp, bias):
@@ -81,6 +98,53 @@ def test_decode_step_matches_library_path(cfg, batch, tokens):
     for a, b in zip(*outs):
         assert a.shape == b.shape and a.dtype == b.dtype
         _close(a, b.double(), 2e-2)
+
+
+def _layer(hidden=256):
+    from tops.layers import GatedLinearAttention
+
+    return GatedLinearAttention(rngs=3, dtype=torch.bfloat16, layer_idx=0, hidden_size=hidden,
+                                num_heads=2)
+
+
+def test_few_row_route_takes_plain_projections_only():
+    """What the few-row kernels would not see keeps the library path: a weight of another width
+    (F.linear's error), another forward, hooks."""
+    from tops.layers.gla import _plain_gate, _plain_linear
+
+    m, x = _layer(), torch.zeros(1, 1, 256, dtype=torch.bfloat16)
+    low = torch.zeros(1, 1, 16, dtype=torch.bfloat16)
+    assert _plain_linear(m.q_proj, x) and _plain_gate(m.gk_proj[1], low)
+    assert not _plain_linear(m.q_proj, torch.zeros(1, 1, 512, dtype=torch.bfloat16))
+    assert not _plain_gate(m.gk_proj[1], x)
+    assert not _plain_linear(m.gk_proj[1], low)   # has a bias
+    m.q_proj.forward = lambda t: t
+    m.k_proj.register_forward_hook(lambda *a: None)
+    m.gk_proj[1].bias = torch.nn.Parameter(m.gk_proj[1].bias.detach()[:8])
+    assert not _plain_linear(m.q_proj, x) and not _plain_linear(m.k_proj, x)
+    assert not _plain_gate(m.gk_proj[1], low)
+
+
+@pytest.mark.gpu
+def test_few_row_route_leaves_tangents_and_global_hooks():
+    import torch.autograd.forward_ad as fwd
+    from torch.nn.modules.module import register_module_forward_hook
+
+    m = _layer().cuda()
+    x = torch.ones(1, 1, 256, device="cuda").bfloat16()
+    from tops.layers.gla import _small_rows
+
+    with torch.no_grad():
+        assert _small_rows(x)
+        with fwd.dual_level():
+            assert not _small_rows(x)
+        seen = []
+        h = register_module_forward_hook(lambda mod, a, o: seen.append(mod))
+        try:
+            m(x)
+        finally:
+            h.remove()
+        assert any(s is m.q_proj for s in seen) and any(s is m.o_proj for s in seen)
 
 
 def test_entry_points_refuse_bad_arguments():

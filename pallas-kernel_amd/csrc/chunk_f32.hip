@@ -1,0 +1,294 @@
+// Per-chunk products of float32 inputs at chunk 64 over whole rows of the value dimension: the
+// forward's output and the backward's dv (reference: tops/ops/gla/chunk.py:441-496, 504-560).
+// With g~ the chunk-local cumsum, gamma its last row and r = (g~_first + gamma) / 2:
+//   qg = q e^{g~-r},  kg = k e^{r-g~},  A = scale qg kg^T
+//   o  = tril(A) v    + qg (scale e^{r} h)
+//   dv = tril(A)^T do + kg (e^{gamma-r} dh)
+// which are one computation: out = M x + L (f (.) S), L [64][K] in LDS.
+//
+// What bounds it: the float32 MFMAs (16x16x4, 256 FLOP a cycle and CU). One 256-thread block
+// takes a (chunk, head) and up to 256 value columns, so that A and the gating are formed once
+// for them; a wave takes 64 of the columns and 16 to 64 of the rows. x (v, do) and the state
+// rows (h, dh) go from global memory to the MFMA operand registers and never through LDS: a
+// lane's 16 bytes are four columns of one row, i.e. the operand of four 16-column tiles (tile j
+// holds the columns 4 n + j), so no operand is transposed and a row of outputs is stored in 16
+// bytes a lane. Each LDS fragment (four contraction steps of 16 rows) feeds 16 products, each
+// global load four to sixteen. Tiles of A above the diagonal are neither formed nor read. LDS 53
+// KB at K = 128 (the tile of the other operand is reused for A): three blocks a CU.
+// Replaced here: one block of 104 KB LDS a CU with transposing stores of v and h (o), one block
+// per 64 columns with A formed in each (dv); both stay for the other chunk sizes, bf16, rows
+// that are not 16-byte aligned, and given A or cumulative gates.
+#include <initializer_list>
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace tops {
+
+namespace {
+
+constexpr int FC = 64;          // rows of a chunk
+constexpr int FP = FC + 4;      // LDS pitch of 64-wide rows
+
+int f32_lds_bytes(int K) {
+  const int KP = (K + 63) / 64 * 64;
+  return (FC * (KP + 4) + FC * FP + KP + 2 * 5 * 64) * 4;
+}
+
+// Lower tiles of A in the order they are dealt to the waves.
+__device__ __forceinline__ void lower_tile(int t, int& mi, int& ni) {
+  mi = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
+  ni = t - mi * (mi + 1) / 2;
+}
+
+}  // namespace
+
+struct F32RowArgs {
+  const float *q, *k, *g;
+  const float* x;      // v or do [tokens, H, V]
+  const float* s;      // h or dh [NC, H, K, V] (nullable)
+  float* out;          // o or dv [tokens, H, V]
+  float scale;
+  int H, K, V;
+  SeqInfo si;
+};
+
+// DV: dv instead of o. NV: 64-column groups of a block (waves: NV column x 4 / NV row groups).
+template <bool DV, int NV>
+__global__ __launch_bounds__(256, 3) void chunk_f32_kernel(F32RowArgs p) {
+  constexpr int RT = NV;   // 16-row tiles of a wave
+  extern __shared__ __attribute__((aligned(16))) float fsm[];
+  const int H = p.H, K = p.K, V = p.V;
+  const int KT = (K + 63) >> 6, KP = KT * 64, PL = KP + 4;
+  float* sL = fsm;                  // [64][PL]: qg (o) or kg (dv)
+  float* sT = sL + FC * PL;         // [64][FP]: the other operand's K tile, then M
+  float* sR = sT + FC * FP;         // [KP]: the state rows' factors
+  float* sTot = sR + KP;            // [2][5][64]: segment sums of g, first row
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, gr = lane >> 4;
+  const int NB = (V + 64 * NV - 1) / (64 * NV);
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int c = L / NB / H, hh = L / NB % H;
+  int seq, t0, len;
+  chunk_range(p.si, c, seq, t0, len);
+  (void)seq;
+  const long rsK = (long)H * K, rsV = (long)H * V;
+  const long baseK = ((long)t0 * H + hh) * K, baseV = ((long)t0 * H + hh) * V;
+
+  const float *qb = p.q + baseK, *kb = p.k + baseK, *gb = p.g + baseK;
+  const float* xbase = p.x + baseV;
+
+  // ---- L, M = tril(A) or its transpose ----
+  f32x4 accA[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) accA[j] = zero4();
+  for (int kt = 0; kt < KT; ++kt) {
+    const int col = kt * 64 + lane;   // thread: one column, rows 16 w .. 16 w + 15
+    const uint32_t cc = (uint32_t)min(col, K - 1);
+    float gv[16], qv[16], kv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {   // no branches: all loads are in flight together
+      const uint32_t at = (uint32_t)min(16 * w + i, len - 1) * (uint32_t)rsK + cc;
+      gv[i] = gb[at];
+      qv[i] = qb[at];
+      kv[i] = kb[at];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (16 * w + i >= len || col >= K) gv[i] = qv[i] = kv[i] = 0.f;
+    float* st = sTot + (kt & 1) * 5 * 64;   // two buffers: one barrier between write and read
+    if (w == 0) st[4 * 64 + lane] = gv[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) gv[i] += gv[i - 1];
+    st[w * 64 + lane] = gv[15];
+    __syncthreads();
+    float off = 0.f, gamma = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float x = st[s * 64 + lane];
+      off += s < w ? x : 0.f;
+      gamma += x;
+    }
+    const float r = 0.5f * (st[4 * 64 + lane] + gamma);
+    if (w == 0) sR[col] = DV ? gexp<float>(gamma - r) : p.scale * gexp<float>(r);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 16 * w + i;
+      const float d = gv[i] + off - r;
+      const float qg = qv[i] * gexp<float>(d), kg = kv[i] * gexp<float>(-d);
+      sL[row * PL + col] = DV ? kg : qg;
+      sT[row * FP + lane] = DV ? qg : kg;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int t = w + 4 * j;
+      if (t >= 10) break;   // uniform
+      int mi, ni;
+      lower_tile(t, mi, ni);
+      const float* a = DV ? sT + mi * 16 * FP : sL + mi * 16 * PL + kt * 64;
+      const float* b = DV ? sL + ni * 16 * PL + kt * 64 : sT + ni * 16 * FP;
+      mma_tile<float>(accA[j], a, DV ? FP : PL, b, DV ? PL : FP, 64, lane);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int t = w + 4 * j;
+    if (t >= 10) break;
+    int mi, ni;
+    lower_tile(t, mi, ni);
+    const int jj = ni * 16 + li, ii = mi * 16 + 4 * gr;   // rows ii + r
+    float a[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = jj <= ii + r ? accA[j][r] * p.scale : 0.f;
+    if (DV) {
+      *reinterpret_cast<float4*>(sT + jj * FP + ii) = make_float4(a[0], a[1], a[2], a[3]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sT[(ii + r) * FP + jj] = a[r];
+    }
+  }
+  __syncthreads();
+
+  // ---- out = M x + L (f (.) S): this wave's 64 columns and 16 RT rows ----
+  const int vb = (L % NB * NV + w % NV) * 64, rt0 = w / NV * RT;
+  if (vb >= V) return;   // uniform; no barrier follows
+  const int vcol = min(vb + 4 * li, V - 4);
+  const bool vok = vb + 4 * li < V;
+  f32x4 acc[RT][4];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[t][j] = zero4();
+
+  // 16 contraction steps: step e of the lane's group is row 4 gr + e of the 16
+  auto products = [&](const float* M, int pitch, const float4 (&b)[4], int lo, int hi) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      if (rt0 + t < lo || rt0 + t > hi) continue;   // uniform
+      const float4 m = *reinterpret_cast<const float4*>(M + ((rt0 + t) * 16 + li) * pitch + 4 * gr);
+      const float me[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(me[e], b[e].x, acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(me[e], b[e].y, acc[t][1], 0, 0, 0);
+        acc[t][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(me[e], b[e].z, acc[t][2], 0, 0, 0);
+        acc[t][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(me[e], b[e].w, acc[t][3], 0, 0, 0);
+      }
+    }
+  };
+  auto load_x = [&](int s, float4 (&b)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * s + 4 * gr + e;
+      const float4 x =
+          *reinterpret_cast<const float4*>(xbase + (uint32_t)min(row, len - 1) * (uint32_t)rsV + vcol);
+      b[e] = row < len ? x : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  const float* srow = p.s + ((long)c * H + hh) * K * V;
+  auto load_s = [&](int s, float4 (&b)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      b[e] = *reinterpret_cast<const float4*>(
+          srow + (uint32_t)min(16 * s + 4 * gr + e, K - 1) * (uint32_t)V + vcol);
+  };
+  float4 xa[4], xb[4];
+  load_x(0, xa);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {   // the next 16 rows are loaded under these products
+    float4(&cur)[4] = s & 1 ? xb : xa;
+    float4(&nxt)[4] = s & 1 ? xa : xb;
+    if (s < 3) load_x(s + 1, nxt);
+    products(sT + 16 * s, FP, cur, DV ? 0 : s, DV ? s : 3);
+  }
+  if (p.s) {
+    const int NS = (K + 15) / 16;
+    auto scaled = [&](int s, const float4 (&b)[4]) {
+      const float4 f = *reinterpret_cast<const float4*>(sR + 16 * s + 4 * gr);
+      const float fe[4] = {f.x, f.y, f.z, f.w};
+      float4 y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = 16 * s + 4 * gr + e < K;
+        y[e] = in ? make_float4(b[e].x * fe[e], b[e].y * fe[e], b[e].z * fe[e], b[e].w * fe[e])
+                  : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+      products(sL + 16 * s, PL, y, 0, 3);
+    };
+    load_s(0, xa);
+    for (int s = 0; s < NS; s += 2) {
+      if (s + 1 < NS) load_s(s + 1, xb);
+      scaled(s, xa);
+      if (s + 1 >= NS) break;
+      if (s + 2 < NS) load_s(s + 2, xa);
+      scaled(s + 1, xb);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = (rt0 + t) * 16 + 4 * gr + r;
+      if (row < len && vok)
+        *reinterpret_cast<float4*>(p.out + baseV + (uint32_t)row * (uint32_t)rsV + vcol) =
+            make_float4(acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]);
+    }
+}
+
+template <bool DV, int NV>
+static hipError_t launch_f32(const F32RowArgs& p, hipStream_t st) {
+  const long blocks = (long)p.si.NC * p.H * ((p.V + 64 * NV - 1) / (64 * NV));
+  if (blocks == 0) return hipSuccess;
+  const int lds = f32_lds_bytes(p.K);
+  const hipError_t e = hipFuncSetAttribute((const void*)chunk_f32_kernel<DV, NV>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((chunk_f32_kernel<DV, NV>), dim3((unsigned)blocks), dim3(256), lds, st, p);
+  return hipGetLastError();
+}
+
+// Columns of a block: as many as V has, up to 256, unless that leaves fewer blocks than CUs.
+template <bool DV>
+static hipError_t pick_f32(const F32RowArgs& p, hipStream_t st) {
+  const long nch = (long)p.si.NC * p.H;
+  if (p.V > 128 && nch * ((p.V + 255) / 256) >= 256) return launch_f32<DV, 4>(p, st);
+  if (p.V > 64 && nch * ((p.V + 127) / 128) >= 256) return launch_f32<DV, 2>(p, st);
+  return launch_f32<DV, 1>(p, st);
+}
+
+// K up to 384: the LDS of a block (118 KB there) stays below that of the kernels replaced.
+// 32-bit offsets within a chunk's rows and a state.
+static bool f32_sizes(int C, int H, int K, int V, std::initializer_list<const void*> ptrs) {
+  if (C != FC || K <= 0 || K > 384 || V % 4 != 0) return false;
+  if (64L * H * (K > V ? K : V) >= (1L << 30) || (long)K * V >= (1L << 30)) return false;
+  for (const void* x : ptrs)
+    if ((uintptr_t)x & 15u) return false;
+  return true;
+}
+
+bool f32_fwd_o_supported(const FwdOArgs& p) {
+  return p.o != nullptr && p.A_in == nullptr && p.A_out == nullptr && !p.g_is_cumsum &&
+         f32_sizes(p.si.C, p.H, p.K, p.V, {p.v, p.h, p.o});
+}
+hipError_t run_f32_fwd_o(const FwdOArgs& p, hipStream_t st) {
+  F32RowArgs a = {(const float*)p.q, (const float*)p.k, (const float*)p.g, (const float*)p.v,
+                  (const float*)p.h, (float*)p.o,       p.scale,           p.H,
+                  p.K,               p.V,               p.si};
+  return pick_f32<false>(a, st);
+}
+
+bool f32_dv_supported(const BwdArgs& p) {
+  return f32_sizes(p.si.C, p.H, p.K, p.V, {p.dout, p.dh, p.dv});
+}
+hipError_t run_f32_dv(const BwdArgs& p, hipStream_t st) {
+  F32RowArgs a = {(const float*)p.q,  (const float*)p.k, (const float*)p.g, (const float*)p.dout,
+                  (const float*)p.dh, (float*)p.dv,      p.scale,           p.H,
+                  p.K,                p.V,               p.si};
+  return pick_f32<true>(a, st);
+}
+
+}  // namespace tops

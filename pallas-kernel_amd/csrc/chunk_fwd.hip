@@ -226,7 +226,8 @@ static hipError_t dispatch_fwd_o(const FwdOArgs& p, hipStream_t st) {
 
 hipError_t run_chunk_fwd_o(const FwdOArgs& p, int dtype, hipStream_t st) {
   if (dtype == DT_BF16) return dispatch_fwd_o<bf16>(p, st);
-  if (dtype == DT_F32) return dispatch_fwd_o<float>(p, st);
+  if (dtype == DT_F32)
+    return f32_fwd_o_supported(p) ? run_f32_fwd_o(p, st) : dispatch_fwd_o<float>(p, st);
   return hipErrorInvalidValue;
 }
 

@@ -1,0 +1,81 @@
+"""float32 chunk-64 output and dv kernels (chunk_f32.hip) against float64 over their tile edges."""
+
+import pytest
+import torch
+
+
+def _ref(q, k, v, g, h0, do, dht, cu):
+    """float64 recurrence, token by token; gradients by autograd."""
+    xs = [t.detach().double().requires_grad_(True) for t in (q, k, v, g, h0)]
+    q, k, v, g, h0 = xs
+    outs, hts = [], []
+    scale = q.shape[-1] ** -0.5
+    for i, (a, b) in enumerate(zip(cu, cu[1:])):
+        S = h0[i]
+        for t in range(a, b):
+            S = S * g[0, t].exp()[..., None] + k[0, t][..., None] * v[0, t][:, None, :]
+            outs.append((q[0, t][..., None] * S).sum(1) * scale)
+        hts.append(S)
+    o, ht = torch.stack(outs)[None], torch.stack(hts)
+    grads = torch.autograd.grad([o, ht], xs, [do.double(), dht.double()])
+    return [o, ht, *grads]
+
+
+# K around 64-column tiles and 16-row contraction steps, V around 64, 128 and 256 columns,
+# sequence lengths around 16-row tiles and chunks of 64
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,V", [(4, 4), (64, 64), (60, 68), (96, 96), (128, 132), (132, 256),
+                                 (100, 260), (256, 512)])
+@pytest.mark.parametrize("lengths", [(1,), (64,), (17, 130, 63), (65, 48)])
+def test_chunk_f32(K, V, lengths):
+    import tops.ops.gla as G
+
+    H = 2
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    T, N = cu[-1], len(lengths)
+    gen = torch.Generator(device="cuda").manual_seed(K * 1000 + V + T)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    print(f"chunk f32 K {K} V {V} lengths {lengths}", flush=True)
+    q, k, v, h0 = mk(1, T, H, K), mk(1, T, H, K), mk(1, T, H, V), mk(N, H, K, V)
+    g = torch.nn.functional.logsigmoid(mk(1, T, H, K)) / 4
+    do, dht = mk(1, T, H, V), mk(N, H, K, V)
+    ref = _ref(*(t.cpu() for t in (q, k, v, g, h0, do, dht)), cu)
+    xs = [t.requires_grad_(True) for t in (q, k, v, g, h0)]
+    o, ht = G.chunk_gla(*xs[:4], initial_state=h0, output_final_state=True, chunk_size=64,
+                        cu_seqlens=torch.tensor(cu) if N > 1 else None)
+    got = [o, ht, *torch.autograd.grad([o, ht], xs, [do, dht])]
+    # float32 sums of at most K + 64 products: 2-norm error about 1e-6
+    for name, a, b in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), got, ref):
+        err = (a.detach().cpu().double() - b).norm() / b.norm().clamp_min(1e-30)
+        assert err < 4e-6, (name, float(err))
+
+
+@pytest.mark.gpu
+def test_rows_past_a_sequence_stay_out():
+    """Non-finite values in the next sequence's rows do not reach a partial chunk."""
+    import tops.ops.gla as G
+
+    T, H, K, V = 70, 1, 64, 128
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    q, k, v, g = mk(1, T, H, K), mk(1, T, H, K), mk(1, T, H, V), -mk(1, T, H, K).abs() / 8
+    v[:, 35:] = float("inf")
+    cu = torch.tensor([0, 35, T])
+    o, _ = G.chunk_gla(q, k, v, g, chunk_size=64, cu_seqlens=cu)
+    alone, _ = G.chunk_gla(q[:, :35], k[:, :35], v[:, :35], g[:, :35], chunk_size=64)
+    assert torch.equal(o[:, :35], alone)
+
+
+@pytest.mark.gpu
+def test_unaligned_rows_take_the_other_kernel():
+    """V of no multiple of four: the same values as the first columns of a wider call."""
+    import tops.ops.gla as G
+
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    q, k, v, g = mk(1, 80, 2, 64), mk(1, 80, 2, 64), mk(1, 80, 2, 68), -mk(1, 80, 2, 64).abs() / 8
+    o, _ = G.chunk_gla(q, k, v, g, chunk_size=64)
+    o2, _ = G.chunk_gla(q, k, v[..., :67].contiguous(), g, chunk_size=64)
+    assert (o[..., :67] - o2).norm() / o2.norm() < 2e-6   # another order of float32 sums

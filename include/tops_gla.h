@@ -133,7 +133,10 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
  *  - wide heads (K = 256, three or more 64-column V tiles): the per-chunk
  *    gating that the scans, the forward and the dv kernel then stream;
  *  - backward only: the fallback's final states (f32 [N, H, K, V], K and V <= 512; without
- *    it a call with dht is not checked).
+ *    it a call with dht is not checked);
+ *  - with bit 1 of `backward` (bit 0: for the backward), float32, chunk 64, K <= 384, V % 4
+ *    == 0: the chunks' decays (f32 [NC, H, K]) of the two-pass state scan, which forms all
+ *    chunks' updates at once.
  * A shorter workspace drops the later parts (varlen: the segments and the gating together,
  * below the varlen = 2 size). The per-chunk states h_ws that the forward
  * stores for flagged pairs are not meaningful (the backward recomputes those pairs).

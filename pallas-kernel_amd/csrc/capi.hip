@@ -138,6 +138,7 @@ bool use_head(int dtype, int chunk, int64_t K, int64_t V, bool g_is_cumsum,
 //   [segment states, decays (full-head, NS > 1)] [gate-range flags, int32]
 //   [wide heads' per-chunk gating (full-head)]
 //   [backward only: fallback final states f32 [N, H, K, V]]
+//   [float32, chunk 64: the two-pass state scan's decays f32 [NC, H, K]]
 // for fixed-length sequences. Varlen sequences have two layouts, told apart by the bytes
 // given: [flags] [final states], which runs every sequence as one segment and gates in every
 // block, and (full-head kernels) that with [segment states, decays] [gating] after it.
@@ -152,14 +153,19 @@ long align256(long x) { return (x + 255) / 256 * 256; }
 struct WsLayout {
   int NS = 1, SL = 0, VT = 1;
   long slots = 0;                              // segment states held
-  long seg = 0, flags = 0, gate = 0, ht = 0;   // bytes of each part
-  long off_seg = 0, off_flags = 0, off_gate = 0, off_ht = 0, total = 0;
+  long seg = 0, flags = 0, gate = 0, ht = 0, dec = 0;   // bytes of each part
+  long off_seg = 0, off_flags = 0, off_gate = 0, off_ht = 0, off_dec = 0, total = 0;
   long flags_end() const { return off_flags + flags; }
 };
 
 // `packed`: varlen sequences with the segment and gating parts.
+// Whether the two-pass state scan can take the sizes (tops::f32_scan_supported has the rest).
+bool two_pass_sizes(int dtype, int C, int64_t K, int64_t V) {
+  return dtype == TOPS_GLA_F32 && C == 64 && K <= 384 && V % 4 == 0;
+}
+
 WsLayout ws_layout(int N, int T, int H, int K, int V, int C, bool varlen, bool head,
-                   bool backward, bool packed) {
+                   bool backward, bool packed, bool two_pass) {
   WsLayout w;
   const long nc = varlen ? (long)(T + C - 1) / C + N : (long)N * ((T + C - 1) / C);
   long nflag = nc * H;
@@ -193,6 +199,11 @@ WsLayout ws_layout(int N, int T, int H, int K, int V, int C, bool varlen, bool h
     w.off_ht = w.off_gate + w.gate;
     w.total = w.off_ht + w.ht;
   }
+  if (two_pass) {
+    w.dec = align256(nc * H * K * 4);
+    w.off_dec = w.total;
+    w.total += w.dec;
+  }
   return w;
 }
 
@@ -203,15 +214,16 @@ struct WsParts {
   float *st = nullptr, *gm = nullptr;
   void* gate = nullptr;
   int* flags = nullptr;
-  float* ht = nullptr;
+  float *ht = nullptr, *dec = nullptr;
 };
 
 WsParts ws_parts(const tops::SeqInfo& si, int64_t H, int64_t K, int64_t V, void* ws,
-                 int64_t ws_bytes, bool head, bool backward) {
-  const bool varlen = si.cu != nullptr;
-  WsLayout w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, true);
-  if (varlen && ws_bytes < w.total)
-    w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, false);
+                 int64_t ws_bytes, bool head, bool backward, int dtype) {
+  const bool varlen = si.cu != nullptr, two = two_pass_sizes(dtype, si.C, K, V);
+  WsLayout w =
+      ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, true, two);
+  if (varlen && head && ws_bytes < w.total)
+    w = ws_layout(si.N, si.T, (int)H, (int)K, (int)V, si.C, varlen, head, backward, false, two);
   WsParts p;
   p.VT = w.VT;
   const bool usable = ws != nullptr && ((uintptr_t)ws & 255u) == 0;
@@ -226,6 +238,7 @@ WsParts ws_parts(const tops::SeqInfo& si, int64_t H, int64_t K, int64_t V, void*
   if (w.flags > 0 && ws_bytes >= w.off_flags + w.flags) p.flags = (int*)(b + w.off_flags);
   if (w.gate > 0 && ws_bytes >= w.off_gate + w.gate) p.gate = b + w.off_gate;
   if (w.ht > 0 && ws_bytes >= w.off_ht + w.ht) p.ht = (float*)(b + w.off_ht);
+  if (w.dec > 0 && ws_bytes >= w.off_dec + w.dec) p.dec = (float*)(b + w.off_dec);
   return p;
 }
 
@@ -336,7 +349,8 @@ int64_t tops_gla_chunk_ws_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int6
   if (!dtype_ok(dtype) || chunk_size <= 0 || chunk_size > 64) return 0;
   const bool head = tops::head_supported(dtype, chunk_size, (int)K, (int)V, false);
   return ws_layout((int)N, (int)T, (int)H, (int)K, (int)V, chunk_size, varlen != 0, head,
-                   backward != 0, varlen == 2).total;
+                   (backward & 1) != 0, varlen == 2,
+                   (backward & 2) && two_pass_sizes(dtype, chunk_size, K, V)).total;
 }
 
 int tops_gla_chunk_local_cumsum(const void* g, void* out, int64_t B, int64_t T, int64_t H,
@@ -410,7 +424,7 @@ int tops_gla_chunk_fwd_h(const void* k, const void* v, const void* g, int g_is_c
     s.s_all = h;
     s.s_final = ht;
     {
-      const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false);
+      const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false, dtype);
       s.NS = w.NS;
       s.SL = w.SL;
       s.seg_state = w.st;
@@ -480,7 +494,7 @@ int tops_gla_chunk_bwd_dh(const void* q, const void* g, int g_is_cumsum, const v
     s.s_all = dh;
     s.s_final = dh0;
     {
-      const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false);
+      const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false, dtype);
       s.NS = w.NS;
       s.SL = w.SL;
       s.seg_state = w.st;
@@ -554,8 +568,8 @@ namespace {
 // tops_gla_chunk_fwd off the full-head path: the fused float32 forward, or the state scan
 // and the per-chunk output kernel.
 int chunk_fwd_other(const void* q, const void* k, const void* v, const void* g, const float* h0,
-                    void* o, float* ht, void* h_ws, float scale, int64_t H, int64_t K,
-                    int64_t V, int chunk_size, const tops::SeqInfo& si, int dtype,
+                    void* o, float* ht, void* h_ws, float* dec, float scale, int64_t H,
+                    int64_t K, int64_t V, int chunk_size, const tops::SeqInfo& si, int dtype,
                     hipStream_t st) {
   int rc;
   if (tops::fused_fwd_supported(dtype, chunk_size, (int)K)) {
@@ -592,6 +606,7 @@ int chunk_fwd_other(const void* q, const void* k, const void* v, const void* g, 
   s.V = (int)V;
   s.vec = vec_ok(dtype, K, V, {k, v, g, h_ws});
   s.si = si;
+  s.dec = dec;
   rc = hip_status(tops::run_state_scan(s, false, dtype, st), "chunk_fwd (state scan)");
   if (rc) return rc;
   tops::FwdOArgs p = {};
@@ -680,7 +695,7 @@ int tops_gla_chunk_fwd(const void* q, const void* k, const void* v, const void* 
     f.o = o;
     f.h_out = h_ws;
     f.ht = ht;
-    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false);
+    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false, dtype);
     f.NS = w.NS;
     f.SL = w.SL;
     f.seg_state = w.st;
@@ -716,11 +731,12 @@ int tops_gla_chunk_fwd(const void* q, const void* k, const void* v, const void* 
     return hip_status(tops::run_recurrent_fwd(r, dtype, dtype, st),
                       "chunk_fwd (gate-range fallback)");
   }
-  rc = chunk_fwd_other(q, k, v, g, h0, o, ht, h_ws, scale, H, K, V, chunk_size, si, dtype, st);
+  const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, false, false, dtype);
+  rc = chunk_fwd_other(q, k, v, g, h0, o, ht, h_ws, w.dec, scale, H, K, V, chunk_size, si, dtype,
+                       st);
   if (rc) return rc;
   // the gate-range check of the per-chunk kernels, and the recurrent forward for the flagged
   // (sequence, head) pairs (o and the final state rewritten)
-  const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, false, false);
   if (w.flags == nullptr || B * T == 0) return rc;
   return gate_fallback_fwd(q, k, v, g, h0, o, ht, scale, H, K, V, si, w.flags, dtype, st);
 }
@@ -793,7 +809,7 @@ int tops_gla_chunk_fwd_noalloc(const void* q, const void* k, const void* v, cons
   // the segment part (full-head shapes) and the gate-range flags
   const bool head = tops::head_supported(dtype, chunk_size, (int)K, (int)V, false);
   const long need = K <= 512 ? ws_layout(si.N, si.T, (int)H, (int)K, (int)V, chunk_size,
-                                         si.cu != nullptr, head, false, false).flags_end()
+                                         si.cu != nullptr, head, false, false, false).flags_end()
                              : 0;
   if (need > kScratchBytes)
     return fail(TOPS_GLA_EINVAL,
@@ -841,7 +857,7 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
   int NS = 1, SL = 0;
   float *seg_st = nullptr, *seg_gm = nullptr;
   void* gate = nullptr;   // per-chunk gating of wide heads (when the workspace holds it)
-  const WsParts wp = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, head, true);
+  const WsParts wp = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, head, true, dtype);
   if (head) {
     NS = wp.NS;
     SL = wp.SL;
@@ -917,6 +933,7 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
     s.V = (int)V;
     s.vec = vec_ok(dtype, K, V, {k, v, g, h_ws});
     s.si = si;
+    s.dec = wp.dec;
     rc = hip_status(tops::run_state_scan(s, false, dtype, st), "chunk_bwd (state recompute)");
     if (rc) return rc;
     h = h_ws;
@@ -993,6 +1010,7 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
     d.V = (int)V;
     d.vec = vec_ok(dtype, K, V, {q, dout, g, dh_ws});
     d.si = si;
+    d.dec = wp.dec;
     rc = hip_status(tops::run_state_scan(d, true, dtype, st), "chunk_bwd (dh scan)");
     if (rc) return rc;
   }
@@ -1092,7 +1110,7 @@ int tops_gla_simple_chunk_fwd(const void* q, const void* k, const void* v, const
   f.h_out = h_ws;
   f.ht = ht;
   {
-    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false);
+    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false, dtype);
     f.NS = w.NS;
     f.SL = w.SL;
     f.seg_state = w.st;
@@ -1135,7 +1153,7 @@ int tops_gla_simple_chunk_bwd(const void* q, const void* k, const void* v, const
   int NS = 1, SL = 0;
   float *seg_st = nullptr, *seg_gm = nullptr;
   {
-    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false);
+    const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, true, false, dtype);
     NS = w.NS;
     SL = w.SL;
     seg_st = w.st;

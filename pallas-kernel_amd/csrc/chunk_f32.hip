@@ -15,7 +15,8 @@
 // bytes a lane. Each LDS fragment (four contraction steps of 16 rows) feeds 16 products, each
 // global load four to sixteen. Tiles of A above the diagonal are neither formed nor read. LDS 53
 // KB at K = 128 (the tile of the other operand is reused for A): three blocks a CU.
-// Replaced here: one block of 104 KB LDS a CU with transposing stores of v and h (o), one block
+// B4 T2048 H4 K128 V256: o 199 -> 47 us, dv 124 -> 47 us. Replaced
+// here: one block of 104 KB LDS a CU with transposing stores of v and h (o), one block
 // per 64 columns with A formed in each (dv); both stay for the other chunk sizes, bf16, rows
 // that are not 16-byte aligned, and given A or cumulative gates.
 #include <initializer_list>
@@ -39,6 +40,25 @@ int f32_lds_bytes(int K) {
 __device__ __forceinline__ void lower_tile(int t, int& mi, int& ni) {
   mi = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
   ni = t - mi * (mi + 1) / 2;
+}
+
+// Chunk-local cumsum of one column (lane) whose 16 rows of this wave are in g: in place without
+// the earlier waves' rows, which are `off`. st: [5][64]. One barrier.
+__device__ __forceinline__ void segment_cumsum(float (&g)[16], float* st, int w, int lane,
+                                               float& first, float& off, float& gamma) {
+  if (w == 0) st[4 * 64 + lane] = g[0];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) g[i] += g[i - 1];
+  st[w * 64 + lane] = g[15];
+  __syncthreads();
+  off = gamma = 0.f;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const float x = st[s * 64 + lane];
+    off += s < w ? x : 0.f;
+    gamma += x;
+  }
+  first = st[4 * 64 + lane];
 }
 
 }  // namespace
@@ -98,20 +118,9 @@ __global__ __launch_bounds__(256, 3) void chunk_f32_kernel(F32RowArgs p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i)
       if (16 * w + i >= len || col >= K) gv[i] = qv[i] = kv[i] = 0.f;
-    float* st = sTot + (kt & 1) * 5 * 64;   // two buffers: one barrier between write and read
-    if (w == 0) st[4 * 64 + lane] = gv[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i) gv[i] += gv[i - 1];
-    st[w * 64 + lane] = gv[15];
-    __syncthreads();
-    float off = 0.f, gamma = 0.f;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float x = st[s * 64 + lane];
-      off += s < w ? x : 0.f;
-      gamma += x;
-    }
-    const float r = 0.5f * (st[4 * 64 + lane] + gamma);
+    float first, off, gamma;   // two buffers of sums: one barrier between write and read
+    segment_cumsum(gv, sTot + (kt & 1) * 5 * 64, w, lane, first, off, gamma);
+    const float r = 0.5f * (first + gamma);
     if (w == 0) sR[col] = DV ? gexp<float>(gamma - r) : p.scale * gexp<float>(r);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -268,6 +277,202 @@ static bool f32_sizes(int C, int H, int K, int V, std::initializer_list<const vo
   for (const void* x : ptrs)
     if ((uintptr_t)x & 15u) return false;
   return true;
+}
+
+// ---------------------------------------------------------------------------
+// Per-chunk states: forward h (a = k, b = v) and reverse dh (a = q, b = do), reference
+// tops/ops/common/chunk_h.py:18-119, 399-591, in two passes. The first forms every chunk's
+// update U_n = a~^T b (a~ = k e^{gamma - g~}, or scale q e^{g~}) at the state's place and its
+// decay e^{gamma_n}, all chunks at once; the second walks the chunks, S <- e^{gamma_n} S + U_n,
+// one thread per four values, and leaves in U_n's place the state entering (reverse: leaving)
+// the chunk.
+//
+// What bounds it: memory, the states written, read and written again. The scan that this replaces
+// (state_scan_kernel, which writes them once) walks the chunks with the gating and the products in
+// the chain: 3.1 us a chunk whatever the number of sequences. B4 T2048 H4 K128 V256, a direction:
+// 100 us -> 36 (updates) + 22 (states); forward + backward 438 -> 354 us. It was faster at every
+// size tried, from B1 T200 (one block of 64 x 32 a state tile) to 512 (sequence, head) pairs of four
+// chunks and 64 pairs of 32 (B4 T2048 H16 K=V=128), so it runs wherever the workspace holds the
+// decays.
+// ---------------------------------------------------------------------------
+
+// a~ in LDS (row-major, 17 KB), b from global memory to the operand registers as above; a block
+// takes 64 key columns and up to 256 value columns of one chunk and head.
+template <bool REV, int NV>
+__global__ __launch_bounds__(256, 3) void f32_update_kernel(ScanArgs p) {
+  constexpr int RT = NV;   // 16-row tiles (of keys) of a wave
+  __shared__ __attribute__((aligned(16))) float sA[FC * FP];
+  __shared__ float sTot[5 * 64];
+  const int H = p.H, K = p.K, V = p.V;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, gr = lane >> 4;
+  const int KT = (K + 63) >> 6, NB = (V + 64 * NV - 1) / (64 * NV);
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int kt = L / NB % KT, ch = L / NB / KT;
+  const int c = ch / H, hh = ch % H;
+  int seq, t0, len;
+  chunk_range(p.si, c, seq, t0, len);
+  (void)seq;
+  const uint32_t rsK = (uint32_t)H * K, rsV = (uint32_t)H * V;
+  const long baseK = ((long)t0 * H + hh) * K, baseV = ((long)t0 * H + hh) * V;
+  const float *ab = (const float*)p.a + baseK, *gb = (const float*)p.g + baseK;
+  const float* bb = (const float*)p.b + baseV;
+
+  const int vb = (L % NB * NV + w % NV) * 64, rt0 = w / NV * RT;
+  const int vcol = min(vb + 4 * li, V - 4);
+  auto load_b = [&](int s, float4 (&b)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * s + 4 * gr + e;
+      const float4 x = *reinterpret_cast<const float4*>(bb + (uint32_t)min(row, len - 1) * rsV + vcol);
+      b[e] = row < len ? x : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  const int col = kt * 64 + lane;
+  const uint32_t cc = (uint32_t)min(col, K - 1);
+  float gv[16], av[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint32_t at = (uint32_t)min(16 * w + i, len - 1) * rsK + cc;
+    gv[i] = gb[at];
+    av[i] = ab[at];
+  }
+  float4 xa[4], xb[4];
+  load_b(0, xa);
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (16 * w + i >= len || col >= K) gv[i] = av[i] = 0.f;
+  float first, off, gamma;
+  segment_cumsum(gv, sTot, w, lane, first, off, gamma);
+  if (w == 0 && L % NB == 0 && col < K) p.dec[(long)ch * K + col] = gexp<float>(gamma);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float x = gv[i] + off;
+    sA[(16 * w + i) * FP + lane] =
+        av[i] * (REV ? p.scale * gexp<float>(x) : gexp<float>(gamma - x));
+  }
+  __syncthreads();
+  if (vb >= V) return;   // uniform; no barrier follows
+
+  f32x4 acc[RT][4];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[t][j] = zero4();
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    float4(&cur)[4] = s & 1 ? xb : xa;
+    float4(&nxt)[4] = s & 1 ? xa : xb;
+    if (s < 3) load_b(s + 1, nxt);
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = sA[(16 * s + 4 * gr + e) * FP + (rt0 + t) * 16 + li];
+        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, cur[e].x, acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, cur[e].y, acc[t][1], 0, 0, 0);
+        acc[t][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, cur[e].z, acc[t][2], 0, 0, 0);
+        acc[t][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, cur[e].w, acc[t][3], 0, 0, 0);
+      }
+  }
+  float* u = (float*)p.s_all + (long)ch * K * V;
+  const bool vok = vb + 4 * li < V;
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = kt * 64 + (rt0 + t) * 16 + 4 * gr + r;
+      if (k < K && vok)
+        *reinterpret_cast<float4*>(u + (uint32_t)k * (uint32_t)V + vcol) =
+            make_float4(acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]);
+    }
+}
+
+// One thread per four values of a (sequence, head)'s state; two batches of SD chunks' updates
+// in registers, so that loads are in flight while a batch is added up.
+constexpr int SD = 8;
+template <bool REV>
+__global__ __launch_bounds__(256) void f32_state_kernel(ScanArgs p) {
+  const int H = p.H, K = p.K, V4 = p.V / 4;
+  const int NB = (K * V4 + 255) / 256;
+  const int bh = blockIdx.x / NB, e = blockIdx.x % NB * 256 + (int)threadIdx.x;
+  const int seq = bh / H, hh = bh % H;
+  if (e >= K * V4) return;
+  int bos, eos, c0, nc;
+  seq_range(p.si, seq, bos, eos, c0, nc);
+  (void)bos;
+  (void)eos;
+  const long step = (long)H * K * V4;   // float4s from a chunk to the next
+  float4* s = (float4*)p.s_all + ((long)c0 * H + hh) * K * V4 + e;
+  const float* dec = p.dec + ((long)c0 * H + hh) * K + e / V4;
+  const long at = ((long)seq * H + hh) * K * V4 + e;
+  float4 S = p.s_init ? ((const float4*)p.s_init)[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+  auto chunk = [&](int n) { return REV ? nc - 1 - n : n; };
+  struct Batch {
+    float4 u[SD];
+    float d[SD];
+  };
+  auto load = [&](int n0, Batch& b) {
+#pragma unroll
+    for (int i = 0; i < SD; ++i) {
+      const int n = chunk(min(n0 + i, nc - 1));   // past the end: the last chunk again, unused
+      b.u[i] = s[n * step];
+      b.d[i] = dec[(long)n * H * K];
+    }
+  };
+  auto walk = [&](int n0, const Batch& b) {
+#pragma unroll
+    for (int i = 0; i < SD; ++i) {
+      if (n0 + i >= nc) break;   // uniform
+      s[chunk(n0 + i) * step] = S;
+      S.x = fmaf(b.d[i], S.x, b.u[i].x);
+      S.y = fmaf(b.d[i], S.y, b.u[i].y);
+      S.z = fmaf(b.d[i], S.z, b.u[i].z);
+      S.w = fmaf(b.d[i], S.w, b.u[i].w);
+    }
+  };
+  if (nc > 0) {
+    Batch A, B;
+    load(0, A);
+    for (int n = 0; n < nc; n += 2 * SD) {
+      load(n + SD, B);
+      walk(n, A);
+      if (n + SD >= nc) break;
+      load(n + 2 * SD, A);
+      walk(n + SD, B);
+    }
+  }
+  if (p.s_final) ((float4*)p.s_final)[at] = S;
+}
+
+template <bool REV, int NV>
+static hipError_t launch_update(const ScanArgs& p, hipStream_t st) {
+  const long blocks =
+      (long)p.si.NC * p.H * ((p.K + 63) / 64) * ((p.V + 64 * NV - 1) / (64 * NV));
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL((f32_update_kernel<REV, NV>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+template <bool REV>
+static hipError_t run_f32_scan_dir(const ScanArgs& p, hipStream_t st) {
+  const hipError_t e = p.V > 128 ? launch_update<REV, 4>(p, st)
+                       : p.V > 64 ? launch_update<REV, 2>(p, st)
+                                  : launch_update<REV, 1>(p, st);
+  if (e != hipSuccess) return e;
+  const long blocks = (long)p.si.N * p.H * ((p.K * (p.V / 4) + 255) / 256);
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL((f32_state_kernel<REV>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+bool f32_scan_supported(const ScanArgs& p) {
+  return p.dec != nullptr && p.s_all != nullptr && !p.g_is_cumsum &&
+         f32_sizes(p.si.C, p.H, p.K, p.V, {p.b, p.s_all, p.s_init, p.s_final});
+}
+hipError_t run_f32_scan(const ScanArgs& p, bool reverse, hipStream_t st) {
+  return reverse ? run_f32_scan_dir<true>(p, st) : run_f32_scan_dir<false>(p, st);
 }
 
 bool f32_fwd_o_supported(const FwdOArgs& p) {

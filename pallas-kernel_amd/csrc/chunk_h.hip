@@ -374,6 +374,7 @@ static hipError_t dispatch_c(const ScanArgs& p, hipStream_t st) {
 hipError_t run_state_scan(const ScanArgs& p, bool reverse, int dtype, hipStream_t st) {
   if (dtype == DT_BF16)
     return reverse ? dispatch_c<bf16, true>(p, st) : dispatch_c<bf16, false>(p, st);
+  if (dtype == DT_F32 && f32_scan_supported(p)) return run_f32_scan(p, reverse, st);
   if (dtype == DT_F32)
     return reverse ? dispatch_c<float, true>(p, st) : dispatch_c<float, false>(p, st);
   return hipErrorInvalidValue;

@@ -22,6 +22,7 @@ struct ScanArgs {
   int H, K, V;
   int vec;              // 16-byte loads/stores allowed (K, V multiples of 16 B, aligned)
   SeqInfo si;
+  float* dec;           // float32, chunk 64: [NC, H, K] workspace of the two-pass scan (nullable)
 };
 hipError_t run_state_scan(const ScanArgs& p, bool reverse, int dtype, hipStream_t st);
 
@@ -86,8 +87,10 @@ __host__ __device__ constexpr long gate_ws_entry(int K) {
 // which: bit 0 = dq/dk/dg kernel, bit 1 = dv kernel
 hipError_t run_chunk_bwd(const BwdArgs& p, int dtype, hipStream_t st, int which = 3);
 
-// Output and dv of float32 inputs at chunk 64 (chunk_f32.hip): V % 4 == 0, 16-byte aligned
-// value rows, K <= 384; raw gates, A neither given nor wanted.
+// Output, dv and per-chunk states of float32 inputs at chunk 64 (chunk_f32.hip): V % 4 == 0,
+// 16-byte aligned value rows, K <= 384; raw gates, A neither given nor wanted.
+bool f32_scan_supported(const ScanArgs& p);
+hipError_t run_f32_scan(const ScanArgs& p, bool reverse, hipStream_t st);
 bool f32_fwd_o_supported(const FwdOArgs& p);
 hipError_t run_f32_fwd_o(const FwdOArgs& p, hipStream_t st);
 bool f32_dv_supported(const BwdArgs& p);

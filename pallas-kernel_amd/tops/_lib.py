@@ -150,7 +150,7 @@ def call(name, *args):
 
 def full_head(K, V, chunk, dtype, backward):
     """True when the full-head kernels run this shape (see tops_gla_full_head)."""
-    return bool(load().tops_gla_full_head(K, V, chunk, dtype_code(dtype), int(bool(backward))))
+    return bool(load().tops_gla_full_head(K, V, chunk, dtype_code(dtype), 3 if backward else 2))
 
 
 def seg_workspace(B, T, H, K, V, chunk, varlen, dtype, device, N=None, backward=False):
@@ -161,7 +161,7 @@ def seg_workspace(B, T, H, K, V, chunk, varlen, dtype, device, N=None, backward=
     if N is None:
         N = len(varlen) - 1 if isinstance(varlen, (list, tuple)) else B
     n = int(load().tops_gla_chunk_ws_bytes(B, T, H, K, V, chunk, N, 2 if varlen else 0,
-                                           dtype_code(dtype), int(bool(backward))))
+                                           dtype_code(dtype), 3 if backward else 2))
     if n <= 0:
         return None, 0
     return torch.empty(n, dtype=torch.uint8, device=device), n

@@ -52,6 +52,49 @@ def test_chunk_f32(K, V, lengths):
         assert err < 4e-6, (name, float(err))
 
 
+# chunks around the state pass's batches of 8, one and two sequences, and the rows' value columns
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [60, 128, 320])
+@pytest.mark.parametrize("chunks", [7, 8, 9, 16, 17, 25])
+def test_two_pass_states_match_the_scan(chunks, V, monkeypatch):
+    """Without the workspace's last part the one-pass scan runs: the same float32 values but for
+    the order of the sums and one rounding of a decay."""
+    import tops.ops.gla as G
+    from tops import _lib
+
+    T, N, H, K = 64 * chunks - 5, 2, 2, 68
+    gen = torch.Generator(device="cuda").manual_seed(chunks * V)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    xs = [mk(N, T, H, K), mk(N, T, H, K), mk(N, T, H, V),
+          torch.nn.functional.logsigmoid(mk(N, T, H, K)) / 16, mk(N, H, K, V)]
+    xs = [x.requires_grad_(True) for x in xs]
+    do, dht = mk(N, T, H, V), mk(N, H, K, V)
+
+    def run():
+        o, ht = G.chunk_gla(*xs[:4], initial_state=xs[4], output_final_state=True, chunk_size=64)
+        return [o, ht, *torch.autograd.grad([o, ht], xs, [do, dht])]
+
+    two = run()
+    real = _lib.seg_workspace
+    part = (N * chunks * H * K * 4 + 255) // 256 * 256
+    monkeypatch.setattr(_lib, "seg_workspace",
+                        lambda *a, **kw: (lambda ws, n: (ws, n - part))(*real(*a, **kw)))
+    for name, a, b in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), two, run()):
+        assert (a - b).norm() < 2e-6 * b.norm(), name
+
+
+def test_two_pass_workspace_part():
+    """The decays are counted with bit 1 of `backward` alone, where the two-pass scan can run."""
+    from tops import _lib
+
+    q = _lib.load().tops_gla_chunk_ws_bytes
+    part = 4 * 32 * 4 * 128 * 4
+    assert q(4, 2048, 4, 128, 256, 64, 4, 0, 0, 3) == q(4, 2048, 4, 128, 256, 64, 4, 0, 0, 1) + part
+    assert q(4, 2048, 4, 128, 256, 64, 4, 0, 0, 2) == q(4, 2048, 4, 128, 256, 64, 4, 0, 0, 0) + part
+    for K, V, C, dt in ((388, 256, 64, 0), (128, 255, 64, 0), (128, 256, 32, 0), (128, 256, 64, 1)):
+        assert q(4, 2048, 4, K, V, C, 4, 0, dt, 2) == q(4, 2048, 4, K, V, C, 4, 0, dt, 0)
+
+
 @pytest.mark.gpu
 def test_rows_past_a_sequence_stay_out():
     """Non-finite values in the next sequence's rows do not reach a partial chunk."""

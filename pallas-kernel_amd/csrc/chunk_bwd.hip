@@ -703,10 +703,10 @@ static hipError_t dispatch_bwd(const BwdArgs& p, hipStream_t st, int which) {
 hipError_t run_chunk_bwd(const BwdArgs& p, int dtype, hipStream_t st, int which) {
   if (dtype == DT_BF16) return dispatch_bwd<bf16>(p, st, which);
   if (dtype == DT_F32) {
-    if ((which & 2) == 0 || !f32_dv_supported(p)) return dispatch_bwd<float>(p, st, which);
     hipError_t e = hipSuccess;
-    if (which & 1) e = dispatch_bwd<float>(p, st, 1);
-    return e == hipSuccess ? run_f32_dv(p, st) : e;
+    if (which & 1) e = f32_dqkg_supported(p) ? run_f32_dqkg(p, st) : dispatch_bwd<float>(p, st, 1);
+    if (e != hipSuccess || (which & 2) == 0) return e;
+    return f32_dv_supported(p) ? run_f32_dv(p, st) : dispatch_bwd<float>(p, st, 2);
   }
   return hipErrorInvalidValue;
 }

@@ -467,6 +467,258 @@ static hipError_t run_f32_scan_dir(const ScanArgs& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// dq, dk and dg (reference: tops/ops/gla/chunk.py:504-743), with dA = scale tril(do v^T):
+//   Xq = dA kg + (scale e^{r}) do h^T,   Xm = e^{gamma-r} v dh^T,   Xk = dA^T qg + Xm
+//   dq = e^{g~-r} Xq,  dk = e^{r-g~} Xk,
+//   dg = revcumsum(qg Xq - kg Xk) + e^{gamma} sum_v h dh + sum_j kg Xm
+//
+// What bounds it: the float32 MFMAs, 10 us of them a block of 64 key columns at V = 256. The
+// operands' value columns go through LDS 32 at a time (37 KB for do, v, h and dh), which with
+// qg and kg makes 72 KB and two blocks a CU, so that one block's loads and barriers lie under the
+// other's products; chunk_bwd_dqkg_kernel, which stages 64 columns and q, k and g raw, has 139 KB
+// and one (B4 T2048 H4 K128 V256: 127 -> 93 us; its 300 MB take about 55 at the rate of a large
+// copy). A wave's 16 key columns of every row stay in its accumulators to the end: dg's sums
+// over the rows are sums within a lane and across its four lane groups, without an exchange.
+// ---------------------------------------------------------------------------
+
+constexpr int DVW = 32, DVP = DVW + 4;   // value columns staged, their pitch
+struct DqkgF32 {
+  static constexpr int tile = FC * FP, vt = FC * DVP;   // floats
+  static constexpr int qg = 0, kg = tile, stage = 2 * tile;   // stage: do, v, h, dh
+  static constexpr int dA = stage, d = stage + tile;          // after the value columns
+  static constexpr int fac = stage + 4 * vt;                  // sR, sEg, sGm, sHd [64], sums
+  static constexpr int bytes = (fac + 4 * 64 + 5 * 64) * 4;
+  static_assert(d + tile <= fac, "dA and d lie in the staged tiles' place");
+};
+
+__global__ __launch_bounds__(256, 2) void f32_dqkg_kernel(BwdArgs p) {
+  extern __shared__ __attribute__((aligned(16))) float fsm[];
+  float *sQg = fsm + DqkgF32::qg, *sKg = fsm + DqkgF32::kg, *sS = fsm + DqkgF32::stage;
+  float *sdA = fsm + DqkgF32::dA, *sD = fsm + DqkgF32::d;
+  float *sR = fsm + DqkgF32::fac, *sEg = sR + 64, *sGm = sR + 128, *sHd = sR + 192,
+        *sTot = sR + 256;
+  const int H = p.H, K = p.K, V = p.V;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, gr = lane >> 4;
+  const int KT = (K + 63) >> 6, VT = (V + DVW - 1) / DVW;
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int kb = L % KT * 64, ch = L / KT;
+  const int c = ch / H, hh = ch % H;
+  int seq, t0, len;
+  chunk_range(p.si, c, seq, t0, len);
+  (void)seq;
+  const uint32_t rsK = (uint32_t)H * K, rsV = (uint32_t)H * V;
+  const long baseK = ((long)t0 * H + hh) * K + kb, baseV = ((long)t0 * H + hh) * V;
+  const long baseS = ((long)ch * K + kb) * V;
+  const int klen = min(64, K - kb);
+  const float* src[4] = {(const float*)p.dout + baseV, (const float*)p.v + baseV,
+                         (const float*)p.h + baseS, (const float*)p.dh + baseS};
+
+  // 16-byte pieces of the staged tiles: rows tid / 8 and + 32, columns 4 (tid % 8)
+  const int pr = tid >> 3, pc = 4 * (tid & 7);
+  float4 st[4][2];
+  auto load = [&](int vt) {
+    const int col = min(vt * DVW + pc, V - 4);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = min(pr + 32 * i, (t < 2 ? len : klen) - 1);
+        st[t][i] = *reinterpret_cast<const float4*>(src[t] + (uint32_t)row * (t < 2 ? rsV : (uint32_t)V) + col);
+      }
+  };
+  auto stage = [&](int vt) {
+    const bool in = vt * DVW + pc < V;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = pr + 32 * i;
+        const bool ok = in && row < (t < 2 ? len : klen);
+        *reinterpret_cast<float4*>(sS + t * DqkgF32::vt + row * DVP + pc) =
+            ok ? st[t][i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+  };
+
+  // ---- qg, kg; d = g~ - r of this thread's column and 16 rows ----
+  float d[16];
+  {
+    const bool cok = lane < klen;
+    const uint32_t cc = (uint32_t)min(lane, klen - 1);
+    const float *qb = (const float*)p.q + baseK, *kbp = (const float*)p.k + baseK,
+                *gb = (const float*)p.g + baseK;
+    float qv[16], kv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t at = (uint32_t)min(16 * w + i, len - 1) * rsK + cc;
+      d[i] = gb[at];
+      qv[i] = qb[at];
+      kv[i] = kbp[at];
+    }
+    load(0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (16 * w + i >= len || !cok) d[i] = qv[i] = kv[i] = 0.f;
+    float first, off, gamma;
+    segment_cumsum(d, sTot, w, lane, first, off, gamma);
+    const float r = 0.5f * (first + gamma);
+    if (w == 0) {
+      sR[lane] = p.scale * gexp<float>(r);
+      sEg[lane] = gexp<float>(gamma - r);
+      sGm[lane] = gexp<float>(gamma);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      d[i] += off - r;
+      sQg[(16 * w + i) * FP + lane] = qv[i] * gexp<float>(d[i]);
+      sKg[(16 * w + i) * FP + lane] = kv[i] * gexp<float>(-d[i]);
+    }
+  }
+
+  // ---- dA = do v^T (lower tiles), do h^T and v dh^T (this wave's 16 key columns) ----
+  f32x4 dA[3], Xq[4], Xm[4];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) dA[j] = zero4();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) Xq[j] = Xm[j] = zero4();
+  float hd = 0.f;   // sum_v h dh of key column tid / 4 over this thread's eight columns a tile
+  const float *sDo = sS, *sV = sS + DqkgF32::vt, *sH = sS + 2 * DqkgF32::vt,
+              *sDh = sS + 3 * DqkgF32::vt;
+  for (int vt = 0; vt < VT; ++vt) {
+    if (vt > 0) __syncthreads();   // the previous columns' readers are done
+    stage(vt);
+    __syncthreads();
+    if (vt + 1 < VT) load(vt + 1);
+    const Frag<float> fh = ld_frag(sH + (16 * w + li) * DVP + 8 * gr);
+    const Frag<float> fd = ld_frag(sDh + (16 * w + li) * DVP + 8 * gr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      mma(Xq[j], ld_frag(sDo + (16 * j + li) * DVP + 8 * gr), fh);
+      mma(Xm[j], ld_frag(sV + (16 * j + li) * DVP + 8 * gr), fd);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int t = w + 4 * j;
+      if (t >= 10) break;   // uniform
+      int mi, ni;
+      lower_tile(t, mi, ni);
+      mma_tile<float>(dA[j], sDo + mi * 16 * DVP, DVP, sV + ni * 16 * DVP, DVP, DVW, lane);
+    }
+    const float* a = sH + (tid >> 2) * DVP + 8 * (tid & 3);
+    const float* b = sDh + (tid >> 2) * DVP + 8 * (tid & 3);
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(a + i);
+      const float4 y = *reinterpret_cast<const float4*>(b + i);
+      hd += x.x * y.x + x.y * y.y + (x.z * y.z + x.w * y.w);
+    }
+  }
+  hd += __shfl_xor(hd, 1);
+  hd += __shfl_xor(hd, 2);
+  if ((tid & 3) == 0) sHd[tid >> 2] = hd;
+  __syncthreads();   // the staged tiles are dead
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int t = w + 4 * j;
+    if (t >= 10) break;
+    int mi, ni;
+    lower_tile(t, mi, ni);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int ii = mi * 16 + 4 * gr + r, jj = ni * 16 + li;
+      sdA[ii * FP + jj] = jj <= ii ? dA[j][r] * p.scale : 0.f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sD[(16 * w + i) * FP + lane] = d[i];
+  __syncthreads();
+
+  // ---- dA kg and dA^T qg: lane l's step e of 16 rows is row 4 (l >> 4) + e ----
+  const int kc = 16 * w + li;
+  const float fr = sR[kc], fe = sEg[kc];
+  f32x4 Xk[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    Xq[j] *= fr;
+    Xm[j] *= fe;
+    Xk[j] = Xm[j];
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    float bk[4], bq[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      bk[e] = sKg[(16 * s + 4 * gr + e) * FP + kc];
+      bq[e] = sQg[(16 * s + 4 * gr + e) * FP + kc];
+    }
+#pragma unroll
+    for (int j = s; j < 4; ++j) {   // rows 16 j.. of dq: columns of dA up to them
+      const float4 m = *reinterpret_cast<const float4*>(sdA + (16 * j + li) * FP + 16 * s + 4 * gr);
+      const float me[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        Xq[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(me[e], bk[e], Xq[j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j <= s; ++j)   // rows 16 j.. of dk: rows of dA from them on
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        Xk[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            sdA[(16 * s + 4 * gr + e) * FP + 16 * j + li], bq[e], Xk[j], 0, 0, 0);
+  }
+
+  // ---- dq, dk, dg: this lane's column, rows 16 j + 4 gr + r ----
+  float *dq = (float*)p.dq + baseK, *dk = (float*)p.dk + baseK, *dg = (float*)p.dg + baseK;
+  const bool cok = kc < klen;
+  float suf[4][4], dki = 0.f;
+#pragma unroll
+  for (int j = 3; j >= 0; --j)
+#pragma unroll
+    for (int r = 3; r >= 0; --r) {
+      const int row = 16 * j + 4 * gr + r;
+      const float dd = sD[row * FP + kc], qg = sQg[row * FP + kc], kg = sKg[row * FP + kc];
+      suf[j][r] = qg * Xq[j][r] - kg * Xk[j][r] + (r < 3 ? suf[j][r < 3 ? r + 1 : 3] : 0.f);
+      dki += kg * Xm[j][r];
+      if (row < len && cok) {
+        dq[(uint32_t)row * rsK + kc] = gexp<float>(dd) * Xq[j][r];
+        dk[(uint32_t)row * rsK + kc] = gexp<float>(-dd) * Xk[j][r];
+      }
+    }
+  dki += __shfl_xor(dki, 16);
+  dki += __shfl_xor(dki, 32);
+  float tail = sGm[kc] * sHd[kc] + dki, after = 0.f;   // after: the later 16-row tiles
+#pragma unroll
+  for (int j = 3; j >= 0; --j) {
+    const float x1 = __shfl_xor(suf[j][0], 16), both = suf[j][0] + x1;
+    const float x2 = __shfl_xor(both, 32);
+    const float off = ((gr & 1) == 0 ? x1 : 0.f) + ((gr & 2) == 0 ? x2 : 0.f) + after;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * j + 4 * gr + r;
+      if (row < len && cok) dg[(uint32_t)row * rsK + kc] = suf[j][r] + off + tail;
+    }
+    after += both + x2;
+  }
+}
+
+bool f32_dqkg_supported(const BwdArgs& p) {
+  return p.dg != nullptr && f32_sizes(p.si.C, p.H, p.K, p.V, {p.v, p.dout, p.h, p.dh});
+}
+hipError_t run_f32_dqkg(const BwdArgs& p, hipStream_t st) {
+  const long blocks = (long)p.si.NC * p.H * ((p.K + 63) / 64);
+  if (blocks == 0) return hipSuccess;
+  const hipError_t e =
+      hipFuncSetAttribute((const void*)f32_dqkg_kernel,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, DqkgF32::bytes);
+  if (e != hipSuccess) return e;
+  ktimer_mark(KT_BWD_DQKG, false, st);
+  hipLaunchKernelGGL(f32_dqkg_kernel, dim3((unsigned)blocks), dim3(256), DqkgF32::bytes, st, p);
+  ktimer_mark(KT_BWD_DQKG, true, st);
+  return hipGetLastError();
+}
+
 bool f32_scan_supported(const ScanArgs& p) {
   return p.dec != nullptr && p.s_all != nullptr && !p.g_is_cumsum &&
          f32_sizes(p.si.C, p.H, p.K, p.V, {p.b, p.s_all, p.s_init, p.s_final});

@@ -87,12 +87,14 @@ __host__ __device__ constexpr long gate_ws_entry(int K) {
 // which: bit 0 = dq/dk/dg kernel, bit 1 = dv kernel
 hipError_t run_chunk_bwd(const BwdArgs& p, int dtype, hipStream_t st, int which = 3);
 
-// Output, dv and per-chunk states of float32 inputs at chunk 64 (chunk_f32.hip): V % 4 == 0,
+// Output, gradients and per-chunk states of float32 inputs at chunk 64 (chunk_f32.hip): V % 4 == 0,
 // 16-byte aligned value rows, K <= 384; raw gates, A neither given nor wanted.
 bool f32_scan_supported(const ScanArgs& p);
 hipError_t run_f32_scan(const ScanArgs& p, bool reverse, hipStream_t st);
 bool f32_fwd_o_supported(const FwdOArgs& p);
 hipError_t run_f32_fwd_o(const FwdOArgs& p, hipStream_t st);
+bool f32_dqkg_supported(const BwdArgs& p);
+hipError_t run_f32_dqkg(const BwdArgs& p, hipStream_t st);
 bool f32_dv_supported(const BwdArgs& p);
 hipError_t run_f32_dv(const BwdArgs& p, hipStream_t st);
 

@@ -566,12 +566,15 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
 namespace {
 
 // tops_gla_chunk_fwd off the full-head path: the fused float32 forward, or the state scan
-// and the per-chunk output kernel.
+// and the per-chunk output kernel. That one also writes the gate-range flags (nullable) where it
+// can; `flags` is then left as given, otherwise set to NULL.
 int chunk_fwd_other(const void* q, const void* k, const void* v, const void* g, const float* h0,
-                    void* o, float* ht, void* h_ws, float* dec, float scale, int64_t H,
-                    int64_t K, int64_t V, int chunk_size, const tops::SeqInfo& si, int dtype,
-                    hipStream_t st) {
+                    void* o, float* ht, void* h_ws, float* dec, int*& flags, float scale,
+                    int64_t H, int64_t K, int64_t V, int chunk_size, const tops::SeqInfo& si,
+                    int dtype, hipStream_t st) {
   int rc;
+  int* const wanted = flags;
+  flags = nullptr;
   if (tops::fused_fwd_supported(dtype, chunk_size, (int)K)) {
     tops::FusedFwdArgs f = {};
     f.q = q;
@@ -624,6 +627,7 @@ int chunk_fwd_other(const void* q, const void* k, const void* v, const void* g, 
   p.K = (int)K;
   p.V = (int)V;
   p.si = si;
+  if (dtype == TOPS_GLA_F32 && tops::f32_fwd_o_supported(p)) p.flags = flags = wanted;
   return hip_status(tops::run_chunk_fwd_o(p, dtype, st), "chunk_fwd (output)");
 }
 
@@ -639,14 +643,12 @@ int gate_check(const void* g, int* flags, int64_t H, int64_t K, const tops::SeqI
   return hip_status(tops::run_gate_range(c, dtype, st), "gate-range check");
 }
 
-// The forward's fallback off the full-head path: check every chunk, then the recurrent
-// forward over the flagged pairs.
+// The forward's fallback off the full-head path: the recurrent forward over the pairs whose
+// chunks are flagged.
 int gate_fallback_fwd(const void* q, const void* k, const void* v, const void* g,
                       const float* h0, void* o, float* ht, float scale, int64_t H, int64_t K,
                       int64_t V, const tops::SeqInfo& si, int* flags, int dtype,
                       hipStream_t st) {
-  int rc = gate_check(g, flags, H, K, si, dtype, st);
-  if (rc) return rc;
   tops::RecArgs r = {};
   r.q = q;
   r.k = k;
@@ -732,12 +734,17 @@ int tops_gla_chunk_fwd(const void* q, const void* k, const void* v, const void* 
                       "chunk_fwd (gate-range fallback)");
   }
   const WsParts w = ws_parts(si, H, K, V, seg_ws, seg_ws_bytes, false, false, dtype);
-  rc = chunk_fwd_other(q, k, v, g, h0, o, ht, h_ws, w.dec, scale, H, K, V, chunk_size, si, dtype,
-                       st);
+  int* checked = w.flags;
+  rc = chunk_fwd_other(q, k, v, g, h0, o, ht, h_ws, w.dec, checked, scale, H, K, V, chunk_size, si,
+                       dtype, st);
   if (rc) return rc;
   // the gate-range check of the per-chunk kernels, and the recurrent forward for the flagged
   // (sequence, head) pairs (o and the final state rewritten)
   if (w.flags == nullptr || B * T == 0) return rc;
+  if (checked == nullptr) {
+    rc = gate_check(g, w.flags, H, K, si, dtype, st);
+    if (rc) return rc;
+  }
   return gate_fallback_fwd(q, k, v, g, h0, o, ht, scale, H, K, V, si, w.flags, dtype, st);
 }
 
@@ -887,9 +894,6 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
     a.si = si;
     rc = hip_status(tops::run_head_gate(a, st), "chunk_bwd (gating)");
     if (rc) return rc;
-  } else if (cflags) {
-    rc = gate_check(g, cflags, H, K, si, dtype, st);
-    if (rc) return rc;
   }
   auto head_scan = [&](bool rev, const void* a, const void* b, const float* s_init, void* s_all,
                        float* s_final, float sc) {
@@ -1033,6 +1037,14 @@ int tops_gla_chunk_bwd(const void* q, const void* k, const void* v, const void* 
   p.V = (int)V;
   p.vec = vec_ok(dtype, K, V, {q, k, v, g, dout, h, dh_ws, dq, dk, dv, dg});
   p.si = si;
+  if (cflags && gate == nullptr) {
+    if (dtype == TOPS_GLA_F32 && tops::f32_dv_supported(p)) {
+      p.flags = cflags;   // written by the dv kernel
+    } else {
+      rc = gate_check(g, cflags, H, K, si, dtype, st);
+      if (rc) return rc;
+    }
+  }
   if (head && tops::head_dqkg_supported((int)K, (int)V)) {
     // dq, dk, dg one block per (chunk, head) over every V tile; dv by the per-chunk kernel
     rc = hip_status(tops::run_head_dqkg(p, st), "chunk_bwd (dq, dk, dg)");

@@ -68,6 +68,7 @@ struct F32RowArgs {
   const float* x;      // v or do [tokens, H, V]
   const float* s;      // h or dh [NC, H, K, V] (nullable)
   float* out;          // o or dv [tokens, H, V]
+  int* flags;          // gate-range flags [NC, H] (gate_range.hip; nullable)
   float scale;
   int H, K, V;
   SeqInfo si;
@@ -104,6 +105,7 @@ __global__ __launch_bounds__(256, 3) void chunk_f32_kernel(F32RowArgs p) {
   f32x4 accA[3];
 #pragma unroll
   for (int j = 0; j < 3; ++j) accA[j] = zero4();
+  int wide = 0;   // a column's |g~ - r| beyond the factors' range, as gate_range_kernel has it
   for (int kt = 0; kt < KT; ++kt) {
     const int col = kt * 64 + lane;   // thread: one column, rows 16 w .. 16 w + 15
     const uint32_t cc = (uint32_t)min(col, K - 1);
@@ -121,6 +123,13 @@ __global__ __launch_bounds__(256, 3) void chunk_f32_kernel(F32RowArgs p) {
     float first, off, gamma;   // two buffers of sums: one barrier between write and read
     segment_cumsum(gv, sTot + (kt & 1) * 5 * 64, w, lane, first, off, gamma);
     const float r = 0.5f * (first + gamma);
+    float mx = -3.0e38f, mn = 3.0e38f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {   // rows past the chunk repeat its last one
+      mx = fmaxf(mx, gv[i] + off);
+      mn = fminf(mn, gv[i] + off);
+    }
+    wide |= fmaxf(mx - r, r - mn) * 1.4426950408889634f > kGateLimit2 ? 1 : 0;
     if (w == 0) sR[col] = DV ? gexp<float>(gamma - r) : p.scale * gexp<float>(r);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -160,7 +169,8 @@ __global__ __launch_bounds__(256, 3) void chunk_f32_kernel(F32RowArgs p) {
       for (int r = 0; r < 4; ++r) sT[(ii + r) * FP + jj] = a[r];
     }
   }
-  __syncthreads();
+  wide = __syncthreads_or(wide);
+  if (tid == 0 && p.flags && L % NB == 0) p.flags[L / NB] = wide ? 1 : 0;
 
   // ---- out = M x + L (f (.) S): this wave's 64 columns and 16 RT rows ----
   const int vb = (L % NB * NV + w % NV) * 64, rt0 = w / NV * RT;
@@ -733,8 +743,8 @@ bool f32_fwd_o_supported(const FwdOArgs& p) {
 }
 hipError_t run_f32_fwd_o(const FwdOArgs& p, hipStream_t st) {
   F32RowArgs a = {(const float*)p.q, (const float*)p.k, (const float*)p.g, (const float*)p.v,
-                  (const float*)p.h, (float*)p.o,       p.scale,           p.H,
-                  p.K,               p.V,               p.si};
+                  (const float*)p.h, (float*)p.o,       p.flags,           p.scale,
+                  p.H,               p.K,               p.V,               p.si};
   return pick_f32<false>(a, st);
 }
 
@@ -743,8 +753,8 @@ bool f32_dv_supported(const BwdArgs& p) {
 }
 hipError_t run_f32_dv(const BwdArgs& p, hipStream_t st) {
   F32RowArgs a = {(const float*)p.q,  (const float*)p.k, (const float*)p.g, (const float*)p.dout,
-                  (const float*)p.dh, (float*)p.dv,      p.scale,           p.H,
-                  p.K,                p.V,               p.si};
+                  (const float*)p.dh, (float*)p.dv,      p.flags,           p.scale,
+                  p.H,                p.K,               p.V,               p.si};
   return pick_f32<true>(a, st);
 }
 

@@ -1,5 +1,6 @@
 // Gate-range check of the chunked paths that do not track it inside their own kernels (the
-// per-chunk float32 kernels, and the bf16 wide-head and V > 128 backward).
+// per-chunk float32 kernels but those of chunk_f32.hip, and the bf16 wide-head and V > 128
+// backward).
 //
 // The chunk kernels factor e^{g~_i - g~_j} around a per-column reference
 // r = (g~_first + g~_last) / 2 (g~ the chunk-local inclusive cumsum of the raw log-gates,

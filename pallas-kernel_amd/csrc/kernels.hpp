@@ -37,6 +37,7 @@ struct FwdOArgs {
   float scale;
   int H, K, V;
   SeqInfo si;
+  int* flags;           // gate-range flags [NC, H] (nullable; f32_fwd_o_supported only)
 };
 hipError_t run_chunk_fwd_o(const FwdOArgs& p, int dtype, hipStream_t st);
 
@@ -76,6 +77,7 @@ struct BwdArgs {
   int H, K, V;
   int vec;              // every base pointer 16-byte aligned and K, V multiples of 16 bytes
   SeqInfo si;
+  int* flags;           // dv kernel: gate-range flags [NC, H] (nullable; f32_dv_supported only)
 };
 // Bytes of one (chunk, head) entry of the per-chunk gating workspace (chunk 64): qs = scale
 // q 2^{g~} and kg = k 2^{r-g~}, [64][K] bf16 each, A [64][64] bf16 (masked, scaled), the

@@ -122,3 +122,28 @@ def test_unaligned_rows_take_the_other_kernel():
     o, _ = G.chunk_gla(q, k, v, g, chunk_size=64)
     o2, _ = G.chunk_gla(q, k, v[..., :67].contiguous(), g, chunk_size=64)
     assert (o[..., :67] - o2).norm() / o2.norm() < 2e-6   # another order of float32 sums
+
+
+# the steep column in the first and last 64 key columns, in whole and partial chunks: the output
+# and dv kernels flag the chunk, and the recurrent kernels take the sequence and head
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [64, 260])
+@pytest.mark.parametrize("row,col", [(0, 0), (40, 99), (129, 70)])
+def test_gates_beyond_the_factors_range(row, col, V):
+    import tops.ops.gla as G
+
+    T, H, K = 130, 2, 100
+    gen = torch.Generator(device="cuda").manual_seed(row + col)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    q, k, v, h0 = mk(1, T, H, K), mk(1, T, H, K), mk(1, T, H, V), mk(1, H, K, V)
+    g = torch.nn.functional.logsigmoid(mk(1, T, H, K)) / 4
+    g[0, row, 1, col] = -300.0
+    do, dht = mk(1, T, H, V), mk(1, H, K, V)
+    ref = _ref(*(t.cpu() for t in (q, k, v, g, h0, do, dht)), [0, T])
+    xs = [t.requires_grad_(True) for t in (q, k, v, g, h0)]
+    o, ht = G.chunk_gla(*xs[:4], initial_state=h0, output_final_state=True, chunk_size=64)
+    got = [o, ht, *torch.autograd.grad([o, ht], xs, [do, dht])]
+    for name, a, b in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), got, ref):
+        assert torch.isfinite(a).all(), name
+        err = (a.detach().cpu().double() - b).norm() / b.norm()
+        assert err < 4e-6, (name, float(err))

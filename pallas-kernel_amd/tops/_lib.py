@@ -150,7 +150,7 @@ def call(name, *args):
 
 def full_head(K, V, chunk, dtype, backward):
     """True when the full-head kernels run this shape (see tops_gla_full_head)."""
-    return bool(load().tops_gla_full_head(K, V, chunk, dtype_code(dtype), 3 if backward else 2))
+    return bool(load().tops_gla_full_head(K, V, chunk, dtype_code(dtype), int(bool(backward))))
 
 
 def seg_workspace(B, T, H, K, V, chunk, varlen, dtype, device, N=None, backward=False):

@@ -57,3 +57,13 @@ def test_norm_without_gradients(dtype, gated):
     with torch.no_grad():
         got = rms_norm_gated(x, g, w, 1e-5)
     assert got.dtype == dtype and torch.equal(got, want)
+
+
+def test_full_head_query_of_each_direction():
+    """Wide heads: full-head forward (no per-chunk states without gradients), per-chunk backward."""
+    from tops import _lib
+
+    assert _lib.full_head(256, 512, 64, torch.bfloat16, False)
+    assert not _lib.full_head(256, 512, 64, torch.bfloat16, True)
+    assert _lib.full_head(128, 128, 64, torch.bfloat16, True)
+    assert not _lib.full_head(128, 128, 64, torch.float32, False)

@@ -903,14 +903,23 @@ bool short_scan(const RecScanArgs& p) {
          (long)p.si.N * p.H * ((p.C + 63) / 64) >= 256;
 }
 
-// The matrix-core scan from kChunkScanT tokens a sequence (packed sequences: on average).
-// Measured at B64 H16 K=V=128: it takes 34 us + 14 us per 16 tokens begun, the VALU scans
-// 22 us + 1.7 us a token (T = 17: 62 against 51 us, T = 64: 90 against 122); at B32 H4 K256
-// V512, 32 + 14 against 29 + 1.9 (T = 33: 73 against 91 us).
+// The matrix-core scan from kChunkScanT tokens a sequence (packed sequences: on average), whose
+// time goes by the 16 tokens begun, the VALU scans' by the token. Measured with the chip full, VALU
+// and matrix-core scan: B64 H16 K=V=128 60 and 65 us at T = 24, 73 and 66 at 32, 98 and 79 at 48,
+// 128 and 92 at 64; B64 H4 K256 V512 147 and 129, 170 and 134, 229 and 163, 286 and 193. So with K
+// up to 128 the VALU scans keep T below 28 and 33 to 40 there, where the last 16 tokens are mostly
+// missing. With K up to 64 a block's one producer wave serves 64 value columns unless 128 of them
+// fill the chip: B24 H8 K64 V128 T100 38 and 42 us, B64 H16 K=V=64 T64 47 and 52 us, so the VALU
+// scans keep those too once there are more blocks than CUs (B8 H16 K=V=64 T100: 34 and 22 us).
 constexpr long kChunkScanT = 24;
 bool chunk_scan(const RecScanArgs& p, int dtype, int o_dtype) {
-  return rec_chunk_supported(p, dtype, o_dtype) &&
-         (long)p.si.T >= kChunkScanT * (p.si.cu ? p.si.N : 1);
+  if (!rec_chunk_supported(p, dtype, o_dtype)) return false;
+  const long pairs = (long)p.si.N * p.H, T = p.si.cu ? p.si.T / p.si.N : p.si.T;
+  if (p.R <= 128 && pairs * ((p.C + 63) / 64) > 256) {
+    if (p.R <= 64 && pairs * (p.C / 128) < 256) return false;
+    if (T < 28 || (T > 32 && T <= 40)) return false;
+  }
+  return T >= kChunkScanT;
 }
 
 hipError_t run_scan(const RecScanArgs& p, int dtype, int o_dtype, hipStream_t st) {

@@ -24,6 +24,9 @@ CASES = [
     dict(B=1, T=100, H=1, K=256, V=130),
     dict(B=40, T=31, H=8, K=72, V=136),                    # 32 columns a wave, partial tiles
     dict(B=64, T=40, H=5, K=40, V=128, gate="none"),
+    dict(B=64, T=41, H=5, K=40, V=128, gate="none"),
+    dict(B=33, T=50, H=8, K=64, V=64),                     # more blocks than CUs: the VALU scan
+    dict(B=32, T=50, H=8, K=64, V=64),                     # as many
     dict(B=1, T=170, H=2, K=96, V=96, cu=[0, 1, 2, 18, 35, 36, 170]),
     dict(B=1, T=90, H=2, K=33, V=20, cu=[0, 16, 69, 70], reverse=True),   # tokens past the last
     dict(B=1, T=90, H=2, K=128, V=70, gate_mul=12.0),      # every chunk beyond the range

@@ -701,10 +701,13 @@ struct Raw {
   }
 };
 
-constexpr int SNT = 256, SNW = SNT / 64, STB = 16;
+constexpr int STB = 16;
 
-template <typename T, typename TO, int RPT>
-__global__ __launch_bounds__(SNT, 4) void rec_short_kernel(RecScanArgs p) {
+// SNW waves of 4 RPT rows each: 4 up to 128 rows, 8 above (RPT = 16 would take twice the
+// registers the loads in flight leave at four waves a SIMD).
+template <typename T, typename TO, int RPT, int SNW>
+__global__ __launch_bounds__(SNW * 64, 4) void rec_short_kernel(RecScanArgs p) {
+  constexpr int SNT = SNW * 64;
   __shared__ float sO[SNW * STB * 64];
   const int H = p.H, R = p.R, C = p.C;
   const int NCT = (C + 63) >> 6;
@@ -875,11 +878,11 @@ hipError_t dispatch_scan(const RecScanArgs& p, hipStream_t st) {
   return hipErrorInvalidValue;
 }
 
-template <typename T, typename TO, int RPT>
+template <typename T, typename TO, int RPT, int SNW = 4>
 hipError_t launch_short(const RecScanArgs& p, hipStream_t st) {
   const long blocks = (long)p.si.N * p.H * ((p.C + 63) / 64);
   if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL((rec_short_kernel<T, TO, RPT>), dim3((unsigned)blocks), dim3(SNT), 0, st,
+  hipLaunchKernelGGL((rec_short_kernel<T, TO, RPT, SNW>), dim3((unsigned)blocks), dim3(SNW * 64), 0, st,
                      p);
   return hipGetLastError();
 }
@@ -888,18 +891,27 @@ template <typename T, typename TO>
 hipError_t dispatch_short(const RecScanArgs& p, hipStream_t st) {
   if (p.R <= 32) return launch_short<T, TO, 2>(p, st);
   if (p.R <= 64) return launch_short<T, TO, 4>(p, st);
-  return launch_short<T, TO, 8>(p, st);
+  if (p.R <= 128) return launch_short<T, TO, 8>(p, st);
+  return launch_short<T, TO, 8, 8>(p, st);
 }
 
 // Plain forward scans (no gate-gradient epilogue, transposed state, shifted gates or flags)
-// of fixed-length sequences of at most kShortT tokens over at most 128 state rows: the short
+// of fixed-length sequences of at most kShortT tokens over at most 256 state rows: the short
 // scan kernel. Its steps wait on their own loads (one step ahead), the staged scan's on 16
 // steps loaded at once: measured at B64 H16 K=V=128, 27 + 3.5 us per token against 36 + 1.9,
 // so the short kernel only for a few tokens (decode).
+// Above 128 rows its blocks have eight waves (H4 K256 V512 bf16, staged scan and short one: B32
+// 34 -> 29 us at T = 1, 38 -> 36 at T = 4; B64 60 -> 52, 72 -> 64; B128 H2 K192 V256 33 -> 21). It
+// is the slower one there with float32 inputs past one token (B32 T2 42 and 43 us, T4 44 and 55) and
+// where the states read and written pass the 256 MB memory-side cache (B128 131 and 134 us, T4 147
+// and 171).
 constexpr int kShortT = 4;
-bool short_scan(const RecScanArgs& p) {
+bool short_scan(const RecScanArgs& p, int dtype) {
+  if (p.R > 128 && ((dtype == DT_F32 && p.si.T > 1) ||
+                    (long)p.si.N * p.H * p.R * p.C * 8 > (256L << 20)))
+    return false;
   return p.dg == nullptr && !p.s_trans && !p.shift && !p.final_gate && p.flags.p == nullptr &&
-         p.si.cu == nullptr && p.si.T <= kShortT && p.R <= 128 &&
+         p.si.cu == nullptr && p.si.T <= kShortT && p.R <= 256 &&
          (long)p.si.N * p.H * ((p.C + 63) / 64) >= 256;
 }
 
@@ -923,7 +935,7 @@ bool chunk_scan(const RecScanArgs& p, int dtype, int o_dtype) {
 }
 
 hipError_t run_scan(const RecScanArgs& p, int dtype, int o_dtype, hipStream_t st) {
-  if (short_scan(p)) {
+  if (short_scan(p, dtype)) {
     if (dtype == DT_BF16 && o_dtype == DT_F32) return dispatch_short<bf16, float>(p, st);
     if (dtype == DT_BF16 && o_dtype == DT_BF16) return dispatch_short<bf16, bf16>(p, st);
     if (dtype == DT_F32 && o_dtype == DT_F32) return dispatch_short<float, float>(p, st);

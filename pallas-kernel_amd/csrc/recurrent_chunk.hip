@@ -29,9 +29,10 @@
 // the decays of the next 16 in the other LDS buffer: one barrier per 16 tokens.
 //
 // Range: where a factored operand is above 2^50 (gates below about -4 a token over half a
-// chunk) or not finite, the 64 key columns of that producer are taken token by token from the
-// inputs, as the recurrence is written (37 us instead of 3.6 us a chunk when all of them are),
-// and all columns where v or the initial state is not finite: non-finite values then stay
+// chunk) or not finite, or a decay is above 2^58 or NaN (the first row's gate is in the decays
+// alone, not in an operand), the 64 key columns of that producer are taken token by token from
+// the inputs, as the recurrence is written (37 us instead of 3.6 us a chunk when all of them
+// are), and all columns where v or the initial state is not finite: non-finite values then stay
 // where the recurrence puts them.
 #include <type_traits>
 #include <utility>
@@ -48,6 +49,7 @@ constexpr int QCW = 4;             // consumer waves
 constexpr int QTP = 20;            // LDS pitch (floats) of rows of 16
 constexpr float kOperandMax = 1125899906842624.f;   // 2^50
 constexpr float kStateMax = 1.2676506e30f;          // 2^100
+constexpr float kDecayWeight = 4398046511104.f;     // 2^42
 constexpr uint32_t kOperandMaxBits = 0x5880u;       // as bf16
 
 template <int KP>
@@ -66,22 +68,25 @@ struct QLayout {   // byte offsets of one buffer
   static constexpr int bytes = 2 * buf;
 };
 
+constexpr float kLog2e = 1.44269502162933349609375f;   // log2(e) rounded to float
+constexpr float kLog2eRest = 1.92596299e-8f;           // log2(e) - kLog2e
 // e^x and e^-x to about an ulp at any size of x: x log2(e) as a rounded product plus its
 // remainder.
 __device__ __forceinline__ void exp_pair(float x, float& p, float& n) {
-  constexpr float L = 1.44269502162933349609375f;   // log2(e) rounded to float
-  constexpr float L2 = 1.92596299e-8f;              // log2(e) - L
-  const float hi = x * L;
-  const float lo = fmaf(x, L2, fmaf(x, L, -hi)) * 0.693147181f;
+  const float hi = x * kLog2e;
+  const float lo = fmaf(x, kLog2eRest, fmaf(x, kLog2e, -hi)) * 0.693147181f;
   p = __builtin_amdgcn_exp2f(hi);
   n = __builtin_amdgcn_exp2f(-hi);
   p = fmaf(p, lo, p);
   n = fmaf(n, -lo, n);
 }
+// e^x alone, for the decays. Where x log2(e) passes the float range (x = -inf among them) the
+// remainder is inf - inf; the maximum drops that NaN, so that e^x is 0 there (a NaN x stays).
 __device__ __forceinline__ float exp_one(float x) {
-  float p, n;
-  exp_pair(x, p, n);
-  return p;
+  const float hi = x * kLog2e;
+  const float lo = fmaf(x, kLog2eRest, fmaf(x, kLog2e, -hi)) * 0.693147181f;
+  const float p = __builtin_amdgcn_exp2f(hi);
+  return fmaf(p, fmaxf(lo, -1.f), p);
 }
 
 // f(0), f(1), .. with the indices as types: a loop that is unrolled before anything else is
@@ -241,7 +246,9 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
         }
         issue(n + 1);
         float dout[4], prevpost[4];
-        float sq = 0.f;   // sum of squares: at most kOperandMax^2, or an operand is too large
+        // sum of the operands' squares and the decays x 2^42: at most kOperandMax^2, or an operand
+        // or a decay (2^58) is too large
+        float sq = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float tot = (xg[0][e] + xg[1][e]) + (xg[2][e] + xg[3][e]);
@@ -276,6 +283,7 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
                                                            __float_as_uint(lpost[e]), false,
                                                            false);
           prevpost[e] = __uint_as_float(pp[1]);
+          sq = fmaf(d, kDecayWeight, sq);
           dout[e] = rg == 3 ? lpost[e] : d;
           lpost[e] = d;
           lsum[e] = half;

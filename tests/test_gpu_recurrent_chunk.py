@@ -90,3 +90,35 @@ def test_recurrent_chunk_non_finite(where, value):
         assert np.array_equal(np.isfinite(got), np.isfinite(ref)), name
         m = np.isfinite(ref)
         check(name, got[m], ref[m], "f32")
+
+
+def _same_non_finite(name, got, ref):
+    """The same infinities and NaN in the same places, the rest at the float32 bar."""
+    assert np.array_equal(np.isnan(got), np.isnan(ref)), name
+    assert np.array_equal(got == np.inf, ref == np.inf), name
+    assert np.array_equal(got == -np.inf, ref == -np.inf), name
+    m = np.isfinite(ref)
+    check(name, got[m], ref[m], "f32")
+
+
+# steps in the order of the scan: the first and last row of a 16-token chunk's halves, of the first
+# chunk (which has no decay before it) and of a later one
+@pytest.mark.parametrize("step", [0, 7, 8, 15, 16, 23, 24, 31])
+@pytest.mark.parametrize("value", [-np.inf, -3e38, np.nan])
+@pytest.mark.parametrize("c", [dict(B=1, T=50, H=2, K=64, V=40),
+                               dict(B=1, T=50, H=2, K=130, V=40, reverse=True),
+                               dict(B=1, T=70, H=2, K=64, V=40, cu=[0, 19, 70])],
+                         ids=["forward", "reverse", "packed"])
+def test_recurrent_chunk_clearing_gate(c, value, step):
+    """A gate whose e^g is 0 clears its row of the state at any row of a chunk; one that is NaN
+    reaches its row of the state and the outputs from there on. The row that is a chunk's first
+    has its gate in the chunk's decays alone, not in its operands."""
+    x = dict(zip(("q", "k", "v", "g", "s0"), _inputs(c)))
+    t = c["T"] - 1 - step if c.get("reverse") else c["cu"][1] + step if "cu" in c else step
+    x["g"][0, t, 1, 3] = value
+    print(f"recurrent chunk {c}, gate {value} at step {step}", flush=True)
+    args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
+    with np.errstate(all="ignore"):
+        refs = _oracle(*args, c)
+    for name, got, ref in zip(("o", "ht"), _call(*args, c), refs):
+        _same_non_finite(name, got, ref)

@@ -29,11 +29,11 @@
 // the decays of the next 16 in the other LDS buffer: one barrier per 16 tokens.
 //
 // Range: where a factored operand is above 2^50 (gates below about -4 a token over half a
-// chunk) or not finite, or a decay is above 2^58 or NaN (the first row's gate is in the decays
+// chunk) or not finite, or a half's decay is above 8 or NaN (the first row's gate is in the decays
 // alone, not in an operand), the 64 key columns of that producer are taken token by token from
 // the inputs, as the recurrence is written (37 us instead of 3.6 us a chunk when all of them
-// are), and all columns where v or the initial state is not finite: non-finite values then stay
-// where the recurrence puts them.
+// are), and all columns where v or the state is not finite or the state is large: non-finite
+// values, also of a state that overflows on the way, then stay where the recurrence puts them.
 #include <type_traits>
 #include <utility>
 
@@ -48,9 +48,9 @@ constexpr int QC = 16;             // tokens per chunk
 constexpr int QCW = 4;             // consumer waves
 constexpr int QTP = 20;            // LDS pitch (floats) of rows of 16
 constexpr float kOperandMax = 1125899906842624.f;   // 2^50
-constexpr float kStateMax = 1.2676506e30f;          // 2^100
-constexpr float kDecayWeight = 4398046511104.f;     // 2^42
-constexpr uint32_t kOperandMaxBits = 0x5880u;       // as bf16
+constexpr float kStateMax = 72057594037927936.f;    // 2^56
+constexpr float kDecayWeight = 1.5845633e29f;       // 2^97
+constexpr uint32_t kValueMaxBits = 0x4980u;         // 2^20 as bf16
 
 template <int KP>
 struct QLayout {   // byte offsets of one buffer
@@ -246,8 +246,8 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
         }
         issue(n + 1);
         float dout[4], prevpost[4];
-        // sum of the operands' squares and the decays x 2^42: at most kOperandMax^2, or an operand
-        // or a decay (2^58) is too large
+        // sum of the operands' squares and four decays x 2^97: above kOperandMax^2 where an operand
+        // is too large or the decays sum to more than 8
         float sq = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -351,7 +351,6 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
   const float* __restrict__ s0 = p.s0 ? p.s0 + sbase : nullptr;
   float* __restrict__ sN = p.sN ? p.sN + sbase : nullptr;
   f32x4 S[NVT][KT];
-  bool s_ok = true;
 #pragma unroll
   for (int i = 0; i < NVT; ++i)
 #pragma unroll
@@ -362,11 +361,22 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
         const float x = s0 ? s0[(uint32_t)min(kk, K - 1) * (uint32_t)V + (uint32_t)min(c, V - 1)]
                            : 0.f;
         S[i][kt][r] = kk < K && c < V ? x : 0.f;
-        s_ok = s_ok && fabsf(S[i][kt][r]) <= kStateMax;
       }
-  // an initial state that is not finite (or near the end of the range) stays with the
-  // recurrence as written
-  const bool s_bad = __ballot(s_ok) != ~0ull;
+  // A state that is not finite (or large enough to leave the range within a few chunks) stays with
+  // the recurrence as written: split into bf16 it would turn to NaN. Looked at before the first
+  // chunk and after every eighth and after columns taken as written. Between, decays of at most 8
+  // a half and 16 products of 2^50 2^20 a chunk keep a value below 2^48 (2^56 + 8 * 2^74).
+  auto state_ok = [&]() __attribute__((always_inline)) {
+    bool s_ok = true;
+#pragma unroll
+    for (int i = 0; i < NVT; ++i)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s_ok = s_ok && fabsf(S[i][kt][r]) <= kStateMax;
+    return __ballot(s_ok) == ~0ull;
+  };
+  bool check = true;
   __builtin_amdgcn_sched_barrier(0);
   uint32_t Rv[NVT][4], vo[4];
 #pragma unroll
@@ -413,20 +423,21 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         x[m] = 4 * g4 + m < len && cb + i * 16 < V ? Rv[i][m] : 0u;
-        ok = ok && (x[m] & 0x7fffu) <= kOperandMaxBits;
+        ok = ok && (x[m] & 0x7fffu) <= kValueMaxBits;
       }
       const uint2 w = make_uint2(x[0] | (x[1] << 16), x[2] | (x[3] << 16));
       vv[i] = __builtin_bit_cast(s4_t, w);
     }
     issue_v(n + 1);
     // key column groups (a producer's 64) to be taken token by token: those flagged, or all
-    // where this wave's columns of v or its initial state are not finite
+    // where this wave's columns of v or its state are not finite
     int seq_groups = 0;
 #pragma unroll
     for (int j = 0; j < PW; ++j)
       seq_groups |= (reinterpret_cast<const int*>(B + Lay::bad)[j] != 0) << j;
     seq_groups = __builtin_amdgcn_readfirstlane(seq_groups);
-    const bool all_seq = s_bad || __ballot(ok) != ~0ull;
+    bool all_seq = __ballot(ok) != ~0ull;
+    if (__builtin_expect(check, 0)) all_seq = all_seq || !state_ok();
     f32x4 o[NVT];
     if (__builtin_expect(!all_seq, 1)) {
       const float* dec = reinterpret_cast<const float*>(B + (owed ? Lay::dec : Lay::pre)) + 4 * g4;
@@ -544,6 +555,7 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
 #pragma unroll
       for (int i = 0; i < NVT; ++i) o[i] = zero4();
     }
+    check = seq_groups != 0 || (n & 7) == 7;
     if (__builtin_expect(seq_groups != 0, 0)) {
       // the recurrence as written for the tiles of these groups, four tokens at a time (their
       // inputs from global memory, the next tile's under the work on this one); a row's part of

@@ -122,3 +122,34 @@ def test_recurrent_chunk_clearing_gate(c, value, step):
         refs = _oracle(*args, c)
     for name, got, ref in zip(("o", "ht"), _call(*args, c), refs):
         _same_non_finite(name, got, ref)
+
+
+@pytest.mark.parametrize("c", [dict(B=1, T=50, H=2, K=64, V=40),
+                               dict(B=1, T=50, H=2, K=130, V=40, reverse=True),
+                               dict(B=1, T=70, H=1, K=256, V=70, cu=[0, 30, 70]),
+                               dict(B=40, T=31, H=8, K=72, V=136)],
+                         ids=["K64", "K130-reverse", "K256-packed", "wide-tiles"])
+def test_recurrent_chunk_state_overflows(c):
+    """A state that grows out of the float range during the scan (gates of +2 on one key column of
+    a state near 1e29) gives the infinities of the recurrence in float32, in its value column
+    alone: columns that stay in range, and the tokens before, keep their values."""
+    x = dict(zip(("q", "k", "v", "g", "s0"), _inputs(c)))
+    V = c["V"]
+    # without keys the row only grows: no term cancels another
+    x["g"][..., 3], x["q"][..., 3], x["k"][..., 3] = 2.0, 1.0, 0.0
+    x["s0"][..., 3, : V // 2] *= 1e29
+    x["s0"] = x["s0"].astype(np.float32).astype(np.float64)
+    print(f"recurrent chunk {c}, a state that overflows", flush=True)
+    args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
+    with np.errstate(all="ignore"):
+        refs = orc.fused_recurrent_gla(*args[:3], gk=args[3], initial_state=args[4],
+                                       output_final_state=True, reverse=c.get("reverse", False),
+                                       cu_seqlens=c.get("cu"), dtype=np.float32)
+    for name, got, ref in zip(("o", "ht"), _call(*args, c), refs):
+        assert np.isinf(ref).any() and np.isfinite(ref).any()
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), name
+        assert np.array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(ref), ref, 0)), name
+        m = np.isfinite(ref)
+        # up to 50 roundings of a state and of e^g, each 2^-23 at most; other rows add order one
+        err = np.abs(got[m] - ref[m]) / np.maximum(np.abs(ref[m]), 1.0)
+        assert err.max() <= 2e-5, (name, err.max())

@@ -28,15 +28,15 @@
 // qa, ka, the 16 x 16 products A (each over its own 64 key columns, summed by the reader) and
 // the decays of the next 16 in the other LDS buffer: one barrier per 16 tokens.
 //
-// Range: where a factored operand is above 2^50 (gates below about -4 a token over half a
-// chunk) or not finite, or a half's decay is above 8 or NaN (the first row's gate is in the decays
-// alone, not in an operand), the 64 key columns of that producer are taken token by token from
-// the inputs, as the recurrence is written (37 us instead of 3.6 us a chunk when all of them
-// are), and all columns where v or the state is not finite or the state is large: non-finite
-// values, also of a state that overflows on the way, then stay where the recurrence puts them.
-#include <type_traits>
-#include <utility>
-
+// Range. A factored operand above 2^50 (gates below about -4 a token over half a chunk) or not
+// finite, a half's decay above 8 or NaN (the first row's gate is in the decays alone, not in an
+// operand), a v above 2^20 or not finite, a state above 2^56 or not finite: the block takes the
+// sequence from that chunk on as the recurrence is written, on the VALU (below), so that
+// non-finite values stay where the recurrence puts them and no gate costs more than the VALU scan
+// of recurrent.hip. Measured with gates near -8, that scan and this kernel: B8 T2048 H4 K256 V512
+// 950 and 921 us, B8 T2048 H16 K=V=128 666 and 561, B3 T1000 H16 K=V=64 313 and 198; only the
+// start weighs on short sequences (B64 T64 H16 K=V=128 124 and 159). Taken token by token from
+// the registers of the matrix path instead, a chunk cost 15 to 37 us in place of 3.6.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -52,7 +52,9 @@ constexpr float kStateMax = 72057594037927936.f;    // 2^56
 constexpr float kDecayWeight = 1.5845633e29f;       // 2^97
 constexpr uint32_t kValueMaxBits = 0x4980u;         // 2^20 as bf16
 
-template <int KP>
+constexpr int RTB = 8;             // tokens per stage of the element-wise phase
+
+template <int KP, int NVT>
 struct QLayout {   // byte offsets of one buffer
   static constexpr int QP = KP + 8, KQ = KP + 16;    // row pitches (bf16) of qa and ka
   static constexpr int PW = KP / 64;                 // producer waves
@@ -63,9 +65,15 @@ struct QLayout {   // byte offsets of one buffer
   // post x pre; pre = e^{sum of rows 0..7}; post = e^{sum of rows 8..15}; the previous post
   static constexpr int dec = A + PW * QC * QTP * 4;
   static constexpr int pre = dec + KP * 4, post = pre + KP * 4, ppost = post + KP * 4;
-  static constexpr int bad = ppost + KP * 4;         // [4] ints
-  static constexpr int buf = bad + 16;
-  static constexpr int bytes = 2 * buf;
+  static constexpr int flag = ppost + KP * 4;        // [4] of the producers, [4] of the consumers
+  static constexpr int buf = flag + 32;
+  // element-wise phase, in the same place: k, so q, e^g [RTB][KP] and v [RTB][CB] f32, twice; the
+  // consumers' sums [QCW][RTB][CB] f32, twice; before it the state [KP][CB + 4] f32
+  static constexpr int CB = QCW * NVT * 16;
+  static constexpr int stage = RTB * (3 * KP + CB) * 4, sums = QCW * RTB * CB * 4;
+  static constexpr int cmax(int a, int b) { return a > b ? a : b; }
+  static constexpr int bytes =
+      cmax(2 * buf, cmax(2 * (stage + sums), KP * (CB + 4) * 4));
 };
 
 constexpr float kLog2e = 1.44269502162933349609375f;   // log2(e) rounded to float
@@ -89,11 +97,8 @@ __device__ __forceinline__ float exp_one(float x) {
   return fmaf(p, fmaxf(lo, -1.f), p);
 }
 
-// f(0), f(1), .. with the indices as types: a loop that is unrolled before anything else is
-// done to it, also around an inner run-time loop.
-template <class F, int... I>
-__device__ __forceinline__ void each_tile(F& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
+__device__ __forceinline__ float comp(const float4& x, int i) {   // i known once unrolled
+  return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w;
 }
 
 __device__ __forceinline__ float4 add4(const float4& a, const float4& b) {
@@ -141,13 +146,230 @@ __device__ __forceinline__ void mma_split(const s4_t (&a)[3], const s4_t (&b)[3]
 
 }  // namespace
 
+// The element-wise phase: the rest of a sequence from token t0 on as the recurrence is written.
+// The producers stage RTB tokens' k, so q, e^g and v as floats and write the outputs of the stage
+// before; a consumer wave has KP / 4 state rows of all CB columns, a lane KP / 16 rows of four
+// (eight) columns, so that an operand read from LDS meets four products, and its sums over the
+// rows meet the other waves' in LDS. VALU issue bounds it (three operations a state value); one
+// barrier a stage, a token's LDS reads under the products of the one before (944 -> 921 us at B8
+// T2048 H4 K256 V512).
+template <int KP, int NVT, bool VEC>
+__device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsigned char* qsm, int t0, int T,
+                                      int bos, int eos, int hh, int ct, int pw, int lane) {
+  using Lay = QLayout<KP, NVT>;
+  constexpr int PW = Lay::PW, CB = Lay::CB, NV = RTB * CB / (PW * 64);
+  const int H = p.H, K = p.R, V = p.C;
+  const long rsK = (long)H * K, rsV = (long)H * V;
+  const bf16* q = (const bf16*)p.o + (long)hh * K;
+  const bf16* k = (const bf16*)p.a + (long)hh * K;
+  const bf16* gk = (const bf16*)(p.ga ? p.ga : p.a) + (long)hh * K;
+  const bf16* v = (const bf16*)p.b + (long)hh * V;
+  const uint32_t gmask = p.ga ? ~0u : 0u;
+  const int NS = (T - t0 + RTB - 1) / RTB, c0 = pw * 64 + 4 * (lane & 15);
+  auto tok = [&](int t) { return (long)(p.dir ? eos - 1 - t : bos + t); };   // t < T
+  uint2 raw[2][3];      // two tokens of four key columns
+  uint32_t rv[NV];      // values: token and column of index (i PW + pw) 64 + lane
+  auto load = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const long at = tok(min(t0 + s * RTB + 2 * (lane >> 4) + u, T - 1)) * rsK;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const bf16* base = (a == 0 ? q : a == 1 ? k : gk) + at;
+        if constexpr (VEC) {
+          raw[u][a] = *reinterpret_cast<const uint2*>(base + max(min(c0, K - 4), 0));
+        } else {
+          uint32_t x[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = base[min(c0 + e, K - 1)].u;
+          raw[u][a] = make_uint2(x[0] | (x[1] << 16), x[2] | (x[3] << 16));
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int x = (i * PW + pw) * 64 + lane;
+      rv[i] = v[tok(min(t0 + s * RTB + x / CB, T - 1)) * rsV + min(ct * CB + x % CB, V - 1)].u;
+    }
+  };
+  auto store = [&](int s) __attribute__((always_inline)) {   // tokens past the end are not read
+    float* B = reinterpret_cast<float*>(qsm + (s & 1) * Lay::stage);
+    uint32_t cm[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      cm[e] = (c0 + 2 * e < K ? 0xffffu : 0u) | (c0 + 2 * e + 1 < K ? 0xffff0000u : 0u);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int at = (2 * (lane >> 4) + u) * KP + c0;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const uint32_t m = a == 2 ? gmask : ~0u;
+        const uint32_t x = raw[u][a].x & cm[0] & m, y = raw[u][a].y & cm[1] & m;
+        float f[4] = {bf16_lo(x), bf16_hi(x), bf16_lo(y), bf16_hi(y)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = a == 0 ? p.so * f[e] : a == 2 ? gexp<bf16>(f[e]) : f[e];
+        // k, so q, e^g
+        *reinterpret_cast<float4*>(B + (a == 0 ? 1 : a == 1 ? 0 : 2) * RTB * KP + at) =
+            make_float4(f[0], f[1], f[2], f[3]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int x = (i * PW + pw) * 64 + lane;
+      B[3 * RTB * KP + x] = ct * CB + x % CB < V ? bf16_lo(rv[i]) : 0.f;
+    }
+  };
+  auto output = [&](int s) __attribute__((always_inline)) {
+    const float* O = reinterpret_cast<const float*>(qsm + 2 * Lay::stage + (s & 1) * Lay::sums);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int x = (i * PW + pw) * 64 + lane, t = t0 + s * RTB + x / CB, c = ct * CB + x % CB;
+      if (t < T && c < V)
+        ((float*)p.out)[tok(t) * rsV + (long)hh * V + c] =
+            (O[x] + O[RTB * CB + x]) + (O[2 * RTB * CB + x] + O[3 * RTB * CB + x]);
+    }
+  };
+  load(0);
+  __syncthreads();
+  __syncthreads();   // the state is in LDS
+  __syncthreads();   // and out of it
+  store(0);
+  if (NS > 1) load(1);
+  for (int s = 0; s < NS; ++s) {
+    __syncthreads();
+    if (s + 1 < NS) store(s + 1);
+    if (s + 2 < NS) load(s + 2);
+    if (s > 0) output(s - 1);
+  }
+  __syncthreads();
+  output(NS - 1);
+}
+
+template <int KP, int NVT>
+__device__ __forceinline__ void rec_elements_consumer(const RecScanArgs& p, unsigned char* qsm, int t0, int T,
+                                      float* sN, int ct, int w, int lane) {
+  using Lay = QLayout<KP, NVT>;
+  constexpr int CB = Lay::CB, R = KP / 16;
+  const int K = p.R, V = p.C;
+  const int cg = 4 * (lane & 15), r0 = (w * 4 + (lane >> 4)) * R;
+  const int NS = (T - t0 + RTB - 1) / RTB;
+  float S[R][NVT][4];
+  __syncthreads();   // the state is in LDS
+  {
+    const float* X = reinterpret_cast<const float*>(qsm);
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int u = 0; u < NVT; ++u) {
+        const float4 x = *reinterpret_cast<const float4*>(X + (r0 + j) * (CB + 4) + 64 * u + cg);
+        S[j][u][0] = x.x;
+        S[j][u][1] = x.y;
+        S[j][u][2] = x.z;
+        S[j][u][3] = x.w;
+      }
+  }
+  __syncthreads();
+  for (int s = 0; s < NS; ++s) {
+    __syncthreads();
+    const float* B = reinterpret_cast<const float*>(qsm + (s & 1) * Lay::stage);
+    float* O = reinterpret_cast<float*>(qsm + 2 * Lay::stage + (s & 1) * Lay::sums) + w * RTB * CB;
+    const int nt = min(RTB, T - t0 - s * RTB);
+    // a token's operands, read while the one before it is computed
+    struct Step {
+      float4 b[NVT], a[R / 4], o[R / 4], e[R / 4];
+    };
+    auto load = [&](int t, Step& x) __attribute__((always_inline)) {
+      t = min(t, RTB - 1);   // past the stage: not used
+#pragma unroll
+      for (int u = 0; u < NVT; ++u)
+        x.b[u] = *reinterpret_cast<const float4*>(B + 3 * RTB * KP + t * CB + 64 * u + cg);
+#pragma unroll
+      for (int j = 0; j < R / 4; ++j) {
+        const float4* row = reinterpret_cast<const float4*>(B + t * KP + r0) + j;
+        x.a[j] = row[0];
+        x.o[j] = row[RTB * KP / 4];
+        x.e[j] = row[2 * RTB * KP / 4];
+      }
+    };
+    auto step = [&](int t, const Step& x) __attribute__((always_inline)) {
+      float sum[NVT][4];
+#pragma unroll
+      for (int u = 0; u < NVT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[u][i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const float a = comp(x.a[j / 4], j % 4), o = comp(x.o[j / 4], j % 4);
+        const float e = comp(x.e[j / 4], j % 4);
+#pragma unroll
+        for (int u = 0; u < NVT; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float& st = S[j][u][i];
+            st *= e;
+            st = fmaf(a, comp(x.b[u], i), st);
+            sum[u][i] = fmaf(o, st, sum[u][i]);
+          }
+      }
+      // over the wave's four row groups: lane l ends with column 4 (l & 15) + (l >> 4)
+#pragma unroll
+      for (int u = 0; u < NVT; ++u) {
+        const auto p0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum[u][0]),
+                                                         __float_as_uint(sum[u][2]), false, false);
+        const auto p1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum[u][1]),
+                                                         __float_as_uint(sum[u][3]), false, false);
+        const float u0 = __uint_as_float(p0[0]) + __uint_as_float(p0[1]);
+        const float u1 = __uint_as_float(p1[0]) + __uint_as_float(p1[1]);
+        const auto p2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(u0), __float_as_uint(u1),
+                                                         false, false);
+        O[t * CB + 64 * u + cg + (lane >> 4)] = __uint_as_float(p2[0]) + __uint_as_float(p2[1]);
+      }
+    };
+    Step x0, x1;
+    load(0, x0);
+#pragma unroll 1
+    for (int t = 0; t < nt; t += 2) {
+      load(t + 1, x1);
+      __builtin_amdgcn_sched_barrier(0);   // the reads issue before the token's products
+      step(t, x0);
+      if (t + 1 >= nt) break;
+      load(t + 2, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      step(t + 1, x1);
+    }
+  }
+  __syncthreads();
+  if (sN) {
+    const bool whole = V % 4 == 0 && ((uintptr_t)sN & 15) == 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int u = 0; u < NVT; ++u) {
+        const int c = ct * CB + 64 * u + cg;
+        if (whole && r0 + j < K && c < V)
+          *reinterpret_cast<float4*>(sN + (uint32_t)(r0 + j) * (uint32_t)V + (uint32_t)c) =
+              make_float4(S[j][u][0], S[j][u][1], S[j][u][2], S[j][u][3]);
+      }
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int u = 0; u < NVT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int c = ct * CB + 64 * u + cg + i;
+          if (!whole && r0 + j < K && c < V)
+            sN[(uint32_t)(r0 + j) * (uint32_t)V + (uint32_t)c] = S[j][u][i];
+        }
+  }
+}
+
 // KP: K rounded up to 64, 128 or 256; NVT: 16-column tiles per consumer wave; VEC: K % 4 == 0
 // and q, k, g rows aligned to 8 bytes.
 template <int KP, int NVT, bool VEC>
 __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
     void rec_chunk_kernel(RecScanArgs p) {
-  using Lay = QLayout<KP>;
-  constexpr int PW = Lay::PW, KT = KP / 16, CB = QCW * NVT * 16;
+  using Lay = QLayout<KP, NVT>;
+  constexpr int PW = Lay::PW, KT = KP / 16, CB = Lay::CB;
   constexpr int NOM = KT == 16 ? 4 : 2;   // sums of o's main products, by tile
   extern __shared__ __attribute__((aligned(16))) unsigned char qsm[];
   const int H = p.H, K = p.R, V = p.C;
@@ -177,6 +399,18 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
   auto chunk_t0 = [&](int n, int len) {   // uniform: the chunk's first token in memory order
     return (long)(p.dir ? eos - n * QC - len : bos + n * QC);
   };
+
+  // Whether the block leaves for the element-wise phase at chunk n: a producer could not factor its
+  // columns of it, or a consumer asked for it before the chunk. The same for every wave: chunk n's
+  // flags stand between its barrier and the next.
+  auto leaves = [&](int n) __attribute__((always_inline)) {
+    const int* f = reinterpret_cast<const int*>(qsm + (n & 1) * Lay::buf + Lay::flag);
+    int x = f[4] | f[5] | f[6] | f[7];
+#pragma unroll
+    for (int j = 0; j < PW; ++j) x |= f[j];
+    return __builtin_amdgcn_readfirstlane(x) != 0;
+  };
+  int left = NC;   // the first chunk of the element-wise phase
 
   if (w >= QCW) {
     // ---- producers: lane = 4 key columns (lane & 15) x 4 rows (lane >> 4) ----
@@ -245,7 +479,7 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
           }
         }
         issue(n + 1);
-        float dout[4], prevpost[4];
+        float dout[4];
         // sum of the operands' squares and four decays x 2^97: above kOperandMax^2 where an operand
         // is too large or the decays sum to more than 8
         float sq = 0.f;
@@ -279,29 +513,13 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
                                                            false);
           const float prev = __uint_as_float(ps[1]);   // the upper half's value
           const float d = exp_one(rg == 0 ? half + prev : half);
-          const auto pp = __builtin_amdgcn_permlane32_swap(__float_as_uint(lpost[e]),
-                                                           __float_as_uint(lpost[e]), false,
-                                                           false);
-          prevpost[e] = __uint_as_float(pp[1]);
           sq = fmaf(d, kDecayWeight, sq);
           dout[e] = rg == 3 ? lpost[e] : d;
           lpost[e] = d;
           lsum[e] = half;
         }
         const bool good = __ballot(sq <= kOperandMax * kOperandMax) == ~0ull;
-        if (lane == 0) reinterpret_cast<int*>(B + Lay::bad)[pw] = !good;
-        if (!good) {
-          // these 64 columns are left to the recurrence as written: operands that add nothing
-          // and leave the state as it enters the chunk
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            dout[e] = rg == 0 ? prevpost[e] : rg == 3 ? dout[e] : 1.f;
-            lpost[e] = 1.f;
-            lsum[e] = 0.f;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) xq[u][e] = xk[u][e] = 0.f;
-          }
-        }
+        if (lane == 0) reinterpret_cast<int*>(B + Lay::flag)[pw] = good ? 0 : 1;
         *reinterpret_cast<float4*>(B + Lay::dec + (rg * KP + c0) * 4) =
             make_float4(dout[0], dout[1], dout[2], dout[3]);
         bf16* sQ = reinterpret_cast<bf16*>(B + Lay::qa);
@@ -338,6 +556,14 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
                                                (lane & 15)] = am[0][r];
       }
       __syncthreads();
+      if (__builtin_expect(leaves(n), 0)) {
+        left = n;
+        break;
+      }
+    }
+    if (left < NC) {
+      rec_elements_producer<KP, NVT, VEC>(p, qsm, left * QC, T, bos, eos, hh, ct, pw, lane);
+      return;
     }
     __syncthreads();
     return;
@@ -362,10 +588,10 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
                            : 0.f;
         S[i][kt][r] = kk < K && c < V ? x : 0.f;
       }
-  // A state that is not finite (or large enough to leave the range within a few chunks) stays with
+  // A state that is not finite (or large enough to leave the range within a few chunks) is left to
   // the recurrence as written: split into bf16 it would turn to NaN. Looked at before the first
-  // chunk and after every eighth and after columns taken as written. Between, decays of at most 8
-  // a half and 16 products of 2^50 2^20 a chunk keep a value below 2^48 (2^56 + 8 * 2^74).
+  // chunk and after every eighth. Between, decays of at most 8 a half and 16 products of 2^50 2^20
+  // a chunk keep a value below 2^48 (2^56 + 8 * 2^74).
   auto state_ok = [&]() __attribute__((always_inline)) {
     bool s_ok = true;
 #pragma unroll
@@ -374,9 +600,8 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s_ok = s_ok && fabsf(S[i][kt][r]) <= kStateMax;
-    return __ballot(s_ok) == ~0ull;
+    return s_ok;
   };
-  bool check = true;
   __builtin_amdgcn_sched_barrier(0);
   uint32_t Rv[NVT][4], vo[4];
 #pragma unroll
@@ -409,13 +634,10 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
   // whether S still has the last chunk's post factor to come (it meets the next chunk's pre
   // in one factor)
   bool owed = false;
-  if (NC > 0) issue_v(0);
-  __syncthreads();
-#pragma unroll 1
-  for (int n = 0; n < NC; ++n) {
-    const unsigned char* B = qsm + (n & 1) * Lay::buf;
-    const int len = min(QC, T - n * QC);
-    s4_t vv[NVT];   // rows 4 g4 .. 4 g4 + 3 of the lane's column
+  s4_t vv[NVT];   // rows 4 g4 .. 4 g4 + 3 of the lane's column
+  // chunk n's v as operands, once loaded; ok: whether every value is small enough
+  auto take_v = [&](int n) __attribute__((always_inline)) {
+    const int len = T - n * QC;
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < NVT; ++i) {
@@ -428,218 +650,141 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
       const uint2 w = make_uint2(x[0] | (x[1] << 16), x[2] | (x[3] << 16));
       vv[i] = __builtin_bit_cast(s4_t, w);
     }
-    issue_v(n + 1);
-    // key column groups (a producer's 64) to be taken token by token: those flagged, or all
-    // where this wave's columns of v or its state are not finite
-    int seq_groups = 0;
-#pragma unroll
-    for (int j = 0; j < PW; ++j)
-      seq_groups |= (reinterpret_cast<const int*>(B + Lay::bad)[j] != 0) << j;
-    seq_groups = __builtin_amdgcn_readfirstlane(seq_groups);
-    bool all_seq = __ballot(ok) != ~0ull;
-    if (__builtin_expect(check, 0)) all_seq = all_seq || !state_ok();
-    f32x4 o[NVT];
-    if (__builtin_expect(!all_seq, 1)) {
-      const float* dec = reinterpret_cast<const float*>(B + (owed ? Lay::dec : Lay::pre)) + 4 * g4;
-      const bf16* pq = reinterpret_cast<const bf16*>(B + Lay::qa) + li * Lay::QP + 4 * g4;
-      // transposed reads of 4 rows x 16 columns: this lane's address is row li >> 2 of its
-      // group's four, columns 4 (li & 3); it receives column li
-      const bf16* pk = reinterpret_cast<const bf16*>(B + Lay::ka) +
-                       (4 * g4 + (li >> 2)) * Lay::KQ + 4 * (li & 3);
-      float4 d[2];
-      s4_t x[2][3], y[2][3];
-      auto operands = [&](int kt) __attribute__((always_inline)) {
-        d[kt & 1] = *reinterpret_cast<const float4*>(dec + kt * 16);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          x[kt & 1][i] = *reinterpret_cast<const s4_t*>(pq + i * QC * Lay::QP + kt * 16);
-          y[kt & 1][i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) s4_t*)(pk + i * QC * Lay::KQ + kt * 16));
-        }
-      };
-      operands(0);
-      // Step kt: tile kt's qa S' (the main products in NOM sums, the others in three)
-      // and ka^T v onto the state, with the next tile decayed to the chunk's middle and split
-      // meanwhile and the one after it read from LDS. The order of the products keeps those of
-      // one sum apart, and the VALU work sits between them (an MFMA occupies its own pipe for
-      // 16 cycles, a VALU operation 4).
-      f32x4 om[NVT][NOM], orest[NVT][3];
-      float4 ap[PW];
-      Split sp[NVT][2];
-      auto decay = [&](int kt) __attribute__((always_inline)) {   // S' of tile kt, split
-        const float4 dd = d[kt & 1];
-#pragma unroll
-        for (int i = 0; i < NVT; ++i) {
-          S[i][kt][0] *= dd.x;
-          S[i][kt][1] *= dd.y;
-          S[i][kt][2] *= dd.z;
-          S[i][kt][3] *= dd.w;
-          const float t[4] = {S[i][kt][0], S[i][kt][1], S[i][kt][2], S[i][kt][3]};
-          sp[i][kt & 1] = split3(t);
-        }
-      };
-      decay(0);
-      operands(1);
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) {
-#pragma unroll
-        for (int j = 0; j < NOM; ++j) om[i][j] = zero4();
-#pragma unroll
-        for (int j = 0; j < 3; ++j) orest[i][j] = zero4();
-      }
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        const int c = kt & 1;
-        s4_t xx[3], yy[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          xx[j] = x[c][j];
-          yy[j] = y[c][j];
-        }
-#pragma unroll
-        for (int i = 0; i < NVT; ++i) {
-          const s4_t(&b)[3] = sp[i][c].p;
-          f32x4(&r)[3] = orest[i];
-          f32x4& t = S[i][kt];
-          om[i][kt % NOM] = mma16(xx[0], b[0], om[i][kt % NOM]);
-          t = mma16(yy[2], vv[i], t);
-          r[0] = mma16(xx[2], b[0], r[0]);
-          r[1] = mma16(xx[0], b[2], r[1]);
-          t = mma16(yy[1], vv[i], t);
-          r[2] = mma16(xx[1], b[1], r[2]);
-          r[0] = mma16(xx[1], b[0], r[0]);
-          t = mma16(yy[0], vv[i], t);
-          r[1] = mma16(xx[0], b[1], r[1]);
-        }
-        if (kt + 1 < KT) decay(kt + 1);
-        if (kt + 2 < KT) {
-          operands(kt + 2);
-        } else if (kt + 2 == KT) {
-#pragma unroll
-          for (int j = 0; j < PW; ++j)
-            ap[j] = *reinterpret_cast<const float4*>(
-                B + Lay::A + ((j * QC + li) * QTP + 4 * g4) * 4);
-        }
-#pragma unroll
-        for (int j = 0; j < 9 * NVT; ++j) {
-          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // one MFMA, four VALU
-          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // A v: row li, tokens 4 g4 ..; those after the row left out
-      const float4 am = PW == 1   ? ap[0]
-                        : PW == 2 ? add4(ap[0], ap[PW / 2])
-                                  : add4(add4(ap[0], ap[1 % PW]), add4(ap[PW / 2], ap[PW - 1]));
-      const int after = li - 4 * g4;
-      const float aa[4] = {after >= 0 ? am.x : 0.f, after >= 1 ? am.y : 0.f,
-                           after >= 2 ? am.z : 0.f, after >= 3 ? am.w : 0.f};
-      const Split as = split3(aa);
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) {
-        f32x4 u = zero4();
-#pragma unroll
-        for (int j = 2; j >= 0; --j) u = mma16(as.p[j], vv[i], u);
-        u += orest[i][0] + orest[i][1] + orest[i][2];
-#pragma unroll
-        for (int st = NOM / 2; st > 0; st /= 2)
-#pragma unroll
-          for (int j = 0; j < st; ++j) om[i][j] += om[i][j + st];
-        o[i] = om[i][0] + u;
-      }
-      owed = true;
-    } else {
-      if (owed) mul_rows(B + Lay::ppost);
-      owed = false;
-      seq_groups = (1 << PW) - 1;
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) o[i] = zero4();
-    }
-    check = seq_groups != 0 || (n & 7) == 7;
-    if (__builtin_expect(seq_groups != 0, 0)) {
-      // the recurrence as written for the tiles of these groups, four tokens at a time (their
-      // inputs from global memory, the next tile's under the work on this one); a row's part of
-      // o is summed over the tiles and lanes and joins the lanes that hold the tokens' rows
+    return ok;
+  };
+  // this wave's request for chunk n: its v or the state are not fit for the matrix cores
+  auto request = [&](int n, bool ok) __attribute__((always_inline)) {
+    const int x = __ballot(ok) == ~0ull ? 0 : 1;
+    if (lane == 0) reinterpret_cast<int*>(qsm + (n & 1) * Lay::buf + Lay::flag)[4 + w] = x;
+  };
+  if (NC > 0) {
+    issue_v(0);
+    const bool s_ok = state_ok();
+    request(0, take_v(0) && s_ok);
+  }
+  __syncthreads();
 #pragma unroll 1
-      for (int b4 = 0; b4 < 4 && 4 * b4 < len; ++b4) {
-        // the lane's indices through an empty asm: formed anew here, not held in registers
-        // (for every tile) around the loops of the other path
-        int gl = g4, cl = cb;
-        asm volatile("" : "+v"(gl), "+v"(cl));
-        // rows past the sequence: its last row's address, gate 0, k and q 0
-        const long at = chunk_t0(n, len);
-        uint32_t to[4];
-        float xv[NVT][4], os[NVT][4];
+  for (int n = 0; n < NC; ++n) {
+    const unsigned char* B = qsm + (n & 1) * Lay::buf;
+    const int len = min(QC, T - n * QC);
+    issue_v(n + 1);
+    if (__builtin_expect(leaves(n), 0)) {
+      left = n;
+      break;
+    }
+    f32x4 o[NVT];
+    const float* dec = reinterpret_cast<const float*>(B + (owed ? Lay::dec : Lay::pre)) + 4 * g4;
+    const bf16* pq = reinterpret_cast<const bf16*>(B + Lay::qa) + li * Lay::QP + 4 * g4;
+    // transposed reads of 4 rows x 16 columns: this lane's address is row li >> 2 of its
+    // group's four, columns 4 (li & 3); it receives column li
+    const bf16* pk = reinterpret_cast<const bf16*>(B + Lay::ka) +
+                     (4 * g4 + (li >> 2)) * Lay::KQ + 4 * (li & 3);
+    float4 d[2];
+    s4_t x[2][3], y[2][3];
+    auto operands = [&](int kt) __attribute__((always_inline)) {
+      d[kt & 1] = *reinterpret_cast<const float4*>(dec + kt * 16);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int row = min(4 * b4 + j, len - 1);
-          to[j] = (uint32_t)(p.dir ? len - 1 - row : row);
-#pragma unroll
-          for (int i = 0; i < NVT; ++i) {
-            xv[i][j] = to_f32(v[(at + to[j]) * rsV + min(cl + i * 16, V - 1)]);
-            os[i][j] = 0.f;
-          }
-          to[j] *= (uint32_t)rsK;
-        }
-        uint2 w[2][3][4];
-        auto load = [&](int kt) __attribute__((always_inline)) {
-          const int k0 = kt * 16 + 4 * gl;   // this lane's four rows
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            const bf16* base = (a == 0 ? q : a == 1 ? k : gk) + at * rsK;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              if constexpr (VEC) {
-                w[kt & 1][a][j] = *reinterpret_cast<const uint2*>(
-                    base + (to[j] + (uint32_t)max(min(k0, K - 4), 0)));
-              } else {
-                uint32_t x[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = base[to[j] + (uint32_t)min(k0 + e, K - 1)].u;
-                w[kt & 1][a][j] = make_uint2(x[0] | (x[1] << 16), x[2] | (x[3] << 16));
-              }
-            }
-          }
-        };
-        load(0);
-        auto tile = [&](auto tile_index) __attribute__((always_inline)) {
-          constexpr int kt = decltype(tile_index)::value;
-          if constexpr (kt + 1 < KT) load(kt + 1);
-          const int k0 = kt * 16 + 4 * gl;
-          if (seq_groups >> (kt / 4) & 1) {   // uniform
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const uint32_t m = 4 * b4 + j < len ? ~0u : 0u;
-              const uint2 wq = w[kt & 1][0][j], wk = w[kt & 1][1][j], wg = w[kt & 1][2][j];
-              const uint32_t qw[2] = {wq.x & m, wq.y & m}, kw[2] = {wk.x & m, wk.y & m};
-              const uint32_t gw[2] = {wg.x & m & gmask, wg.y & m & gmask};
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const bool in = k0 + r < K;
-                const float qx = r & 1 ? bf16_hi(qw[r >> 1]) : bf16_lo(qw[r >> 1]);
-                const float kx = r & 1 ? bf16_hi(kw[r >> 1]) : bf16_lo(kw[r >> 1]);
-                const float eg = gexp<bf16>(r & 1 ? bf16_hi(gw[r >> 1]) : bf16_lo(gw[r >> 1]));
-#pragma unroll
-                for (int i = 0; i < NVT; ++i) {
-                  const float x = m ? xv[i][j] : 0.f;
-                  S[i][kt][r] = fmaf(in ? kx : 0.f, x, S[i][kt][r] * (in ? eg : 1.f));
-                  os[i][j] = fmaf(in ? qx : 0.f, S[i][kt][r], os[i][j]);
-                }
-              }
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        each_tile(tile, std::make_integer_sequence<int, KT>{});
-#pragma unroll
-        for (int i = 0; i < NVT; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            os[i][j] += __shfl_xor(os[i][j], 16);
-            os[i][j] += __shfl_xor(os[i][j], 32);
-            if (g4 == b4) o[i][j] += os[i][j];
-          }
+      for (int i = 0; i < 3; ++i) {
+        x[kt & 1][i] = *reinterpret_cast<const s4_t*>(pq + i * QC * Lay::QP + kt * 16);
+        y[kt & 1][i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s4_t*)(pk + i * QC * Lay::KQ + kt * 16));
       }
+    };
+    operands(0);
+    // Step kt: tile kt's qa S' (the main products in NOM sums, the others in three)
+    // and ka^T v onto the state, with the next tile decayed to the chunk's middle and split
+    // meanwhile and the one after it read from LDS. The order of the products keeps those of
+    // one sum apart, and the VALU work sits between them (an MFMA occupies its own pipe for
+    // 16 cycles, a VALU operation 4).
+    f32x4 om[NVT][NOM], orest[NVT][3];
+    float4 ap[PW];
+    Split sp[NVT][2];
+    auto decay = [&](int kt) __attribute__((always_inline)) {   // S' of tile kt, split
+      const float4 dd = d[kt & 1];
+#pragma unroll
+      for (int i = 0; i < NVT; ++i) {
+        S[i][kt][0] *= dd.x;
+        S[i][kt][1] *= dd.y;
+        S[i][kt][2] *= dd.z;
+        S[i][kt][3] *= dd.w;
+        const float t[4] = {S[i][kt][0], S[i][kt][1], S[i][kt][2], S[i][kt][3]};
+        sp[i][kt & 1] = split3(t);
+      }
+    };
+    decay(0);
+    operands(1);
+#pragma unroll
+    for (int i = 0; i < NVT; ++i) {
+#pragma unroll
+      for (int j = 0; j < NOM; ++j) om[i][j] = zero4();
+#pragma unroll
+      for (int j = 0; j < 3; ++j) orest[i][j] = zero4();
+    }
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      const int c = kt & 1;
+      s4_t xx[3], yy[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        xx[j] = x[c][j];
+        yy[j] = y[c][j];
+      }
+#pragma unroll
+      for (int i = 0; i < NVT; ++i) {
+        const s4_t(&b)[3] = sp[i][c].p;
+        f32x4(&r)[3] = orest[i];
+        f32x4& t = S[i][kt];
+        om[i][kt % NOM] = mma16(xx[0], b[0], om[i][kt % NOM]);
+        t = mma16(yy[2], vv[i], t);
+        r[0] = mma16(xx[2], b[0], r[0]);
+        r[1] = mma16(xx[0], b[2], r[1]);
+        t = mma16(yy[1], vv[i], t);
+        r[2] = mma16(xx[1], b[1], r[2]);
+        r[0] = mma16(xx[1], b[0], r[0]);
+        t = mma16(yy[0], vv[i], t);
+        r[1] = mma16(xx[0], b[1], r[1]);
+      }
+      if (kt + 1 < KT) decay(kt + 1);
+      if (kt + 2 < KT) {
+        operands(kt + 2);
+      } else if (kt + 2 == KT) {
+#pragma unroll
+        for (int j = 0; j < PW; ++j)
+          ap[j] = *reinterpret_cast<const float4*>(
+              B + Lay::A + ((j * QC + li) * QTP + 4 * g4) * 4);
+      }
+#pragma unroll
+      for (int j = 0; j < 9 * NVT; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // one MFMA, four VALU
+        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // A v: row li, tokens 4 g4 ..; those after the row left out
+    const float4 am = PW == 1   ? ap[0]
+                      : PW == 2 ? add4(ap[0], ap[PW / 2])
+                                : add4(add4(ap[0], ap[1 % PW]), add4(ap[PW / 2], ap[PW - 1]));
+    const int after = li - 4 * g4;
+    const float aa[4] = {after >= 0 ? am.x : 0.f, after >= 1 ? am.y : 0.f,
+                         after >= 2 ? am.z : 0.f, after >= 3 ? am.w : 0.f};
+    const Split as = split3(aa);
+#pragma unroll
+    for (int i = 0; i < NVT; ++i) {
+      f32x4 u = zero4();
+#pragma unroll
+      for (int j = 2; j >= 0; --j) u = mma16(as.p[j], vv[i], u);
+      u += orest[i][0] + orest[i][1] + orest[i][2];
+#pragma unroll
+      for (int st = NOM / 2; st > 0; st /= 2)
+#pragma unroll
+        for (int j = 0; j < st; ++j) om[i][j] += om[i][j + st];
+      o[i] = om[i][0] + u;
+    }
+    owed = true;
+    {   // before the output's stores, which a wait for v behind them would wait for too
+      bool ok = take_v(n + 1);
+      if ((n & 7) == 7) ok = ok && state_ok();
+      request(n + 1, ok);
     }
     {
       float* ob = (float*)p.out + chunk_t0(n, len) * rsV + (long)hh * V;
@@ -655,6 +800,21 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
       }
     }
     __syncthreads();
+  }
+  if (__builtin_expect(left < NC, 0)) {
+    if (owed) mul_rows(qsm + (left & 1) * Lay::buf + Lay::ppost);
+    __syncthreads();   // the factors are read
+    float* X = reinterpret_cast<float*>(qsm);
+    int gl = g4, cl = w * NVT * 16 + li;
+    asm volatile("" : "+v"(gl), "+v"(cl));
+#pragma unroll
+    for (int i = 0; i < NVT; ++i)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) X[(kt * 16 + 4 * gl + r) * (CB + 4) + cl + i * 16] = S[i][kt][r];
+    rec_elements_consumer<KP, NVT>(p, qsm, left * QC, T, sN, ct, w, lane);
+    return;
   }
   if (owed) mul_rows(qsm + ((NC - 1) & 1) * Lay::buf + Lay::post);
   if (sN) {
@@ -676,7 +836,7 @@ namespace {
 
 template <int KP, int NVT, bool VEC>
 hipError_t launch_rec_chunk(const RecScanArgs& p, hipStream_t st) {
-  using Lay = QLayout<KP>;
+  using Lay = QLayout<KP, NVT>;
   static_assert(Lay::bytes <= 163840, "LDS budget exceeded");
   constexpr int CB = QCW * NVT * 16;
   const long blocks = (long)p.si.N * p.H * ((p.C + CB - 1) / CB);

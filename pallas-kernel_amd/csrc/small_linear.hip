@@ -53,6 +53,21 @@ __device__ __forceinline__ void split8(const float (&x)[8], Frag<bf16> (&f)[3]) 
   }
 }
 
+// w without its infinities and NaN (zeros in their place).
+__device__ __forceinline__ Frag<bf16> finite_part(const Frag<bf16>& w) {
+  const uint32_t x[4] = {w.d.x, w.d.y, w.d.z, w.d.w};
+  uint32_t y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t lo = (x[e] & 0x7f80u) != 0x7f80u ? 0xffffu : 0u;
+    const uint32_t hi = (x[e] & 0x7f800000u) != 0x7f800000u ? 0xffff0000u : 0u;
+    y[e] = x[e] & (lo | hi);
+  }
+  Frag<bf16> r;
+  r.d = make_uint4(y[0], y[1], y[2], y[3]);
+  return r;
+}
+
 }  // namespace
 
 // MT: 16-row tiles of x. TX: x's type.
@@ -109,6 +124,10 @@ __global__ __launch_bounds__(SLT) void small_linear_kernel(SmallLinearArgs p) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (k + 32 * u >= KW) break;   // uniform
+      // the lower parts of x are often 0: they leave out weights that are not finite, whose product
+      // with x's first part has x's sign (or is NaN for x = 0) already
+      Frag<bf16> wl;
+      if constexpr (sizeof(TX) == 4) wl = finite_part(wf[u]);
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         if constexpr (sizeof(TX) == 2) {
@@ -121,7 +140,8 @@ __global__ __launch_bounds__(SLT) void small_linear_kernel(SmallLinearArgs p) {
           __builtin_memcpy(x, &xf[u][t][0], 32);
           split8(x, f);
 #pragma unroll
-          for (int i = 2; i >= 0; --i) mma(acc[t], wf[u], f[i]);
+          for (int i = 2; i >= 1; --i) mma(acc[t], wl, f[i]);
+          mma(acc[t], wf[u], f[0]);
         }
       }
     }
@@ -159,7 +179,7 @@ __global__ __launch_bounds__(SLT) void small_linear_kernel(SmallLinearArgs p) {
 }
 
 // y[m][c] = max(log_sigmoid(bf16(x[m] . w[c] + bias[c])) inv_n, clamp): one thread per column,
-// its weight row (R <= 64 values) read once for LGM rows of x.
+// its weight row (R values, 16 in the layer) read once for LGM rows of x.
 constexpr int LGM = 4;
 __global__ __launch_bounds__(256) void low_rank_gate_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w, const bf16* __restrict__ bias,

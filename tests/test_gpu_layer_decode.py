@@ -52,6 +52,32 @@ def test_small_linear_scratch_values():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 20])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_small_linear_non_finite_weights(rows, value):
+    """A weight that is not finite meets x as in F.linear, also where x is a bfloat16 value (one
+    that needs no second and third part), 0 or infinite; other outputs keep their values."""
+    import torch.nn.functional as F
+
+    from tops.layers.gla import _small_linear
+
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, 512, generator=gen, device="cuda")
+    x[:, 3] = torch.tensor([1.5, 0.1, -2.0, 0.0, -0.3], device="cuda").repeat(4)[:rows]
+    x[-1, 300] = float("inf")
+    w = torch.randn(16, 512, generator=gen, device="cuda").bfloat16()
+    w[2, 3] = w[5, 300] = value
+    print(f"small linear, {value} in the weights, {rows} rows", flush=True)
+    y, ref = _small_linear(x, [w])[0], F.linear(x, w.float())
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(y), inf) and torch.equal(y[inf], ref[inf])
+    m = torch.isfinite(ref)
+    # float32 sums of 512 products, largest sums about 100
+    assert (y[m] - ref[m]).abs().max().item() <= 1e-4 if m.any() else True
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,n,clamp,bias", [(1, 256, None, True), (5, 300, -0.03, True),
                                                (128, 1024, None, False)])
 def test_low_rank_gate(rows, n, clamp, bias):

@@ -152,6 +152,33 @@ def test_few_row_route_takes_plain_projections_only():
 
 
 @pytest.mark.gpu
+def test_norm_gate_hooks_see_the_gate_in_its_own_dtype():
+    """A hooked or replaced gated norm gets the output gate as g_proj gives it, and the layer's
+    result with a hook that only looks is the one without."""
+    m = _layer().cuda()
+    x = torch.randn(2, 1, 256, generator=torch.Generator("cuda").manual_seed(1),
+                    device="cuda").bfloat16()
+    with torch.no_grad():
+        plain = m(x)[0]
+        seen = []
+        h = m.g_norm_swish_gate.register_forward_pre_hook(
+            lambda mod, a: seen.append([t.dtype for t in a]))
+        hooked = m(x)[0]
+        h.remove()
+        inner = m.g_norm_swish_gate
+
+        class Norm(torch.nn.Module):
+            def forward(self, o, g):
+                seen.append([o.dtype, g.dtype])
+                return inner(o, g)
+
+        m.g_norm_swish_gate = Norm()
+        replaced = m(x)[0]
+    assert seen == [[torch.float32, torch.bfloat16]] * 2
+    assert torch.equal(plain, hooked) and torch.equal(plain, replaced)
+
+
+@pytest.mark.gpu
 def test_few_row_route_leaves_tangents_and_global_hooks():
     import torch.autograd.forward_ad as fwd
     from torch.nn.modules.module import register_module_forward_hook

@@ -219,7 +219,7 @@ def _plain_linear(m, x):
         return False
     w = m._parameters.get("weight")
     return (w is not None and _plain_matrix(w, x.shape[-1], x.get_device())
-            and w.shape[0] % 4 == 0 and _unhooked(m))
+            and w.shape[0] > 0 and w.shape[0] % 4 == 0 and _unhooked(m))
 
 
 def _plain_matrix(w, features, device):
@@ -234,7 +234,7 @@ def _plain_gate(up, x):
         return False
     w, b = up._parameters.get("weight"), up._parameters.get("bias")
     return (w is not None and _plain_matrix(w, x.shape[-1], x.get_device())
-            and w.shape[1] % 8 == 0
+            and w.shape[1] % 8 == 0 and w.shape[1] <= 4096
             and (b is None or (type(b) is torch.nn.Parameter and b.dtype == torch.bfloat16
                                and b.shape == w.shape[:1] and b.is_contiguous()
                                and b.get_device() == w.get_device())))

@@ -151,6 +151,21 @@ def test_few_row_route_takes_plain_projections_only():
     assert not _plain_gate(m.gk_proj[1], low)
 
 
+def test_few_row_route_leaves_wide_ranks_and_empty_weights():
+    """Sizes that the entry points refuse keep the library path: a gate rank above 4096, a weight
+    without rows."""
+    from tops.layers.gla import Linear, _plain_gate, _plain_linear
+
+    low = torch.zeros(1, 1, 4104, dtype=torch.bfloat16)
+    assert _plain_gate(Linear(4096, 8, True, dtype=torch.bfloat16), low[..., :4096])
+    assert not _plain_gate(Linear(4104, 8, True, dtype=torch.bfloat16), low)
+    x = torch.zeros(1, 1, 256, dtype=torch.bfloat16)
+    lin = Linear(256, 4, dtype=torch.bfloat16)
+    assert _plain_linear(lin, x)
+    lin.weight = torch.nn.Parameter(lin.weight.detach()[:0])
+    assert not _plain_linear(lin, x)
+
+
 @pytest.mark.gpu
 def test_norm_gate_hooks_see_the_gate_in_its_own_dtype():
     """A hooked or replaced gated norm gets the output gate as g_proj gives it, and the layer's

@@ -83,6 +83,39 @@ def test_two_pass_states_match_the_scan(chunks, V, monkeypatch):
         assert (a - b).norm() < 2e-6 * b.norm(), name
 
 
+# packed sequences of more chunks than the state pass's two batches of 8, short ones between them
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,K,V", [(2, 68, 128), (1, 256, 320)])
+def test_packed_sequences_longer_than_the_batches(H, K, V):
+    import tops.ops.gla as G
+    from torch_ref import chunk_gla_torch
+
+    lengths = (64 * 17 + 1, 30, 64 * 9 - 5, 1, 64 * 25)
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    T, N = cu[-1], len(lengths)
+    gen = torch.Generator(device="cuda").manual_seed(K + V)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    print(f"chunk f32 packed K {K} V {V} lengths {lengths}", flush=True)
+    xs = [mk(1, T, H, K), mk(1, T, H, K), mk(1, T, H, V),
+          torch.nn.functional.logsigmoid(mk(1, T, H, K)) / 16, mk(N, H, K, V)]
+    do, dht = mk(1, T, H, V), mk(N, H, K, V)
+    ys = [x.double().requires_grad_() for x in xs]
+    parts = [chunk_gla_torch(*(t[:, a:b] for t in ys[:4]), h0=ys[4][i:i + 1])
+             for i, (a, b) in enumerate(zip(cu, cu[1:]))]
+    ref = [torch.cat([p[0] for p in parts], 1), torch.cat([p[1] for p in parts], 0)]
+    ref += torch.autograd.grad(ref, ys, [do.double(), dht.double()])
+    xs = [x.requires_grad_() for x in xs]
+    o, ht = G.chunk_gla(*xs[:4], initial_state=xs[4], output_final_state=True,
+                        cu_seqlens=torch.tensor(cu), chunk_size=64)
+    got = [o, ht, *torch.autograd.grad([o, ht], xs, [do, dht])]
+    # float32 sums of at most K + 64 products: 2-norm error about 1e-6
+    for name, a, b in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), got, ref):
+        err = (a.detach().double() - b).norm() / b.norm()
+        assert err < 4e-6, (name, float(err))
+
+
 def test_two_pass_workspace_part():
     """The decays are counted with bit 1 of `backward` alone, where the two-pass scan can run."""
     from tops import _lib

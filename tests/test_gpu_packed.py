@@ -98,3 +98,78 @@ def test_packed_segments_head_decay():
     refs = [on, hn, ref[0], ref[1], ref[2], ref[4]]
     for name, x, r in zip(["o", "ht", "dq", "dk", "dv", "dh0"], [o, ht, *grads], refs):
         check(name, to_np(x), r, "bf16")
+
+
+def _ref64(q, k, v, g, h0, cu):
+    """Every sequence alone, in float64 on the GPU (weak gates)."""
+    from torch_ref import chunk_gla_torch
+
+    parts = [chunk_gla_torch(*(t[:, a:b] for t in (q, k, v, g)), h0=h0[i:i + 1])
+             for i, (a, b) in enumerate(zip(cu, cu[1:]))]
+    return torch.cat([p[0] for p in parts], 1), torch.cat([p[1] for p in parts], 0)
+
+
+# 132 chunks: pieces of up to 13 where heads x V tiles are 32 (63 chunks in 5 pieces, 40 in 4, 24
+# in 2; short sequences between them), of up to 7 where they are 16
+LONG = [4000, 64, 1, 2500, 1500, 130]
+
+
+@pytest.mark.parametrize("shape", [(32, 64, 64), (16, 128, 128), (32, 72, 128), (8, 128, 256),
+                                   (4, 256, 512)], ids=lambda s: "H%dK%dV%d" % s)
+def test_packed_long_pieces(shape):
+    import tops.ops.gla as G
+    from tops import _lib
+
+    H, K, V = shape
+    cu, N = _cu(LONG), len(LONG)
+    T = cu[-1]
+    print(f"packed, long pieces {shape}", flush=True)
+    # the plan cuts: the workspace holds segment states
+    q1 = _lib.load().tops_gla_chunk_ws_bytes
+    assert q1(1, T, H, K, V, 64, N, 2, 1, 2) > q1(1, T, H, K, V, 64, N, 1, 1, 2)
+    gen = torch.Generator(device="cuda").manual_seed(H + K + V)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    xs = [mk(1, T, H, K).bfloat16(), mk(1, T, H, K).bfloat16(), mk(1, T, H, V).bfloat16(),
+          (torch.nn.functional.logsigmoid(mk(1, T, H, K)) / 16).bfloat16(), mk(N, H, K, V)]
+    do, dht = mk(1, T, H, V).bfloat16(), mk(N, H, K, V)
+    ys = [x.double().requires_grad_() for x in xs]
+    ref = _ref64(*ys, cu)
+    ref = [*ref, *torch.autograd.grad(list(ref), ys, [do.double(), dht.double()])]
+    xs = [x.requires_grad_() for x in xs]
+    o, ht = G.chunk_gla(*xs[:4], initial_state=xs[4], output_final_state=True,
+                        cu_seqlens=torch.tensor(cu), chunk_size=64)
+    got = [o, ht, *torch.autograd.grad([o, ht], xs, [do, dht])]
+    for name, x, r in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), got, ref):
+        err = (x.detach().double() - r).abs().max().item() / r.abs().max().item()
+        assert err <= 2e-2, (name, err)
+
+
+@pytest.mark.parametrize("shape", [(32, 64, 64), (8, 256, 256), (8, 256, 200)],
+                         ids=lambda s: "H%dK%dV%d" % s)
+def test_packed_long_pieces_head_decay(shape):
+    """Scalar gates; heads wider than 128 forward only (their backward takes another path)."""
+    import tops.ops.gla as G
+
+    H, K, V = shape
+    cu, N = _cu(LONG), len(LONG)
+    T = cu[-1]
+    print(f"packed, long pieces, per-head decay {shape}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(H + K + V)
+    mk = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    xs = [mk(1, T, H, K).bfloat16(), mk(1, T, H, K).bfloat16(), mk(1, T, H, V).bfloat16(),
+          mk(N, H, K, V)]
+    do, dht = mk(1, T, H, V).bfloat16(), mk(N, H, K, V)
+    gg = -torch.rand(1, 1, H, 1, generator=gen, device="cuda") / 8 - 1e-3
+    train = K <= 128
+    ys = [x.double().requires_grad_(train) for x in xs]
+    ref = list(_ref64(*ys[:3], gg.double().expand(1, T, H, K), ys[3], cu))
+    xs = [x.requires_grad_(train) for x in xs]
+    with torch.set_grad_enabled(train):
+        got = list(G.chunk_gla(*xs[:3], g_gamma=gg, initial_state=xs[3], output_final_state=True,
+                               cu_seqlens=torch.tensor(cu), chunk_size=64))
+    if train:
+        ref += torch.autograd.grad(ref, ys, [do.double(), dht.double()])
+        got += torch.autograd.grad(got, xs, [do, dht])
+    for name, x, r in zip(("o", "ht", "dq", "dk", "dv", "dh0"), got, ref):
+        err = (x.detach().double() - r).abs().max().item() / r.abs().max().item()
+        assert err <= 2e-2, (name, err)

@@ -418,10 +418,10 @@ class GatedLinearAttention(torch.nn.Module):
             # gate's second matrix and its activation in another; the output gate comes in
             # float32 where the float32 output of the recurrent kernel meets it in our own gated
             # norm and nothing else sees it
+            norm = self._modules.get("g_norm_swish_gate")
             f32_g = (self.use_output_gate and self.fuse_norm_and_gate
-                     and mode == "fused_recurrent"
-                     and type(self.g_norm_swish_gate) is FusedRMSNormGated
-                     and _unhooked(self.g_norm_swish_gate))
+                     and mode == "fused_recurrent" and type(norm) is FusedRMSNormGated
+                     and _unhooked(norm))
             ys = _small_linear(hidden_states, [m.weight for m in lins], (4,) if f32_g else ())
             q, k, v = ys[0], ys[1], ys[2]
             if self.use_output_gate:

@@ -16,13 +16,13 @@ Other legs (``--op``; not the headline, same JSON fields):
                     output's gradient a fixed random probe (flops / bytes: the GLA core's);
   simple_gla      : the C4 shape with a per-head constant log-decay (chunk_gla(g_gamma=...));
   decode_t1 / _t64: fused_recurrent_gla forward at a decode shape, B64 H16 K=V=128, T = 1 / 64:
-                    the recurrent kernel where HBM, not VALU, bounds it.
+                    the short scan, and the matrix-core scan over four chunks of 16 tokens.
 
 The default run (``--op chunk_gla``) first measures the other configurations, C2, C3 and C5,
 and the two decode shapes (the legs above, fixed warmup and step counts each), and reports
 them compactly under
 ``legs`` in the headline's line: ms per step, tokens/s, the step's HBM fraction, and the
-dominant kernel's roofline fraction (C2: fp32 VALU, with its HBM fraction beside it). They
+dominant kernel's roofline fraction. They
 run before the headline's warmup, so its timed steps also start at the GPU's steady clocks.
 
 The JSON line carries the driver's fields plus
@@ -35,11 +35,9 @@ The JSON line carries the driver's fields plus
                         stream) around every launch of it, against its binding roofline with
                         its algorithmic bytes (every input read once, every output written
                         once; the per-chunk state residual h / dh is
-                        implementation traffic, reported apart) -- or, for the recurrent
-                        kernel, its fp32 VALU lane-ops against the non-packed VALU peak with
-                        the HBM fraction beside it; ``traffic`` = its HBM bytes per launch
-                        from the copy-calibrated rocprofv3 FETCH_SIZE / WRITE_SIZE summary
-                        (profiles/hbm_traffic.json);
+                        implementation traffic, reported apart); ``traffic`` = its HBM
+                        bytes per launch from the copy-calibrated rocprofv3 FETCH_SIZE /
+                        WRITE_SIZE summary (profiles/hbm_traffic.json);
   kernels             : every timed kernel of the step (average ms, algorithmic GB/s);
   cpu_baseline        : the float32 numpy oracle (the reference's jnp algorithm restated) on
                         a sample of the workload's batch rows (every head at full length),
@@ -62,9 +60,6 @@ for _p in (ROOT, os.path.join(ROOT, "pallas-kernel_amd")):
 
 HBM_PEAK_GBS = 8000.0
 MFMA_BF16_PEAK = 2.517e15
-# fp32 VALU without packed-fp32 instructions (disabled in this build): 256 CUs x 4 SIMDs x 16
-# lanes per clock x 2.4 GHz lane-ops per second
-VALU_LANE_OPS_PEAK = 256 * 64 * 2.4e9
 BF = 2      # bf16 bytes
 F4 = 4      # fp32 bytes
 METRIC = "chunk_gla fwd+bwd tokens/s & % bf16 MFMA peak, B4 T8192 H16 K=V=128"
@@ -186,16 +181,14 @@ def leg_fused_recurrent(dev):
 
     tok = B * T * H
     nbytes = tok * (3 * K + V) * BF + tok * V * F4 + 2 * B * H * K * V * F4
-    lane_ops = 3 * tok * K * V   # decay multiply, rank-1 FMA, output FMA per state element
     return dict(
         metric="fused_recurrent_gla fwd tokens/s, B8 T2048 H4 K256 V512 (BASELINE configs[1])",
         tokens=B * T, flops=None, bytes=nbytes, step=step,
         config={"workload": "fused_recurrent_gla fwd + final state (BASELINE configs[1])",
                 "B": B, "T": T, "H": H, "K": K, "V": V, "h0": True, "o_dtype": "f32",
                 "global_batch": B, "seq_len": T, "parallelism": "single-gpu"},
-        kernels={"rec_scan_kernel": dict(slot=KT_REC_FWD, bytes=nbytes, residual=0,
-                                         lane_ops=lane_ops)},
-        bound="valu",
+        kernels={"rec_chunk_kernel": dict(slot=KT_REC_FWD, bytes=nbytes, residual=0)},
+        bound="hbm",
         cpu=dict(fn="fused_recurrent_fwd", shape=(B, T, H, K, V), seed=2, rows=B),
         stages=None,
     )
@@ -203,8 +196,8 @@ def leg_fused_recurrent(dev):
 
 def leg_recurrent_decode(dev, T):
     """fused_recurrent_gla forward at a decode shape: B64 H16 K=V=128,
-    T = 1 or 64 tokens, bf16 inputs, h0 and the final state fp32, o fp32 -- the shape where
-    the recurrent kernel is bound by HBM (state in and out) rather than by its VALU work."""
+    T = 1 or 64 tokens, bf16 inputs, h0 and the final state fp32, o fp32: the state in and out
+    is most of the bytes (T = 1: rec_short_kernel; T = 64: rec_chunk_kernel)."""
     import torch
 
     import tops.ops.gla as G
@@ -226,8 +219,8 @@ def leg_recurrent_decode(dev, T):
         config={"workload": f"fused_recurrent_gla fwd + final state, decode shape T={T}",
                 "B": B, "T": T, "H": H, "K": K, "V": V, "h0": True, "o_dtype": "f32",
                 "global_batch": B, "seq_len": T, "parallelism": "single-gpu"},
-        kernels={"rec_scan_kernel": dict(slot=KT_REC_FWD, bytes=nbytes, residual=0,
-                                         lane_ops=3 * tok * K * V)},
+        kernels={"rec_short_kernel" if T == 1 else "rec_chunk_kernel":
+                 dict(slot=KT_REC_FWD, bytes=nbytes, residual=0)},
         bound="hbm", cpu=None, stages=None,
     )
 
@@ -519,25 +512,15 @@ def _report(leg, ms, kms, op):
     elif kernels:
         dom = max(kernels, key=lambda n: kernels[n]["ms"])
         d, kd = kernels[dom], leg["kernels"][dom]
-        if leg["bound"] == "valu":
-            achieved = kd["lane_ops"] / (d["ms"] * 1e-3) / 1e12
-            peak = VALU_LANE_OPS_PEAK / 1e12
-            out["roofline"] = {
-                "bound": "valu", "kernel": dom, "achieved": round(achieved, 2),
-                "peak": round(peak, 2), "unit": "T fp32 lane-ops/s (non-packed)",
-                "frac": round(achieved / peak, 4),
-                "traffic": _measured_traffic(dom, op),
-                "hbm_achieved_gbs": d["gbs"], "hbm_frac": round(d["gbs"] / HBM_PEAK_GBS, 4)}
-        else:
-            res = int(kd.get("residual", 0))
-            out["roofline"] = {
-                "bound": "hbm", "kernel": dom, "achieved": d["gbs"], "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(d["gbs"] / HBM_PEAK_GBS, 4),
-                "traffic": _measured_traffic(dom, op),
-                "residual_bytes": res,
-                # the same launch with its per-chunk state traffic counted as well
-                "frac_with_residual": round((kd["bytes"] + res) / (d["ms"] * 1e-3) / 1e9 /
-                                            HBM_PEAK_GBS, 4)}
+        res = int(kd.get("residual", 0))
+        out["roofline"] = {
+            "bound": "hbm", "kernel": dom, "achieved": d["gbs"], "peak": HBM_PEAK_GBS,
+            "unit": "GB/s", "frac": round(d["gbs"] / HBM_PEAK_GBS, 4),
+            "traffic": _measured_traffic(dom, op),
+            "residual_bytes": res,
+            # the same launch with its per-chunk state traffic counted as well
+            "frac_with_residual": round((kd["bytes"] + res) / (d["ms"] * 1e-3) / 1e9 /
+                                        HBM_PEAK_GBS, 4)}
     if kernels:
         out["kernels"] = kernels
     return out
@@ -563,8 +546,6 @@ def _side_leg(leg, op, warmup, steps, timing):
     rf = r.get("roofline")
     if rf:
         d["roofline"] = {"kernel": rf["kernel"], "bound": rf["bound"], "frac": rf["frac"]}
-        if rf["bound"] == "valu":
-            d["roofline"]["hbm_frac"] = rf["hbm_frac"]
         if rf.get("residual_bytes"):
             d["roofline"]["frac_with_residual"] = rf["frac_with_residual"]
         if rf["bound"] == "hbm" and rf["unit"] == "GB/s" and rf["kernel"] in r.get("kernels", {}):

@@ -138,7 +138,10 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
  *    == 0: the chunks' decays (f32 [NC, H, K]) of the two-pass state scan, which forms all
  *    chunks' updates at once.
  * A shorter workspace drops the later parts (varlen: the segments and the gating together,
- * below the varlen = 2 size). The per-chunk states h_ws that the forward
+ * below the varlen = 2 size). The largest piece of a packed sequence follows from the call's
+ * chunks and heads together, as a fixed-length call's segments follow from its batch: the same
+ * sequence beside others may be cut elsewhere, and its sums then round differently (within the
+ * bf16 operands' rounding). Without the segment part it is one segment whatever is beside it. The per-chunk states h_ws that the forward
  * stores for flagged pairs are not meaningful (the backward recomputes those pairs).
  * No counterpart in the reference (its scans are sequential grid axes, chunk_h.py:252-271).
  */

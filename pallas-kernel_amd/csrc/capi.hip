@@ -158,12 +158,12 @@ struct WsLayout {
   long flags_end() const { return off_flags + flags; }
 };
 
-// `packed`: varlen sequences with the segment and gating parts.
 // Whether the two-pass state scan can take the sizes (tops::f32_scan_supported has the rest).
 bool two_pass_sizes(int dtype, int C, int64_t K, int64_t V) {
   return dtype == TOPS_GLA_F32 && C == 64 && K <= 384 && V % 4 == 0;
 }
 
+// `packed`: varlen sequences with the segment and gating parts.
 WsLayout ws_layout(int N, int T, int H, int K, int V, int C, bool varlen, bool head,
                    bool backward, bool packed, bool two_pass) {
   WsLayout w;

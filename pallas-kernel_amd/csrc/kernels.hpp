@@ -69,7 +69,7 @@ struct BwdArgs {
   const void* h;        // [NC, H, K, V] forward states (chunk start)
   const void* dh;       // [NC, H, K, V] state gradients (chunk end)
   void *dq, *dk, *dv, *dg;
-  // per-chunk gating workspace (head_gate_kernel: bf16, chunk 64, fixed-length; nullable):
+  // per-chunk gating workspace (head_gate_kernel: bf16, chunk 64; nullable):
   // the dv kernel then streams gated k, A and the column factors instead of recomputing
   // them in every V tile's block
   const void* gate_ws;
@@ -320,7 +320,7 @@ struct HeadFwdArgs {
   const float* h0;        // nullable
   void* o;
   void* h_out;            // [NC, H, K, V] bf16 (nullable)
-  void* gate_ws;          // per-chunk gating workspace of wide heads (nullable; fixed length)
+  void* gate_ws;          // per-chunk gating workspace of wide heads (nullable)
   float* ht;              // nullable
   float* seg_state;       // segmented only
   float* seg_gam;

@@ -918,7 +918,7 @@ bool short_scan(const RecScanArgs& p, int dtype) {
 // The matrix-core scan from kChunkScanT tokens a sequence (packed sequences: on average), whose
 // time goes by the 16 tokens begun, the VALU scans' by the token. Measured with the chip full, VALU
 // and matrix-core scan: B64 H16 K=V=128 60 and 65 us at T = 24, 73 and 66 at 32, 98 and 79 at 48,
-// 128 and 92 at 64; B64 H4 K256 V512 147 and 129, 170 and 134, 229 and 163, 286 and 193. So with K
+// 128 and 92 at 64 (98 to 102 with inputs that no earlier call left in the caches); B64 H4 K256 V512 147 and 129, 170 and 134, 229 and 163, 286 and 193. So with K
 // up to 128 the VALU scans keep T below 28 and 33 to 40 there, where the last 16 tokens are mostly
 // missing. With K up to 64 a block's one producer wave serves 64 value columns unless 128 of them
 // fill the chip: B24 H8 K64 V128 T100 38 and 42 us, B64 H16 K=V=64 T64 47 and 52 us, so the VALU

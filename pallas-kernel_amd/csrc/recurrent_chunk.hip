@@ -20,8 +20,9 @@
 // registers: a wave holds all K rows of 16 (or 32) columns as accumulators (rows 4g + r,
 // column l & 15 in lane l = 16 g + column), which is also the B operand of an MFMA over those
 // rows, so qa S' and ka^T v need no transposition and no exchange between waves. Measured: B8
-// T2048 H4 K256 V512 951 -> 461 us, B64 T64 H16 K=V=128 131 -> 92 us, B3 T1000 H16 K=V=64
-// 317 -> 155 us (the VALU scan and this kernel).
+// T2048 H4 K256 V512 951 -> 458 us, B64 T64 H16 K=V=128 131 -> 101 us (92 with inputs left in
+// the caches), B3 T1000 H16 K=V=64 317 -> 157 us (the VALU scan and this kernel). VALU busy 69 %,
+// the MFMA pipe 31 % in the first.
 //
 // Block = (sequence, head, 64 or 128 columns): four consumer waves, each 16 or 32 columns,
 // and KP / 64 producer waves. While the consumers work on tokens 16 n .., the producers make

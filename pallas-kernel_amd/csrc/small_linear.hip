@@ -9,7 +9,7 @@
 // of one weight and all M rows of x; its eight waves split K, so that a wave's loads are issued
 // before its first product, and their sums meet in LDS. Measured, M = 32, hidden 2048: 15 us for
 // the five projections in one launch (five hipBLASLt calls: 43 us on the GPU and about 20 us
-// each on the host, which is what a decode step waits for), 13 us for the output projection of
+// each on the host, which is what a decode step waits for), 16 us for the output projection of
 // float32 rows (a float32 GEMM and the weight's conversion: 19 us); the layer's decode step at
 // batch 32 256 -> 123 us (85 us with a cheaper host path).
 //

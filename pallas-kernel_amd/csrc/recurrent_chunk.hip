@@ -33,11 +33,15 @@
 // finite, a half's decay above 8 or NaN (the first row's gate is in the decays alone, not in an
 // operand), a v above 2^20 or not finite, a state above 2^56 or not finite: the block takes the
 // sequence from that chunk on as the recurrence is written, on the VALU (below), so that
-// non-finite values stay where the recurrence puts them and no gate costs more than the VALU scan
-// of recurrent.hip. Measured with gates near -8, that scan and this kernel: B8 T2048 H4 K256 V512
-// 950 and 921 us, B8 T2048 H16 K=V=128 666 and 561, B3 T1000 H16 K=V=64 313 and 198; only the
-// start weighs on short sequences (B64 T64 H16 K=V=128 124 and 159). Taken token by token from
-// the registers of the matrix path instead, a chunk cost 15 to 37 us in place of 3.6.
+// non-finite values stay where the recurrence puts them; after 8 chunks, then 32 and so on, it
+// comes back to the matrix cores. Measured, the VALU scan of recurrent.hip and this kernel, gates
+// near -8 / one gate of -60 in a sequence: B8 T2048 H4 K256 V512 950 and 943 / 491 us, B8 T2048
+// H16 K=V=128 666 and 586 / 377, B3 T1000 H16 K=V=64 313 and 205 / 160; only the start weighs on
+// short sequences (B64 T64 H16 K=V=128 124 and 159 / 145). Without a way back the dense gates took
+// 921, 561, 198 and 159 us, a single one up to as much; token by token from the registers of the
+// matrix path a chunk cost 15 to 37 us in place of 3.6.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -54,6 +58,7 @@ constexpr float kDecayWeight = 1.5845633e29f;       // 2^97
 constexpr uint32_t kValueMaxBits = 0x4980u;         // 2^20 as bf16
 
 constexpr int RTB = 8;             // tokens per stage of the element-wise phase
+constexpr int kSpan = 8;           // chunks of its first stretch; each is four times the one before
 
 template <int KP, int NVT>
 struct QLayout {   // byte offsets of one buffer
@@ -147,7 +152,8 @@ __device__ __forceinline__ void mma_split(const s4_t (&a)[3], const s4_t (&b)[3]
 
 }  // namespace
 
-// The element-wise phase: the rest of a sequence from token t0 on as the recurrence is written.
+// The element-wise phase: tokens t0 .. t1 - 1 as the recurrence is written, from and (`again`) to a
+// state in LDS.
 // The producers stage RTB tokens' k, so q, e^g and v as floats and write the outputs of the stage
 // before; a consumer wave has KP / 4 state rows of all CB columns, a lane KP / 16 rows of four
 // (eight) columns, so that an operand read from LDS meets four products, and its sums over the
@@ -155,10 +161,12 @@ __device__ __forceinline__ void mma_split(const s4_t (&a)[3], const s4_t (&b)[3]
 // barrier a stage, a token's LDS reads under the products of the one before (944 -> 921 us at B8
 // T2048 H4 K256 V512).
 template <int KP, int NVT, bool VEC>
-__device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsigned char* qsm, int t0, int T,
-                                      int bos, int eos, int hh, int ct, int pw, int lane) {
+__device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsigned char* qsm,
+                                                      int t0, int t1, bool again, int bos,
+                                                      int eos, int hh, int ct, int pw, int lane) {
   using Lay = QLayout<KP, NVT>;
   constexpr int PW = Lay::PW, CB = Lay::CB, NV = RTB * CB / (PW * 64);
+  asm volatile("" : "+v"(lane));   // nothing that depends on it is kept over the matrix path
   const int H = p.H, K = p.R, V = p.C;
   const long rsK = (long)H * K, rsV = (long)H * V;
   const bf16* q = (const bf16*)p.o + (long)hh * K;
@@ -166,14 +174,14 @@ __device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsi
   const bf16* gk = (const bf16*)(p.ga ? p.ga : p.a) + (long)hh * K;
   const bf16* v = (const bf16*)p.b + (long)hh * V;
   const uint32_t gmask = p.ga ? ~0u : 0u;
-  const int NS = (T - t0 + RTB - 1) / RTB, c0 = pw * 64 + 4 * (lane & 15);
-  auto tok = [&](int t) { return (long)(p.dir ? eos - 1 - t : bos + t); };   // t < T
+  const int NS = (t1 - t0 + RTB - 1) / RTB, c0 = pw * 64 + 4 * (lane & 15);
+  auto tok = [&](int t) { return (long)(p.dir ? eos - 1 - t : bos + t); };
   uint2 raw[2][3];      // two tokens of four key columns
   uint32_t rv[NV];      // values: token and column of index (i PW + pw) 64 + lane
   auto load = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const long at = tok(min(t0 + s * RTB + 2 * (lane >> 4) + u, T - 1)) * rsK;
+      const long at = tok(min(t0 + s * RTB + 2 * (lane >> 4) + u, t1 - 1)) * rsK;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
         const bf16* base = (a == 0 ? q : a == 1 ? k : gk) + at;
@@ -190,7 +198,7 @@ __device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsi
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int x = (i * PW + pw) * 64 + lane;
-      rv[i] = v[tok(min(t0 + s * RTB + x / CB, T - 1)) * rsV + min(ct * CB + x % CB, V - 1)].u;
+      rv[i] = v[tok(min(t0 + s * RTB + x / CB, t1 - 1)) * rsV + min(ct * CB + x % CB, V - 1)].u;
     }
   };
   auto store = [&](int s) __attribute__((always_inline)) {   // tokens past the end are not read
@@ -225,7 +233,7 @@ __device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsi
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int x = (i * PW + pw) * 64 + lane, t = t0 + s * RTB + x / CB, c = ct * CB + x % CB;
-      if (t < T && c < V)
+      if (t < t1 && c < V)
         ((float*)p.out)[tok(t) * rsV + (long)hh * V + c] =
             (O[x] + O[RTB * CB + x]) + (O[2 * RTB * CB + x] + O[3 * RTB * CB + x]);
     }
@@ -244,16 +252,23 @@ __device__ __forceinline__ void rec_elements_producer(const RecScanArgs& p, unsi
   }
   __syncthreads();
   output(NS - 1);
+  if (again) {
+    __syncthreads();   // the sums are read
+    __syncthreads();   // the state is in LDS
+    __syncthreads();   // and out of it
+  }
 }
 
 template <int KP, int NVT>
-__device__ __forceinline__ void rec_elements_consumer(const RecScanArgs& p, unsigned char* qsm, int t0, int T,
-                                      float* sN, int ct, int w, int lane) {
+__device__ __forceinline__ void rec_elements_consumer(const RecScanArgs& p, unsigned char* qsm,
+                                                      int t0, int t1, bool again, float* sN,
+                                                      int ct, int w, int lane) {
   using Lay = QLayout<KP, NVT>;
   constexpr int CB = Lay::CB, R = KP / 16;
   const int K = p.R, V = p.C;
+  asm volatile("" : "+v"(lane));   // as above
   const int cg = 4 * (lane & 15), r0 = (w * 4 + (lane >> 4)) * R;
-  const int NS = (T - t0 + RTB - 1) / RTB;
+  const int NS = (t1 - t0 + RTB - 1) / RTB;
   float S[R][NVT][4];
   __syncthreads();   // the state is in LDS
   {
@@ -274,7 +289,7 @@ __device__ __forceinline__ void rec_elements_consumer(const RecScanArgs& p, unsi
     __syncthreads();
     const float* B = reinterpret_cast<const float*>(qsm + (s & 1) * Lay::stage);
     float* O = reinterpret_cast<float*>(qsm + 2 * Lay::stage + (s & 1) * Lay::sums) + w * RTB * CB;
-    const int nt = min(RTB, T - t0 - s * RTB);
+    const int nt = min(RTB, t1 - t0 - s * RTB);
     // a token's operands, read while the one before it is computed
     struct Step {
       float4 b[NVT], a[R / 4], o[R / 4], e[R / 4];
@@ -340,6 +355,18 @@ __device__ __forceinline__ void rec_elements_consumer(const RecScanArgs& p, unsi
     }
   }
   __syncthreads();
+  if (again) {
+    __syncthreads();   // the sums are read
+    float* X = reinterpret_cast<float*>(qsm);
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int u = 0; u < NVT; ++u)
+        *reinterpret_cast<float4*>(X + (r0 + j) * (CB + 4) + 64 * u + cg) =
+            make_float4(S[j][u][0], S[j][u][1], S[j][u][2], S[j][u][3]);
+    __syncthreads();   // the state is in LDS
+    return;
+  }
   if (sN) {
     const bool whole = V % 4 == 0 && ((uintptr_t)sN & 15) == 0;
 #pragma unroll
@@ -411,10 +438,15 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
     for (int j = 0; j < PW; ++j) x |= f[j];
     return __builtin_amdgcn_readfirstlane(x) != 0;
   };
-  int left = NC;   // the first chunk of the element-wise phase
+  // The matrix path from chunk `start` to the end or to chunk `left`, from there the element-wise
+  // phase for `span` chunks, and again.
+  int start = 0, span = kSpan, left = NC;
 
   if (w >= QCW) {
     // ---- producers: lane = 4 key columns (lane & 15) x 4 rows (lane >> 4) ----
+    // a single producer wave is what the block waits for (B3 T1000 H16 K=V=64 156 -> 149 us; four
+    // of them take the consumers' slots: B8 T2048 H4 K256 V512 462 -> 522)
+    if constexpr (PW == 1 && NVT == 1) __builtin_amdgcn_s_setprio(1);
     const int pw = w - QCW, rg = lane >> 4, c0 = pw * 64 + 4 * (lane & 15);
     const uint32_t cv = (uint32_t)max(min(c0, K - 4), 0);
     uint32_t cm[2];   // masks of the columns past the head
@@ -450,129 +482,135 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
         Rg[u] = ld4(gk + at, off);
       }
     };
-    // per column: the previous chunk's rows 8..15 in sum and as a factor (groups 2, 3)
-    float lsum[4], lpost[4];
+    for (;;) {
+      // per column: the previous chunk's rows 8..15 in sum and as a factor (groups 2, 3)
+      float lsum[4], lpost[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      lsum[e] = 0.f;
-      lpost[e] = 1.f;
-    }
-    if (NC > 0) issue(0);
-    for (int n = 0; n < NC; ++n) {
-      {
-        unsigned char* B = qsm + (n & 1) * Lay::buf;
-        const int len = T - n * QC;
-        float xq[4][4], xk[4][4], xg[4][4];   // [row][column]
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t m = row_of(u) < len ? ~0u : 0u, m0 = m & cm[0], m1 = m & cm[1];
-          const uint32_t wq[2] = {Rq[u].x & m0, Rq[u].y & m1};
-          const uint32_t wk[2] = {Rk[u].x & m0, Rk[u].y & m1};
-          const uint32_t wg[2] = {Rg[u].x & m0 & gmask, Rg[u].y & m1 & gmask};
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            xq[u][2 * e] = bf16_lo(wq[e]);
-            xq[u][2 * e + 1] = bf16_hi(wq[e]);
-            xk[u][2 * e] = bf16_lo(wk[e]);
-            xk[u][2 * e + 1] = bf16_hi(wk[e]);
-            xg[u][2 * e] = bf16_lo(wg[e]);
-            xg[u][2 * e + 1] = bf16_hi(wg[e]);
-          }
-        }
-        issue(n + 1);
-        float dout[4];
-        // sum of the operands' squares and four decays x 2^97: above kOperandMax^2 where an operand
-        // is too large or the decays sum to more than 8
-        float sq = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float tot = (xg[0][e] + xg[1][e]) + (xg[2][e] + xg[3][e]);
-          // permlane16_swap of x with itself: [0] holds the even group of the lane's pair of
-          // groups, [1] the odd one
-          const auto pr = __builtin_amdgcn_permlane16_swap(__float_as_uint(tot),
-                                                           __float_as_uint(tot), false, false);
-          const float even = __uint_as_float(pr[0]), odd = __uint_as_float(pr[1]);
-          const float half = even + odd;   // groups 0, 1: rows 0..7; groups 2, 3: rows 8..15
-          // the sum from the middle to this group's inner edge: groups 1 and 2 start there
-          float run = rg == 0 ? odd : rg == 3 ? even : 0.f;
+      for (int e = 0; e < 4; ++e) {
+        lsum[e] = 0.f;
+        lpost[e] = 1.f;
+      }
+      if (NC > 0) issue(start);
+      for (int n = start; n < NC; ++n) {
+        {
+          unsigned char* B = qsm + (n & 1) * Lay::buf;
+          const int len = T - n * QC;
+          float xq[4][4], xk[4][4], xg[4][4];   // [row][column]
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const float nx = run + xg[u][e];
-            const float sum = rg < 2 ? -run : nx;   // E: rows before the middle exclude their own
-            run = nx;
-            float f, fi;
-            exp_pair(sum, f, fi);
-            xq[u][e] *= f;
-            xk[u][e] *= fi;
-            sq = fmaf(xq[u][e], xq[u][e], sq);
-            sq = fmaf(xk[u][e], xk[u][e], sq);
+            const uint32_t m = row_of(u) < len ? ~0u : 0u, m0 = m & cm[0], m1 = m & cm[1];
+            const uint32_t wq[2] = {Rq[u].x & m0, Rq[u].y & m1};
+            const uint32_t wk[2] = {Rk[u].x & m0, Rk[u].y & m1};
+            const uint32_t wg[2] = {Rg[u].x & m0 & gmask, Rg[u].y & m1 & gmask};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              xq[u][2 * e] = bf16_lo(wq[e]);
+              xq[u][2 * e + 1] = bf16_hi(wq[e]);
+              xk[u][2 * e] = bf16_lo(wk[e]);
+              xk[u][2 * e + 1] = bf16_hi(wk[e]);
+              xg[u][2 * e] = bf16_lo(wg[e]);
+              xg[u][2 * e + 1] = bf16_hi(wg[e]);
+            }
           }
-          // decays: groups 0, 1 make pre and (with the previous chunk's rows 8..15, held by
-          // groups 2, 3) dec; groups 2, 3 post
-          const auto ps = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[e]),
-                                                           __float_as_uint(lsum[e]), false,
-                                                           false);
-          const float prev = __uint_as_float(ps[1]);   // the upper half's value
-          const float d = exp_one(rg == 0 ? half + prev : half);
-          sq = fmaf(d, kDecayWeight, sq);
-          dout[e] = rg == 3 ? lpost[e] : d;
-          lpost[e] = d;
-          lsum[e] = half;
-        }
-        const bool good = __ballot(sq <= kOperandMax * kOperandMax) == ~0ull;
-        if (lane == 0) reinterpret_cast<int*>(B + Lay::flag)[pw] = good ? 0 : 1;
-        *reinterpret_cast<float4*>(B + Lay::dec + (rg * KP + c0) * 4) =
-            make_float4(dout[0], dout[1], dout[2], dout[3]);
-        bf16* sQ = reinterpret_cast<bf16*>(B + Lay::qa);
-        bf16* sK = reinterpret_cast<bf16*>(B + Lay::ka);
+          issue(n + 1);
+          float dout[4];
+          // sum of the operands' squares and four decays x 2^97: above kOperandMax^2 where an
+          // operand is too large or the decays sum to more than 8
+          float sq = 0.f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const Split x = split3(xq[u]), y = split3(xk[u]);
+          for (int e = 0; e < 4; ++e) {
+            const float tot = (xg[0][e] + xg[1][e]) + (xg[2][e] + xg[3][e]);
+            // permlane16_swap of x with itself: [0] holds the even group of the lane's pair of
+            // groups, [1] the odd one
+            const auto pr = __builtin_amdgcn_permlane16_swap(__float_as_uint(tot),
+                                                             __float_as_uint(tot), false, false);
+            const float even = __uint_as_float(pr[0]), odd = __uint_as_float(pr[1]);
+            const float half = even + odd;   // groups 0, 1: rows 0..7; groups 2, 3: rows 8..15
+            // the sum from the middle to this group's inner edge: groups 1 and 2 start there
+            float run = rg == 0 ? odd : rg == 3 ? even : 0.f;
 #pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            *reinterpret_cast<s4_t*>(sQ + (i * QC + row_of(u)) * Lay::QP + c0) = x.p[i];
-            *reinterpret_cast<s4_t*>(sK + (i * QC + row_of(u)) * Lay::KQ + c0) = y.p[i];
+            for (int u = 0; u < 4; ++u) {
+              const float nx = run + xg[u][e];
+              const float sum = rg < 2 ? -run : nx;   // E: rows before the middle exclude their own
+              run = nx;
+              float f, fi;
+              exp_pair(sum, f, fi);
+              xq[u][e] *= f;
+              xk[u][e] *= fi;
+              sq = fmaf(xq[u][e], xq[u][e], sq);
+              sq = fmaf(xk[u][e], xk[u][e], sq);
+            }
+            // decays: groups 0, 1 make pre and (with the previous chunk's rows 8..15, held by
+            // groups 2, 3) dec; groups 2, 3 post
+            const auto ps = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[e]),
+                                                             __float_as_uint(lsum[e]), false,
+                                                             false);
+            const float prev = __uint_as_float(ps[1]);   // the upper half's value
+            const float d = exp_one(rg == 0 ? half + prev : half);
+            sq = fmaf(d, kDecayWeight, sq);
+            dout[e] = rg == 3 ? lpost[e] : d;
+            lpost[e] = d;
+            lsum[e] = half;
           }
-        }
-        // A over this wave's 64 columns: its own LDS rows, in order behind the writes
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        f32x4 am[2], ar[3];
-        am[0] = am[1] = ar[0] = ar[1] = ar[2] = zero4();
+          const bool good = __ballot(sq <= kOperandMax * kOperandMax) == ~0ull;
+          if (lane == 0) reinterpret_cast<int*>(B + Lay::flag)[pw] = good ? 0 : 1;
+          *reinterpret_cast<float4*>(B + Lay::dec + (rg * KP + c0) * 4) =
+              make_float4(dout[0], dout[1], dout[2], dout[3]);
+          bf16* sQ = reinterpret_cast<bf16*>(B + Lay::qa);
+          bf16* sK = reinterpret_cast<bf16*>(B + Lay::ka);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int kb = pw * 64 + t * 16 + 4 * (lane >> 4), li = lane & 15;
-          s4_t x[3], y[3];
+          for (int u = 0; u < 4; ++u) {
+            const Split x = split3(xq[u]), y = split3(xk[u]);
 #pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            x[i] = *reinterpret_cast<const s4_t*>(sQ + (i * QC + li) * Lay::QP + kb);
-            y[i] = *reinterpret_cast<const s4_t*>(sK + (i * QC + li) * Lay::KQ + kb);
+            for (int i = 0; i < 3; ++i) {
+              *reinterpret_cast<s4_t*>(sQ + (i * QC + row_of(u)) * Lay::QP + c0) = x.p[i];
+              *reinterpret_cast<s4_t*>(sK + (i * QC + row_of(u)) * Lay::KQ + c0) = y.p[i];
+            }
           }
-          mma_split(x, y, am[t & 1], ar);
-        }
-        am[0] = (am[0] + am[1]) + (ar[0] + ar[1] + ar[2]);
+          // A over this wave's 64 columns: its own LDS rows, in order behind the writes
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          f32x4 am[2], ar[3];
+          am[0] = am[1] = ar[0] = ar[1] = ar[2] = zero4();
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          reinterpret_cast<float*>(B + Lay::A)[(pw * QC + 4 * (lane >> 4) + r) * QTP +
-                                               (lane & 15)] = am[0][r];
+          for (int t = 0; t < 4; ++t) {
+            const int kb = pw * 64 + t * 16 + 4 * (lane >> 4), li = lane & 15;
+            s4_t x[3], y[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              x[i] = *reinterpret_cast<const s4_t*>(sQ + (i * QC + li) * Lay::QP + kb);
+              y[i] = *reinterpret_cast<const s4_t*>(sK + (i * QC + li) * Lay::KQ + kb);
+            }
+            mma_split(x, y, am[t & 1], ar);
+          }
+          am[0] = (am[0] + am[1]) + (ar[0] + ar[1] + ar[2]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            reinterpret_cast<float*>(B + Lay::A)[(pw * QC + 4 * (lane >> 4) + r) * QTP +
+                                                 (lane & 15)] = am[0][r];
+        }
+        __syncthreads();
+        if (__builtin_expect(leaves(n), 0)) {
+          left = n;
+          break;
+        }
       }
-      __syncthreads();
-      if (__builtin_expect(leaves(n), 0)) {
-        left = n;
-        break;
-      }
-    }
-    if (left < NC) {
-      rec_elements_producer<KP, NVT, VEC>(p, qsm, left * QC, T, bos, eos, hh, ct, pw, lane);
-      return;
+      if (left == NC) break;
+      const int end = min(left + span, NC);
+      rec_elements_producer<KP, NVT, VEC>(p, qsm, left * QC, min(T, end * QC), end < NC, bos, eos,
+                                          hh, ct, pw, lane);
+      if (end == NC) return;
+      start = end;
+      span *= 4;
+      left = NC;
     }
     __syncthreads();
     return;
   }
 
   // ---- consumers: all K rows of NVT 16-column tiles ----
-  const int g4 = lane >> 4, li = lane & 15;
-  const int cb = ct * CB + w * NVT * 16 + li;   // this lane's column of tile 0
+  int g4 = lane >> 4, li = lane & 15;
+  int cb = ct * CB + w * NVT * 16 + li;   // this lane's column of tile 0
   // a lane's state element (kt, r): uniform base plus a 32-bit offset
   const long sbase = ((long)seq * H + hh) * K * V;
   const float* __restrict__ s0 = p.s0 ? p.s0 + sbase : nullptr;
@@ -583,12 +621,26 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kk = kt * 16 + 4 * g4 + r, c = cb + i * 16;
-        const float x = s0 ? s0[(uint32_t)min(kk, K - 1) * (uint32_t)V + (uint32_t)min(c, V - 1)]
-                           : 0.f;
-        S[i][kt][r] = kk < K && c < V ? x : 0.f;
-      }
+      for (int r = 0; r < 4; ++r)
+        S[i][kt][r] = 0.f;
+  if (s0) {   // one run of loads, masked when all are under way
+#pragma unroll
+    for (int i = 0; i < NVT; ++i)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[i][kt][r] = s0[(uint32_t)min(kt * 16 + 4 * g4 + r, K - 1) * (uint32_t)V +
+                           (uint32_t)min(cb + i * 16, V - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NVT; ++i)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[i][kt][r] = kt * 16 + 4 * g4 + r < K && cb + i * 16 < V ? S[i][kt][r] : 0.f;
+  }
   // A state that is not finite (or large enough to leave the range within a few chunks) is left to
   // the recurrence as written: split into bf16 it would turn to NaN. Looked at before the first
   // chunk and after every eighth. Between, decays of at most 8 a half and 16 products of 2^50 2^20
@@ -604,9 +656,12 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
     return s_ok;
   };
   __builtin_amdgcn_sched_barrier(0);
-  uint32_t Rv[NVT][4], vo[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) vo[m] = (uint32_t)(4 * g4 + m) * (uint32_t)rsV;
+  // the next chunk's v, as loaded: extended at the load, every load is waited for (two tiles a
+  // wave, B64 T64 H16 K=V=128: 90 against 123 us). With two producers and one tile that wait, in
+  // the middle of the chunk, leaves issue slots to the producers, which the block waits for (B8
+  // T2048 H16 K=V=128 372 -> 357 us).
+  std::conditional_t<PW == 2 && NVT == 1, uint32_t, uint16_t> Rv[NVT][4];
+  uint32_t vo[4];
   auto issue_v = [&](int n) __attribute__((always_inline)) {
     n = min(n, NC - 1);
     const int len = min(QC, T - n * QC);
@@ -645,7 +700,7 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
       uint32_t x[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        x[m] = 4 * g4 + m < len && cb + i * 16 < V ? Rv[i][m] : 0u;
+        x[m] = 4 * g4 + m < len && cb + i * 16 < V ? (uint32_t)Rv[i][m] : 0u;
         ok = ok && (x[m] & 0x7fffu) <= kValueMaxBits;
       }
       const uint2 w = make_uint2(x[0] | (x[1] << 16), x[2] | (x[3] << 16));
@@ -658,152 +713,158 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
     const int x = __ballot(ok) == ~0ull ? 0 : 1;
     if (lane == 0) reinterpret_cast<int*>(qsm + (n & 1) * Lay::buf + Lay::flag)[4 + w] = x;
   };
-  if (NC > 0) {
-    issue_v(0);
-    const bool s_ok = state_ok();
-    request(0, take_v(0) && s_ok);
-  }
-  __syncthreads();
-#pragma unroll 1
-  for (int n = 0; n < NC; ++n) {
-    const unsigned char* B = qsm + (n & 1) * Lay::buf;
-    const int len = min(QC, T - n * QC);
-    issue_v(n + 1);
-    if (__builtin_expect(leaves(n), 0)) {
-      left = n;
-      break;
-    }
-    f32x4 o[NVT];
-    const float* dec = reinterpret_cast<const float*>(B + (owed ? Lay::dec : Lay::pre)) + 4 * g4;
-    const bf16* pq = reinterpret_cast<const bf16*>(B + Lay::qa) + li * Lay::QP + 4 * g4;
-    // transposed reads of 4 rows x 16 columns: this lane's address is row li >> 2 of its
-    // group's four, columns 4 (li & 3); it receives column li
-    const bf16* pk = reinterpret_cast<const bf16*>(B + Lay::ka) +
-                     (4 * g4 + (li >> 2)) * Lay::KQ + 4 * (li & 3);
-    float4 d[2];
-    s4_t x[2][3], y[2][3];
-    auto operands = [&](int kt) __attribute__((always_inline)) {
-      d[kt & 1] = *reinterpret_cast<const float4*>(dec + kt * 16);
+  for (;;) {
+    // what follows from these is formed anew after the element-wise phase, not kept over it
+    asm volatile("" : "+v"(g4), "+v"(li), "+v"(cb));
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        x[kt & 1][i] = *reinterpret_cast<const s4_t*>(pq + i * QC * Lay::QP + kt * 16);
-        y[kt & 1][i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s4_t*)(pk + i * QC * Lay::KQ + kt * 16));
-      }
-    };
-    operands(0);
-    // Step kt: tile kt's qa S' (the main products in NOM sums, the others in three)
-    // and ka^T v onto the state, with the next tile decayed to the chunk's middle and split
-    // meanwhile and the one after it read from LDS. The order of the products keeps those of
-    // one sum apart, and the VALU work sits between them (an MFMA occupies its own pipe for
-    // 16 cycles, a VALU operation 4).
-    f32x4 om[NVT][NOM], orest[NVT][3];
-    float4 ap[PW];
-    Split sp[NVT][2];
-    auto decay = [&](int kt) __attribute__((always_inline)) {   // S' of tile kt, split
-      const float4 dd = d[kt & 1];
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) {
-        S[i][kt][0] *= dd.x;
-        S[i][kt][1] *= dd.y;
-        S[i][kt][2] *= dd.z;
-        S[i][kt][3] *= dd.w;
-        const float t[4] = {S[i][kt][0], S[i][kt][1], S[i][kt][2], S[i][kt][3]};
-        sp[i][kt & 1] = split3(t);
-      }
-    };
-    decay(0);
-    operands(1);
-#pragma unroll
-    for (int i = 0; i < NVT; ++i) {
-#pragma unroll
-      for (int j = 0; j < NOM; ++j) om[i][j] = zero4();
-#pragma unroll
-      for (int j = 0; j < 3; ++j) orest[i][j] = zero4();
-    }
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const int c = kt & 1;
-      s4_t xx[3], yy[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        xx[j] = x[c][j];
-        yy[j] = y[c][j];
-      }
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) {
-        const s4_t(&b)[3] = sp[i][c].p;
-        f32x4(&r)[3] = orest[i];
-        f32x4& t = S[i][kt];
-        om[i][kt % NOM] = mma16(xx[0], b[0], om[i][kt % NOM]);
-        t = mma16(yy[2], vv[i], t);
-        r[0] = mma16(xx[2], b[0], r[0]);
-        r[1] = mma16(xx[0], b[2], r[1]);
-        t = mma16(yy[1], vv[i], t);
-        r[2] = mma16(xx[1], b[1], r[2]);
-        r[0] = mma16(xx[1], b[0], r[0]);
-        t = mma16(yy[0], vv[i], t);
-        r[1] = mma16(xx[0], b[1], r[1]);
-      }
-      if (kt + 1 < KT) decay(kt + 1);
-      if (kt + 2 < KT) {
-        operands(kt + 2);
-      } else if (kt + 2 == KT) {
-#pragma unroll
-        for (int j = 0; j < PW; ++j)
-          ap[j] = *reinterpret_cast<const float4*>(
-              B + Lay::A + ((j * QC + li) * QTP + 4 * g4) * 4);
-      }
-#pragma unroll
-      for (int j = 0; j < 9 * NVT; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // one MFMA, four VALU
-        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // A v: row li, tokens 4 g4 ..; those after the row left out
-    const float4 am = PW == 1   ? ap[0]
-                      : PW == 2 ? add4(ap[0], ap[PW / 2])
-                                : add4(add4(ap[0], ap[1 % PW]), add4(ap[PW / 2], ap[PW - 1]));
-    const int after = li - 4 * g4;
-    const float aa[4] = {after >= 0 ? am.x : 0.f, after >= 1 ? am.y : 0.f,
-                         after >= 2 ? am.z : 0.f, after >= 3 ? am.w : 0.f};
-    const Split as = split3(aa);
-#pragma unroll
-    for (int i = 0; i < NVT; ++i) {
-      f32x4 u = zero4();
-#pragma unroll
-      for (int j = 2; j >= 0; --j) u = mma16(as.p[j], vv[i], u);
-      u += orest[i][0] + orest[i][1] + orest[i][2];
-#pragma unroll
-      for (int st = NOM / 2; st > 0; st /= 2)
-#pragma unroll
-        for (int j = 0; j < st; ++j) om[i][j] += om[i][j + st];
-      o[i] = om[i][0] + u;
-    }
-    owed = true;
-    {   // before the output's stores, which a wait for v behind them would wait for too
-      bool ok = take_v(n + 1);
-      if ((n & 7) == 7) ok = ok && state_ok();
-      request(n + 1, ok);
-    }
-    {
-      float* ob = (float*)p.out + chunk_t0(n, len) * rsV + (long)hh * V;
-#pragma unroll
-      for (int i = 0; i < NVT; ++i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 4 * g4 + r;
-          if (row < len && cb + i * 16 < V)
-            ob[(uint32_t)(p.dir ? len - 1 - row : row) * (uint32_t)rsV + (uint32_t)(cb + i * 16)] =
-                p.so * o[i][r];
-        }
-      }
+    for (int m = 0; m < 4; ++m) vo[m] = (uint32_t)(4 * g4 + m) * (uint32_t)rsV;
+    if (NC > 0) {
+      issue_v(start);
+      const bool s_ok = state_ok();
+      request(start, take_v(start) && s_ok);
     }
     __syncthreads();
-  }
-  if (__builtin_expect(left < NC, 0)) {
+#pragma unroll 1
+    for (int n = start; n < NC; ++n) {
+      const unsigned char* B = qsm + (n & 1) * Lay::buf;
+      const int len = min(QC, T - n * QC);
+      issue_v(n + 1);
+      if (__builtin_expect(leaves(n), 0)) {
+        left = n;
+        break;
+      }
+      f32x4 o[NVT];
+      const float* dec = reinterpret_cast<const float*>(B + (owed ? Lay::dec : Lay::pre)) + 4 * g4;
+      const bf16* pq = reinterpret_cast<const bf16*>(B + Lay::qa) + li * Lay::QP + 4 * g4;
+      // transposed reads of 4 rows x 16 columns: this lane's address is row li >> 2 of its
+      // group's four, columns 4 (li & 3); it receives column li
+      const bf16* pk = reinterpret_cast<const bf16*>(B + Lay::ka) +
+                       (4 * g4 + (li >> 2)) * Lay::KQ + 4 * (li & 3);
+      float4 d[2];
+      s4_t x[2][3], y[2][3];
+      auto operands = [&](int kt) __attribute__((always_inline)) {
+        d[kt & 1] = *reinterpret_cast<const float4*>(dec + kt * 16);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          x[kt & 1][i] = *reinterpret_cast<const s4_t*>(pq + i * QC * Lay::QP + kt * 16);
+          y[kt & 1][i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s4_t*)(pk + i * QC * Lay::KQ + kt * 16));
+        }
+      };
+      operands(0);
+      // Step kt: tile kt's qa S' (the main products in NOM sums, the others in three)
+      // and ka^T v onto the state, with the next tile decayed to the chunk's middle and split
+      // meanwhile and the one after it read from LDS. The order of the products keeps those of
+      // one sum apart, and the VALU work sits between them (an MFMA occupies its own pipe for
+      // 16 cycles, a VALU operation 4).
+      f32x4 om[NVT][NOM], orest[NVT][3];
+      float4 ap[PW];
+      Split sp[NVT][2];
+      auto decay = [&](int kt) __attribute__((always_inline)) {   // S' of tile kt, split
+        const float4 dd = d[kt & 1];
+#pragma unroll
+        for (int i = 0; i < NVT; ++i) {
+          S[i][kt][0] *= dd.x;
+          S[i][kt][1] *= dd.y;
+          S[i][kt][2] *= dd.z;
+          S[i][kt][3] *= dd.w;
+          const float t[4] = {S[i][kt][0], S[i][kt][1], S[i][kt][2], S[i][kt][3]};
+          sp[i][kt & 1] = split3(t);
+        }
+      };
+      decay(0);
+      operands(1);
+#pragma unroll
+      for (int i = 0; i < NVT; ++i) {
+#pragma unroll
+        for (int j = 0; j < NOM; ++j) om[i][j] = zero4();
+#pragma unroll
+        for (int j = 0; j < 3; ++j) orest[i][j] = zero4();
+      }
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        const int c = kt & 1;
+        s4_t xx[3], yy[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          xx[j] = x[c][j];
+          yy[j] = y[c][j];
+        }
+#pragma unroll
+        for (int i = 0; i < NVT; ++i) {
+          const s4_t(&b)[3] = sp[i][c].p;
+          f32x4(&r)[3] = orest[i];
+          f32x4& t = S[i][kt];
+          om[i][kt % NOM] = mma16(xx[0], b[0], om[i][kt % NOM]);
+          t = mma16(yy[2], vv[i], t);
+          r[0] = mma16(xx[2], b[0], r[0]);
+          r[1] = mma16(xx[0], b[2], r[1]);
+          t = mma16(yy[1], vv[i], t);
+          r[2] = mma16(xx[1], b[1], r[2]);
+          r[0] = mma16(xx[1], b[0], r[0]);
+          t = mma16(yy[0], vv[i], t);
+          r[1] = mma16(xx[0], b[1], r[1]);
+        }
+        if (kt + 1 < KT) decay(kt + 1);
+        if (kt + 2 < KT) {
+          operands(kt + 2);
+        } else if (kt + 2 == KT) {
+#pragma unroll
+          for (int j = 0; j < PW; ++j)
+            ap[j] = *reinterpret_cast<const float4*>(
+                B + Lay::A + ((j * QC + li) * QTP + 4 * g4) * 4);
+        }
+#pragma unroll
+        for (int j = 0; j < 9 * NVT; ++j) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // one MFMA, four VALU
+          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // A v: row li, tokens 4 g4 ..; those after the row left out
+      const float4 am = PW == 1   ? ap[0]
+                        : PW == 2 ? add4(ap[0], ap[PW / 2])
+                                  : add4(add4(ap[0], ap[1 % PW]), add4(ap[PW / 2], ap[PW - 1]));
+      const int after = li - 4 * g4;
+      const float aa[4] = {after >= 0 ? am.x : 0.f, after >= 1 ? am.y : 0.f,
+                           after >= 2 ? am.z : 0.f, after >= 3 ? am.w : 0.f};
+      const Split as = split3(aa);
+#pragma unroll
+      for (int i = 0; i < NVT; ++i) {
+        f32x4 u = zero4();
+#pragma unroll
+        for (int j = 2; j >= 0; --j) u = mma16(as.p[j], vv[i], u);
+        u += orest[i][0] + orest[i][1] + orest[i][2];
+#pragma unroll
+        for (int st = NOM / 2; st > 0; st /= 2)
+#pragma unroll
+          for (int j = 0; j < st; ++j) om[i][j] += om[i][j + st];
+        o[i] = om[i][0] + u;
+      }
+      owed = true;
+      {   // before the output's stores, which a wait for v behind them would wait for too
+        bool ok = take_v(n + 1);
+        if ((n & 7) == 7) ok = ok && state_ok();
+        request(n + 1, ok);
+      }
+      {
+        float* ob = (float*)p.out + chunk_t0(n, len) * rsV + (long)hh * V;
+#pragma unroll
+        for (int i = 0; i < NVT; ++i) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = 4 * g4 + r;
+            if (row < len && cb + i * 16 < V)
+              ob[(uint32_t)(p.dir ? len - 1 - row : row) * (uint32_t)rsV +
+                 (uint32_t)(cb + i * 16)] = p.so * o[i][r];
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (__builtin_expect(left == NC, 1)) break;
     if (owed) mul_rows(qsm + (left & 1) * Lay::buf + Lay::ppost);
+    owed = false;
     __syncthreads();   // the factors are read
     float* X = reinterpret_cast<float*>(qsm);
     int gl = g4, cl = w * NVT * 16 + li;
@@ -813,9 +874,23 @@ __global__ __launch_bounds__((QCW + KP / 64) * 64, KP < 256 && NVT == 1 ? 3 : 2)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) X[(kt * 16 + 4 * gl + r) * (CB + 4) + cl + i * 16] = S[i][kt][r];
-    rec_elements_consumer<KP, NVT>(p, qsm, left * QC, T, sN, ct, w, lane);
-    return;
+        for (int r = 0; r < 4; ++r)
+          X[(kt * 16 + 4 * gl + r) * (CB + 4) + cl + i * 16] = S[i][kt][r];
+    const int end = min(left + span, NC);
+    rec_elements_consumer<KP, NVT>(p, qsm, left * QC, min(T, end * QC), end < NC, sN, ct, w, lane);
+    if (end == NC) return;
+    asm volatile("" : "+v"(gl), "+v"(cl));
+#pragma unroll
+    for (int i = 0; i < NVT; ++i)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[i][kt][r] = X[(kt * 16 + 4 * gl + r) * (CB + 4) + cl + i * 16];
+    __syncthreads();   // the state is out of LDS
+    start = end;
+    span *= 4;
+    left = NC;
   }
   if (owed) mul_rows(qsm + ((NC - 1) & 1) * Lay::buf + Lay::post);
   if (sN) {

@@ -1,9 +1,9 @@
 """GPU parity of fused_recurrent_gla's bf16 forward on the matrix cores (16 tokens at a time;
-sequences of 24 tokens and more, packed ones of 24 on average) against the oracle, at the float32 bar (max-abs error <= 1e-4) and at the sizes where its tiles
-end: tokens around multiples of 16, key sizes around 64 / 128 / 256 and odd ones (element
-loads), column counts around the 16-column tiles and the 64- and 128-column blocks, packed
-sequences of one token, reversed order; gates beyond the factoring's range and non-finite
-inputs, which it takes token by token."""
+sequences of 24 tokens and more, packed ones of 24 on average) against the oracle, at the float32
+bar (max-abs error <= 1e-4) and at the sizes where its tiles end: tokens around multiples of 16,
+key sizes around 64 / 128 / 256 and odd ones (element loads), column counts around the 16-column
+tiles and the 64- and 128-column blocks, packed sequences of one token, reversed order; gates
+beyond the factoring's range and non-finite inputs, which it takes as the recurrence is written."""
 
 import numpy as np
 import pytest
@@ -195,3 +195,27 @@ def test_recurrent_chunk_leaves_the_matrix_cores(c, at, what):
         scale = 2.0 ** 21 if what == "large v" else 1.0
         if (m & col).any():
             check(name, got[m & col], ref[m & col], "f32", atol=max(1e-4, scale * 2 ** -18))
+
+
+# strong gates at these steps of the scan: it leaves the matrix cores there and returns after 8
+# chunks of 16 tokens, then after 32: once and back, twice and back, to the end in either phase
+@pytest.mark.parametrize("c,steps", [
+    (dict(B=1, T=300, H=2, K=64, V=40), [5]),
+    (dict(B=2, T=1000, H=1, K=96, V=70), [40, 260]),
+    (dict(B=1, T=999, H=1, K=256, V=64, reverse=True), [40, 260]),
+    (dict(B=1, T=400, H=2, K=130, V=20), [20, 200]),
+    (dict(B=40, T=330, H=8, K=72, V=136), [5, 200]),
+    (dict(B=40, T=300, H=8, K=48, V=128), [130]),
+    (dict(B=1, T=700, H=2, K=128, V=33, cu=[0, 290, 305, 700]), [20, 60]),
+], ids=lambda x: "-".join(f"{a}{b}" for a, b in x.items()) if isinstance(x, dict) else str(x))
+def test_recurrent_chunk_returns_to_the_matrix_cores(c, steps):
+    x = dict(zip(("q", "k", "v", "g", "s0"), _inputs(c)))
+    cu = c.get("cu", [0, c["T"]])
+    for i in steps:
+        for a, b in zip(cu, cu[1:]):
+            if i < b - a:
+                x["g"][:, b - 1 - i if c.get("reverse") else a + i, :, 2::3] = -45.0
+    print(f"recurrent chunk {c}, strong gates at {steps}", flush=True)
+    args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
+    for name, got, ref in zip(("o", "ht"), _call(*args, c), _oracle(*args, c)):
+        check(name, got, ref, "f32")

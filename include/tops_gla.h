@@ -141,8 +141,9 @@ int tops_gla_chunk_fwd_o(const void* q, const void* k, const void* v, const void
  * below the varlen = 2 size). The largest piece of a packed sequence follows from the call's
  * chunks and heads together, as a fixed-length call's segments follow from its batch: the same
  * sequence beside others may be cut elsewhere, and its sums then round differently (within the
- * bf16 operands' rounding). Without the segment part it is one segment whatever is beside it. The per-chunk states h_ws that the forward
- * stores for flagged pairs are not meaningful (the backward recomputes those pairs).
+ * bf16 operands' rounding). Without the segment part it is one segment whatever is beside it.
+ * The per-chunk states h_ws that the forward stores for flagged pairs are not meaningful (the
+ * backward recomputes those pairs).
  * No counterpart in the reference (its scans are sequential grid axes, chunk_h.py:252-271).
  */
 int64_t tops_gla_chunk_ws_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V,

@@ -16,13 +16,13 @@
 // What bounds it: VALU issue of the splits and of the producers' exponentials (bf16 MFMAs run
 // beside other waves' VALU work; float32 MFMAs do not -- 923 us of them and 575 us of FMAs in
 // another wave of the SIMD took 1444 us together, bf16 ones 971 -> 986 -- and are a sixteenth
-// as fast: this kernel with them ran at 520 us instead of 461). The state never leaves the
+// as fast: this kernel with them ran at 520 us instead of 458). The state never leaves the
 // registers: a wave holds all K rows of 16 (or 32) columns as accumulators (rows 4g + r,
 // column l & 15 in lane l = 16 g + column), which is also the B operand of an MFMA over those
 // rows, so qa S' and ka^T v need no transposition and no exchange between waves. Measured: B8
 // T2048 H4 K256 V512 951 -> 458 us, B64 T64 H16 K=V=128 131 -> 101 us (92 with inputs left in
-// the caches), B3 T1000 H16 K=V=64 317 -> 157 us (the VALU scan and this kernel). VALU busy 69 %,
-// the MFMA pipe 31 % in the first.
+// the caches), B3 T1000 H16 K=V=64 317 -> 149 us (the VALU scan and this kernel). VALU busy 65 %,
+// the MFMA pipe 29 % in the first.
 //
 // Block = (sequence, head, 64 or 128 columns): four consumer waves, each 16 or 32 columns,
 // and KP / 64 producer waves. While the consumers work on tokens 16 n .., the producers make

@@ -219,3 +219,27 @@ def test_recurrent_chunk_returns_to_the_matrix_cores(c, steps):
     args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
     for name, got, ref in zip(("o", "ht"), _call(*args, c), _oracle(*args, c)):
         check(name, got, ref, "f32")
+
+
+@pytest.mark.parametrize("where", ["v", "s0"])
+@pytest.mark.parametrize("c", [
+    dict(B=1, T=300, H=2, K=64, V=40), dict(B=1, T=300, H=2, K=130, V=70, reverse=True),
+    dict(B=40, T=190, H=8, K=72, V=136), dict(B=1, T=420, H=1, K=256, V=33, cu=[0, 400, 420])],
+    ids=lambda c: "-".join(f"{a}{b}" for a, b in c.items()))
+def test_recurrent_chunk_carries_nan(c, where):
+    """A NaN in the state stays in its column, with infinities beside it, over strong gates and the
+    sequence's end."""
+    x = dict(zip(("q", "k", "v", "g", "s0"), _inputs(c)))
+    if where == "v":
+        x["v"][0, 21, 0, 3] = np.nan
+    else:
+        x["s0"][0, 0, 1, 3] = np.nan
+        x["s0"][0, 0, 2, 4] = np.inf
+    x["g"][0, 170, 0, 5] = -45.0
+    x["g"][0, 185, 0, 6] = -np.inf
+    print(f"recurrent chunk {c}, NaN in {where}", flush=True)
+    args = (x["q"], x["k"], x["v"], x["g"], x["s0"])
+    with np.errstate(all="ignore"):
+        refs = _oracle(*args, c)
+    for name, got, ref in zip(("o", "ht"), _call(*args, c), refs):
+        _same_non_finite(name, got, ref)
